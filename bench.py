@@ -48,8 +48,7 @@ HBM_PEAK_GBS = 8000.0
 # kernel only).
 PHASES = {
     "acoustic_substep": {"bytes_s": 17, "per_step": "substeps",
-                         "kernels": ("acoustic_forward", "acoustic_hevi_explicit", "acoustic_hevi_column",
-                                     "acoustic_hevi_column_seg", "acoustic_momentum", "acoustic_commit",
+                         "kernels": ("acoustic_forward", "acoustic_hevi_solve", "acoustic_momentum", "acoustic_commit",
                                      "bc_west_east", "bc_south_north", "bc_vertical", "seed_radiation")},
     "slow_rk2_apply": {"bytes_s": 44, "per_step": 1, "kernels": ("slow_stage1", "slow_stage2")},
     "scalar_transport": {"bytes_s": 13, "per_step": 1,
@@ -98,13 +97,9 @@ ALGO_PER_CELL = {
     "acoustic_forward": (13, 0),
     # read rho'(new) p' u v w; write u v, and w for explicit members
     "acoustic_momentum": {"explicit": (8, 0), "hevi": (7, 0)},
-    # HE-VI horizontal part: read rho' u v theta mfx mfy; write mfx mfy rho* p*
-    "acoustic_hevi_explicit": (10, 0),
-    # HE-VI column solve: read rho* p* p' w rho' theta mfz; write w rho' p' mfz;
-    # the FP64 Thomas coefficients c', d' are written and read back (32 B)
-    "acoustic_hevi_column": (11, 32),
-    # the partitioned column solve of FP64 members: the same 11 fields, no coefficient arrays
-    "acoustic_hevi_column_seg": (11, 0),
+    # HE-VI horizontal part and column solve: read rho' u v theta mfx mfy p' w mfz;
+    # write mfx mfy w mfz rho' p'
+    "acoustic_hevi_solve": (15, 0),
     # read mfx mfy mfz and four scalars; write 3 face fluxes per scalar
     "transport_flux": (19, 0),
     # read rho_b, and fluxes and value of the three moisture scalars; write 3 limiter ratios

@@ -355,15 +355,17 @@ int nimbus_hip_member_set_tiling(nimbus_hip_ctx* ctx, uint32_t id, int tile_w, i
 /* HE-VI column-solve form of a member. It is fixed per member (never chosen
  * by the batch), so a member's results are the same alone and in any batch.
  * AUTO: partitioned for FP64 members of at most 129 levels and for FP32
- * members of fewer than 32768 columns and at most 129 levels, the sequential
- * sweep otherwise. PARTITIONED is refused above 129 levels, SEQUENTIAL for FP64
- * members of at most 129 levels (they hold no coefficient scratch). No
- * reference counterpart: the reference has no vertically implicit solve. */
+ * members of fewer than 32768 columns and at most 129 levels, sequential
+ * otherwise. PARTITIONED is refused above 129 levels, SEQUENTIAL for FP64
+ * members of at most 129 levels. Both forms are solved by the same kernel with
+ * the same operations (whole columns in LDS, eliminated from both ends), so
+ * the choice changes neither results nor time. No reference counterpart: the
+ * reference has no vertically implicit solve. */
 enum
 {
     NIMBUS_COLUMN_SOLVE_AUTO = 0,
-    NIMBUS_COLUMN_SOLVE_SEQUENTIAL = 1,  /* one thread per column, FP64 coefficients in scratch */
-    NIMBUS_COLUMN_SOLVE_PARTITIONED = 2  /* 16 runs of faces per column, reduced system in LDS */
+    NIMBUS_COLUMN_SOLVE_SEQUENTIAL = 1,
+    NIMBUS_COLUMN_SOLVE_PARTITIONED = 2
 };
 int nimbus_hip_member_set_column_solve(nimbus_hip_ctx* ctx, uint32_t id, int form);
 /* The member's form (SEQUENTIAL or PARTITIONED; AUTO for explicit-acoustic members). */

@@ -14,7 +14,7 @@
 // workgroups an XCD runs back to back are vertical neighbours and a
 // stencil's planes above and below are still in that XCD's L2 while every
 // thread stays independent (full occupancy, no serial march). The HE-VI
-// column solve gives each thread one whole column.
+// columns are solved by workgroups of a few whole columns (k_hevi_solve).
 //
 // Precision: S is the storage type. Continuity, EOS, base-state terms,
 // mass-flux accumulation and the HE-VI column system with its Thomas solve
@@ -58,6 +58,26 @@ template <class S>
 __device__ __forceinline__ gptr<S> P(void* p)
 {
     return (gptr<S>)(static_cast<S*>(p));
+}
+
+// The element `off` bytes from a field's (wave-uniform) base: a 32-bit offset
+// keeps the base in scalar registers, so the lanes do no 64-bit address
+// arithmetic and every field of a member shares one offset per cell. A field
+// holds fewer than 2^28 elements (runtime grid check), so offsets fit.
+template <class S>
+__device__ __forceinline__ S ld(gptr<const S> p, unsigned off)
+{
+    return *(gptr<const S>)((gptr<const char>)p + off);
+}
+template <class S>
+__device__ __forceinline__ S ld(gptr<S> p, unsigned off)
+{
+    return *(gptr<S>)((gptr<char>)p + off);
+}
+template <class S>
+__device__ __forceinline__ void st(gptr<S> p, unsigned off, S v)
+{
+    *(gptr<S>)((gptr<char>)p + off) = v;
 }
 
 __device__ __forceinline__ double finite0(double x) { return isfinite(x) ? x : 0.0; }
@@ -434,23 +454,64 @@ __global__ __launch_bounds__(kBlock) void k_slow(const MemberArgs* __restrict__ 
 // (1 + x)^gamma - 1 in FP32. For |x| < 1/8 (every realistic perturbation)
 // it is the binomial series sum_{n=1..8} C(gamma, n) x^n, whose truncation
 // error is below 2e-10 relative, evaluated by Horner's rule (about 1 ulp);
-// larger |x| take expm1(gamma log1p(x)).
-__device__ __forceinline__ float pow1p_gamma_m1(float x)
+// larger |x| take exp(gamma log(1 + x)) - 1 in FP64: 1 + x = m 2^e with m in
+// [sqrt(1/2), sqrt(2)), log m = 2 atanh((m - 1) / (m + 1)) to its s^15 term
+// (|s| <= 0.172: 1e-13), the exponential of the remainder below ln(2) / 2 to
+// its 11th power (3e-14). It takes a quarter of the instructions and
+// registers of expm1f(gamma log1pf(x)), which this path made every kernel
+// with an EOS carry, and its result rounds correctly but for ties. x < -1
+// gives not-a-number and x = -1 gives -1, as those functions do.
+__device__ __forceinline__ double pow_gamma_m1_far(double y)
 {
-    if (fabsf(x) < 0.125f)
-    {
-        // C(gamma, n) for gamma = cp / (cp - Rd) = 1004 / 717
-        float p = 3.214725001e-03f;
-        p = fmaf(x, p, -4.592693052e-03f);
-        p = fmaf(x, p, 6.989304557e-03f);
-        p = fmaf(x, p, -1.164974359e-02f);
-        p = fmaf(x, p, 2.240575685e-02f);
-        p = fmaf(x, p, -5.602415924e-02f);
-        p = fmaf(x, p, 2.802510849e-01f);
-        p = fmaf(x, p, 1.400278940e+00f);
-        return x * p;
-    }
-    return expm1f(float(kGamma) * log1pf(x));
+    if (!(y > 0.0)) return y == 0.0 ? -1.0 : __builtin_nan("");
+    if (!(y < __builtin_inf())) return y;
+    double m = __builtin_amdgcn_frexp_mant(y);
+    int e = __builtin_amdgcn_frexp_exp(y);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e = low ? e - 1 : e;
+    const double s = (m - 1.0) / (m + 1.0), s2 = s * s;
+    double l = 1.0 / 15.0;
+    l = fma(l, s2, 1.0 / 13.0);
+    l = fma(l, s2, 1.0 / 11.0);
+    l = fma(l, s2, 1.0 / 9.0);
+    l = fma(l, s2, 1.0 / 7.0);
+    l = fma(l, s2, 1.0 / 5.0);
+    l = fma(l, s2, 1.0 / 3.0);
+    l = fma(l, s2, 1.0);
+    // gamma log2(1 + x) = n + r, |r| <= 1/2
+    const double t = kGamma * fma(2.0 * 1.4426950408889634 * s, l, double(e));
+    const double n = rint(t), r = (t - n) * 0.69314718055994531;
+    double x = 1.0 / 39916800.0;
+    x = fma(x, r, 1.0 / 3628800.0);
+    x = fma(x, r, 1.0 / 362880.0);
+    x = fma(x, r, 1.0 / 40320.0);
+    x = fma(x, r, 1.0 / 5040.0);
+    x = fma(x, r, 1.0 / 720.0);
+    x = fma(x, r, 1.0 / 120.0);
+    x = fma(x, r, 1.0 / 24.0);
+    x = fma(x, r, 1.0 / 6.0);
+    x = fma(x, r, 0.5);
+    x = fma(x, r, 1.0);
+    x = fma(x, r, 1.0);
+    return __builtin_amdgcn_ldexp(x, int(fmin(fmax(n, -4096.0), 4096.0))) - 1.0;
+}
+
+__device__ __forceinline__ float pow1p_gamma_m1(double xd)
+{
+    const float x = float(xd);
+    // C(gamma, n) for gamma = cp / (cp - Rd) = 1004 / 717
+    float p = 3.214725001e-03f;
+    p = fmaf(x, p, -4.592693052e-03f);
+    p = fmaf(x, p, 6.989304557e-03f);
+    p = fmaf(x, p, -1.164974359e-02f);
+    p = fmaf(x, p, 2.240575685e-02f);
+    p = fmaf(x, p, -5.602415924e-02f);
+    p = fmaf(x, p, 2.802510849e-01f);
+    p = fmaf(x, p, 1.400278940e+00f);
+    p *= x;
+    if (__builtin_expect(!(fabsf(x) < 0.125f), 0)) p = float(pow_gamma_m1_far(1.0 + double(x)));
+    return p;
 }
 
 // Base-state profiles used by the EOS: rho0, p0, 1 / (rho0 theta0),
@@ -520,7 +581,7 @@ __device__ __forceinline__ double eos_full_pressure(const Prof& pr, int k, doubl
     if constexpr (sizeof(S) == sizeof(float))
     {
         const double x = rho * theta * pr.inv_rt0(k) - 1.0;
-        const float e = pow1p_gamma_m1(float(x));
+        const float e = pow1p_gamma_m1(x);
         return pr.p0(k) + (double(e) * pr.pe0(k) + pr.pe_diff(k));
     }
     else
@@ -703,583 +764,387 @@ __global__ __launch_bounds__(kBlock) void k_acoustic_forward(const MemberArgs* _
 // HE-VI substep: horizontal continuity explicit, vertical w-rho-p coupling
 // off-centred implicit (alpha = (1+beta)/2): the vertical pressure gradient
 // acts on alpha p^{n+1} + (1 - alpha) p^n with p^{n+1} linearised about
-// p* = EOS(rho*); FP64 Thomas sweep per column, flux-form density update and
-// EOS re-diagnosis. Two kernels: k_hevi_explicit (one thread per cell) does
-// the horizontal part, k_hevi_column (one thread per column) the vertical
-// solve. rho' is read from buffer s & 1 and written to (s + 1) & 1; u, v, w
-// stay in their home buffers (w is only touched by its own column).
+// p* = EOS(rho*); FP64 elimination per column, flux-form density update and
+// EOS re-diagnosis. rho' is read from buffer s & 1 and written to (s + 1) & 1;
+// u, v, w stay in their home buffers (w is only touched by its own column).
 // ---------------------------------------------------------------------
 
-// Part 1, per cell: retained horizontal mass fluxes, the density after the
-// explicit horizontal divergence rho* and its EOS pressure p*, stored as
-// perturbations (rho* - rho0 in the new-density buffer, p* - p0 in the u2
-// scratch field, which is dead between the slow stage 2 and transport).
-// Ghost columns get the reference's pass-2 clamp/EOS here and are not
-// touched by the column solve.
+// HE-VI substep, one kernel: the explicit horizontal part of every cell and
+// the implicit vertical solve of every column. A workgroup takes CW
+// consecutive columns of one row, LL lanes per level and V consecutive cells
+// (16 bytes) per lane, so each thread loads its cells' operands once, at the
+// start, as 16-byte loads, and keeps what the end needs in registers. With
+// Y_r = rb_r w_r (rb_r the face density) the rows of the w system are
+// symmetric:
+//   -g_r Y_{r-1} + (1 + g_r + g_{r+1}) Y_r - g_{r+1} Y_{r+1} = F_r - (H_{r+1} - H_r),
+//   g_k = (alpha dts / dz)^2 gamma p*_k / rho*_k,  F_r = rb_r w_r at the substep start,
+//   H_k = (dts / dz)(alpha p*'_k + (1 - alpha) p^n'_k) - ((1 - alpha) / alpha) g_k (F_k - F_{k-1}),
+// so a cell contributes two numbers and no row needs a division by rb.
+//  1. All threads: retained horizontal mass fluxes, rho*, p* = EOS(rho*), g
+//     and H, exchanged through LDS to the right-hand sides.
+//  2. Two waves eliminate the rows, one upwards from the ground, one downwards
+//     from the lid, meet in the middle and substitute back: half the length
+//     of one sweep, which is a chain of dependent FP64 operations. The pivots
+//     are at least 1 (g >= 0, 0 <= c' < 1); a column with a non-positive or
+//     non-finite one keeps its substep-start w.
+//  3. All threads: w = Y / rb, the off-centred mass flux, density and EOS.
+// Cells outside the columns to solve (x ghosts, the row padding) go through
+// the same code with a zero g and H and keep their w; rows of y ghosts skip
+// the solve.
+//
+// Bound by latency: a workgroup's time is its loads (10-16 k cycles), the
+// cells (9 k), the two chains (13 k) and the end (7 k), and the register file
+// holds two (100 levels) to four (64 levels) workgroups per CU, so the time
+// follows the columns in flight. 16-byte lanes because 8- and 4-byte ones
+// took 576 and 914 us per substep where these take 426 (400 x 400 x 100), and
+// four lanes per level because a row segment is then one 64-byte line.
+// Against a kernel for the horizontal part and one thread per column, or one
+// per 8 faces, for the vertical (us per substep): 400 x 400 x 100 mixed
+// 441 -> 417, 640 x 640 x 60 674 -> 463, 100 x 120 x 140 138 -> 78,
+// 160 x 160 x 80 82 -> 64, 48 x 48 x 40 21 -> 13, 256 x 256 x 80 FP64 262 -> 251.
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_hevi_explicit(const MemberArgs* __restrict__ ma,
-                                                          const int2* __restrict__ map, int s, int accumulate,
-                                                          int init)
+using Vec = __attribute__((ext_vector_type(16 / sizeof(S)))) S;
+
+template <class S>
+__device__ __forceinline__ Vec<S> ldv(const void* p, unsigned off)
 {
-    const Work wk = work_of(map);
-    const MemberArgs& A = ma[wk.m];
-    if (s >= A.p.substeps) return;
-    const Cell cl = cell_of(A, wk.local);
-    if (!cl.valid) return;
-    const DevGrid& g = A.g;
-    const int NX = g.nx, NY = g.ny, NZ = g.nz;
-    const int i = cl.i, j = cl.j, k = cl.k;
-    const DevFields& f = A.f;
-    const int par = s & 1;
-    const auto u = P<S>(f.u), v = P<S>(f.v), th = P<S>(f.th);
-    const auto rp_in = P<S>(par ? f.rp2 : f.rp);
-    const auto rp_out = P<S>(par ? f.rp : f.rp2);
-    const auto mfx = P<S>(f.mfx), mfy = P<S>(f.mfy);
-    const bool acc = accumulate != 0, first = init != 0 && s == 0;
-    const double dts = A.p.dts, weight = A.p.mf_weight;
-    const std::size_t sy = std::size_t(g.px);
-    const std::size_t c = g.at(i, j, k);
-    const std::size_t cxp = i < NX - 1 ? c + 1 : c, cyp = j < NY - 1 ? c + sy : c;
-    const std::size_t cxm = i >= 1 ? c - 1 : c, cym = j >= 1 ? c - sy : c;
-    S rpc = rp_in[c], rpxp = rp_in[cxp], rpyp = rp_in[cyp], rpxm = rp_in[cxm], rpym = rp_in[cym];
-    S uc = u[c], um = u[cxm], vc = v[c], vm = v[cym], thc = th[c];
-    S mfx0 = mfx[c], mfy0 = mfy[c];  // used only when accumulating onto them
-    const VProf pv = vprof(f.base, NZ, k);
-    pin(rpc); pin(rpxp); pin(rpyp); pin(rpxm); pin(rpym); pin(uc); pin(um); pin(vc); pin(vm); pin(thc);
-    pin(mfx0); pin(mfy0);
-    const double r0 = pv.r0;
-    const double rc = r0 + double(rpc);
-    const double rxp = r0 + double(rpxp), ryp = r0 + double(rpyp);
-    if (acc)
-    {
-        if (i < NX - 1) mfx[c] = S((first ? 0.0 : double(mfx0)) + weight * (0.5 * (rc + rxp) * double(uc)));
-        if (j < NY - 1) mfy[c] = S((first ? 0.0 : double(mfy0)) + weight * (0.5 * (rc + ryp) * double(vc)));
-    }
-    if (first) P<S>(f.rb)[c] = rpc;
-    if (!(i >= 1 && i < NX - 1 && j >= 1 && j < NY - 1))
-    {
-        // ghost column: density unchanged (clamped), EOS pressure, no vertical flux
-        if (acc && first) P<S>(f.mfz)[c] = S(0);
-        const RhoP<S> o = density_eos<S>(A.p.bounds, pv, k, rc, double(thc));
-        rp_out[c] = o.r;
-        P<S>(f.pp)[c] = o.p;
-        return;
-    }
-    const double rxm = r0 + double(rpxm), rym = r0 + double(rpym);
-    const double dh = -((0.5 * (rc + rxp) * double(uc) - 0.5 * (rxm + rc) * double(um)) * g.idx +
-                        (0.5 * (rc + ryp) * double(vc) - 0.5 * (rym + rc) * double(vm)) * g.idy);
-    const double rstar = rc + dts * finite0(dh);
-    // linearisation point p* = EOS(rho*): FP64 power law in FP64 storage, the
-    // perturbation form (FP32 relative accuracy on p* - p0) in the mixed mode
-    const double ps = eos_full_pressure<S>(pv, k, rstar, double(thc));
-    rp_out[c] = S(rstar - r0);
-    P<S>(f.u2)[c] = S(ps - pv.p0_);
+    return *(gptr<const Vec<S>>)((gptr<const char>)p + off);
+}
+template <class S>
+__device__ __forceinline__ void stv(void* p, unsigned off, Vec<S> v)
+{
+    *(gptr<Vec<S>>)((gptr<char>)p + off) = v;
 }
 
-// Part 2, one thread per interior column. Up-sweep: each row (face) of the
-// w system from its two cells' rho*, p*, substep-start p and face
-// densities, eliminated at once (FP64 c', d' kept in tri_c / tri_r).
-// Down-sweep: back substitution, off-centred vertical mass flux, final
-// density and EOS pressure. The inputs of the next kRing - 1 levels are in
-// flight while a level is processed: a ring of kRing register sets, the loop
-// unrolled by kRing so the ring rotates by renaming, every load unconditional
-// (levels clamped to the column), the base-state profiles in LDS.
-constexpr int kRing = 4;
-
-template <class S>
-struct HeviUp
+// One direction of the elimination: h rows from *bq, *gq (g on the side
+// already eliminated) in steps of ST, c' and d' replacing g and the
+// right-hand side. Rows go in groups of four: a group's operands are loaded
+// while the one before is eliminated.
+template <int ST>
+__device__ __forceinline__ void eliminate(double* gq, double* bq, int h, double& cp, double& dp, double& least)
 {
-    S rs, ps, pn, w, rp;  // rho* - rho0, p* - p0, substep-start p', w, substep-start rho'
-};
-
-template <class S>
-struct HeviDown
-{
-    double tr, tc;
-    S w, rp, rs, th, mfz;
-};
-
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_hevi_column(const MemberArgs* __restrict__ ma,
-                                                        const int2* __restrict__ map, int s, int accumulate, int init)
-{
-    const Work wk = work_of(map);
-    const MemberArgs& A = ma[wk.m];
-    const DevGrid& g = A.g;
-    // uniform over the block (one member per block); members the batch solves
-    // in the partitioned form are not this kernel's
-    if (s >= A.p.substeps || A.p.hevi_seg) return;
-    const Column t = column_of(A, wk.local);
-    const int NX = g.nx, NY = g.ny, NZ = g.nz;
-    extern __shared__ double s_prof[];
-    const LProf pr = stage_profiles(s_prof, A.f.base, NZ);
-    const int i = t.i, j = t.j;
-    if (!(i >= 1 && i < NX - 1 && j >= 1 && j < NY - 1)) return;  // no barrier after this point
-    const DevFields& f = A.f;
-    const int par = s & 1;
-    const gptr<S> __restrict__ w = P<S>(f.w);
-    const gptr<const S> __restrict__ rp_in = P<S>(par ? f.rp2 : f.rp);
-    const gptr<S> __restrict__ rp_out = P<S>(par ? f.rp : f.rp2);
-    const gptr<S> __restrict__ pp = P<S>(f.pp);
-    const gptr<const S> __restrict__ psb = P<S>(f.u2);
-    const gptr<const S> __restrict__ th = P<S>(f.th);
-    const gptr<S> __restrict__ mfz = P<S>(f.mfz);
-    const gptr<double> __restrict__ tc = G(f.tri_c);
-    const gptr<double> __restrict__ tr = G(f.tri_r);
-    const Bounds bd = A.p.bounds;
-    const double dts = A.p.dts, alpha = A.p.hevi_alpha, weight = A.p.mf_weight;
-    const bool acc = accumulate != 0, first = init != 0 && s == 0;
-    const std::size_t c0 = g.at(i, j, 0), sz = g.plane();
-    const double idz = g.idz;
-    const double a1 = 1.0 - alpha;
-
-    // ---- up-sweep
-    auto load_up = [&](int k) {
-        const std::size_t c = c0 + std::size_t(k) * sz;
-        HeviUp<S> L;
-        L.rs = rp_out[c]; L.ps = psb[c]; L.pn = pp[c]; L.w = w[c]; L.rp = rp_in[c];
-        return L;
+    constexpr int U = 4;
+    double gi = gq[0];
+    auto row = [&](double go, double bb, int e) {
+        const double piv = fma(-gi, cp, 1.0 + gi + go);
+        least = fmin(least, piv);  // infinite and not-a-number pivots show in the solution
+        // 1 / piv = r (1 + t), r the hardware estimate and t = err + err^2 (the error left is err^3)
+        const double r = __builtin_amdgcn_rcp(piv);
+        const double err = fma(-piv, r, 1.0), gr = go * r, dr = fma(gi, dp, bb) * r;
+        const double t = fma(err, err, err);
+        cp = fma(gr, t, gr);
+        dp = fma(dr, t, dr);
+        gq[e * ST] = cp;
+        bq[e * ST] = dp;
+        gi = go;
     };
-    HeviUp<S> ring[kRing];
-#pragma unroll
-    for (int q = 0; q < kRing; ++q) ring[q] = load_up(min(q, NZ - 1));
-    double rb_prev = 0.0, C_prev = 0.0, ps_prev = 0.0, pn_prev = 0.0, wo_prev = 0.0, e_prev = 0.0;
-    double rb_prev2 = 0.0, cp_prev = 0.0, rr_prev = 0.0;
-    bool ok = true;
-    for (int k0 = 0; k0 < NZ; k0 += kRing)
+    int q = 0;
+    if (h >= U)
     {
+        double gn[U], bn[U];
 #pragma unroll
-        for (int q = 0; q < kRing; ++q)
+        for (int e = 0; e < U; ++e) { gn[e] = gq[(e + 1) * ST]; bn[e] = bq[e * ST]; }
+        for (; q + 2 * U <= h; q += U)
         {
-            const int k = k0 + q;
-            const HeviUp<S> cur = ring[q];
-            const HeviUp<S> nxt = ring[(q + 1) % kRing];  // level k + 1
-            if (k < NZ)  // not a loop exit, and the refill below reuses cur's registers
+            double go[U], bb[U];
+#pragma unroll
+            for (int e = 0; e < U; ++e)
             {
-                const double r0 = pr.rho0(k);
-                const double rc = r0 + double(cur.rp);
-                const double rstar = r0 + double(cur.rs);
-                const double ps = pr.p0(k) + double(cur.ps);
-                const double C = kGamma * ps * (1.0 / rstar);
-                const double wo = double(cur.w);
-                // face density above level k (zero at the lid)
-                const double rbk = k < NZ - 1 ? 0.5 * (rc + (pr.rho0(k + 1) + double(nxt.rp))) : 0.0;
-                const double e = -a1 * dts * idz * (rbk * wo - rb_prev * wo_prev);
-                const double pnk = double(cur.pn);
-                if (k >= 1)
-                {
-                    // row r = k-1 (face k-1/2): unknowns w_{r-1}, w_r, w_{r+1}
-                    const double rbr = rb_prev;
-                    const double inv_rbr = 1.0 / rbr;
-                    const double Bc = alpha * dts * idz;
-                    const double Ak = Bc * inv_rbr;
-                    const double Aa = (k - 1) > 0 ? -Ak * Bc * C_prev * rb_prev2 : 0.0;
-                    const double U = (k - 1) < NZ - 2 ? -Ak * Bc * C * rbk : 0.0;
-                    const double D = 1.0 + Ak * Bc * (C + C_prev) * rbr;
-                    // PGF on alpha p* + (1 - alpha) p^n (p^n: substep-start pressure), base gradient removed
-                    const double G_ = (alpha * ((ps - ps_prev) - (pr.p0(k) - pr.p0(k - 1))) + a1 * (pnk - pn_prev)) * idz;
-                    const double R = wo_prev - dts * inv_rbr * G_ - Ak * (C * e - C_prev * e_prev);
-                    const double piv = D - Aa * cp_prev;
-                    if (!(piv > 0.0) || !isfinite(piv)) ok = false;
-                    const double inv_piv = 1.0 / piv;
-                    const double cpr = U * inv_piv;
-                    const double rrr = (R - Aa * rr_prev) * inv_piv;
-                    const std::size_t cr = c0 + std::size_t(k - 1) * sz;
-                    tc[cr] = cpr;
-                    tr[cr] = rrr;
-                    cp_prev = cpr;
-                    rr_prev = rrr;
-                }
-                rb_prev2 = rb_prev;
-                rb_prev = rbk;
-                C_prev = C;
-                ps_prev = ps;
-                pn_prev = pnk;
-                wo_prev = wo;
-                e_prev = e;
+                go[e] = gn[e];
+                bb[e] = bn[e];
+                gn[e] = gq[(U + e + 1) * ST];
+                bn[e] = bq[(U + e) * ST];
             }
-            ring[q] = load_up(min(k + kRing, NZ - 1));
+#pragma unroll
+            for (int e = 0; e < U; ++e) row(go[e], bb[e], e);
+            gq += U * ST;
+            bq += U * ST;
         }
+#pragma unroll
+        for (int e = 0; e < U; ++e) row(gn[e], bn[e], e);
+        gq += U * ST;
+        bq += U * ST;
+        q += U;
     }
-
-    // ---- down-sweep: iteration t handles face r = NZ-2-t (none at r = -1)
-    // and finalises cell r+1 (top face r+1, zero at the lid; bottom face r).
-    auto load_down = [&](int r) {
-        const std::size_t cr = c0 + std::size_t(r) * sz;
-        HeviDown<S> d;
-        d.w = w[cr]; d.tr = tr[cr]; d.tc = tc[cr]; d.rp = rp_in[cr]; d.rs = rp_out[cr]; d.th = th[cr];
-        d.mfz = mfz[cr];
-        return d;
-    };
-    double w_above = 0.0, wo_above = 0.0, rb_above = 0.0;  // face r+1 quantities (stored w)
-    double x_above = 0.0;                                  // face r+1 Thomas solution (unclamped)
-    HeviDown<S> cell = load_down(NZ - 1);                  // cell r+1 (its w, tr, tc are not used)
-    HeviDown<S> dring[kRing];
-#pragma unroll
-    for (int q = 0; q < kRing; ++q) dring[q] = load_down(max(NZ - 2 - q, 0));
-    for (int t0 = 0; t0 < NZ; t0 += kRing)
+    for (; q < h; ++q)
     {
-#pragma unroll
-        for (int q = 0; q < kRing; ++q)
-        {
-            const int r = NZ - 2 - (t0 + q);
-            const HeviDown<S> dn = dring[q];
-            if (r >= -1)
-            {
-                double wn = 0.0, wo = 0.0, rbr = 0.0;
-                if (r >= 0)
-                {
-                    const std::size_t cr = c0 + std::size_t(r) * sz;
-                    wo = double(dn.w);
-                    const double x = ok ? dn.tr - dn.tc * x_above : wo;
-                    x_above = x;
-                    wn = clamp_store<S>(x, 0.0, -bd.wind_v, bd.wind_v);
-                    w[cr] = S(wn);
-                    wn = double(S(wn));
-                    rbr = 0.5 * ((pr.rho0(r) + double(dn.rp)) + (pr.rho0(r + 1) + double(cell.rp)));
-                }
-                const int kc = r + 1;
-                const std::size_t cc = c0 + std::size_t(kc) * sz;
-                const double ft = kc < NZ - 1 ? rb_above * (alpha * w_above + a1 * wo_above) : 0.0;
-                const double fb = r >= 0 ? rbr * (alpha * wn + a1 * wo) : 0.0;
-                if (acc) mfz[cc] = S((first ? 0.0 : double(cell.mfz)) + weight * ft);
-                const double rstar = pr.rho0(kc) + double(cell.rs);
-                const RhoP<S> o = density_eos<S>(bd, pr, kc, rstar - dts * idz * (ft - fb), double(cell.th));
-                rp_out[cc] = o.r;
-                pp[cc] = o.p;
-                w_above = wn;
-                wo_above = wo;
-                rb_above = rbr;
-                cell = dn;
-            }
-            dring[q] = load_down(max(r - kRing, 0));
-        }
+        row(gq[ST], *bq, 0);
+        gq += ST;
+        bq += ST;
     }
 }
 
-// Part 2, partitioned form (columns of at most kSegMaxNz levels, chosen per
-// member by StepParams::hevi_seg): the same rows as the sequential sweep, in
-// FP64, solved without coefficient arrays in memory. Each column's faces
-// 0 .. nz-2 are split into runs of ls consecutive faces, one thread per run
-// (kSegCols consecutive columns of one row x kSegments runs per workgroup, so
-// every load is 16 contiguous lanes of one level). A thread
-//  1. loads its run's levels once (one level below and two above for the
-//     face densities);
-//  2. forward-eliminates its rows to x_r + c1_r x_{r+1} + a1_r L' = d1_r,
-//     where L' is the last unknown of the run below (a1 carries that
-//     coupling; the first run has none, and its c1, d1 are the sequential
-//     sweep's c', d'), and back-eliminates its first row to
-//     x_{s0} = dt0 - at0 L' - ct0 L, with L its own last unknown;
-//  3. forms its row of the system of the runs' last unknowns (row p:
-//     a1 L_{p-1} + (1 - c1 at') L_p - c1 ct' L_{p+1} = d1 - c1 dt', primes for
-//     run p + 1's first row), solved by cyclic reduction over the column's
-//     run threads in LDS;
-//  4. substitutes back down its run and finalises the cells whose lower face
-//     is in it (the face above the run is run p + 1's first unknown,
-//     evaluated from the same LDS values by the same expression).
-// Quotients use rcp_nr (about an ulp) rather than correctly rounded
-// division. Every pivot of the runs and of the reduction must be positive
-// and finite, otherwise the whole column keeps its substep-start w, as in the
-// sequential sweep. A run's neighbours overwrite its halo levels only after
-// the barriers, by which time every halo value has been consumed.
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_hevi_column_seg(const MemberArgs* __restrict__ ma,
-                                                            const int2* __restrict__ map, int s, int accumulate,
-                                                            int init)
+// Back substitution of h - 1 rows in steps of -ST from the row before the
+// one at *bq, *gq (c', d' of that row), whose solution y is already stored.
+template <int ST>
+__device__ __forceinline__ double substitute(const double* gq, double* bq, int h, double y)
 {
-    constexpr int NQ = kSegRows + 3;  // levels s0 - 1 .. s0 + ls + 1
+    constexpr int U = 4;
+    int q = h - 1;
+    if (q >= U)
+    {
+        double cn[U], dn[U];
+#pragma unroll
+        for (int e = 0; e < U; ++e) { cn[e] = gq[-(e + 1) * ST]; dn[e] = bq[-(e + 1) * ST]; }
+        for (; q >= 2 * U; q -= U)
+        {
+            double c[U], d[U];
+#pragma unroll
+            for (int e = 0; e < U; ++e)
+            {
+                c[e] = cn[e];
+                d[e] = dn[e];
+                cn[e] = gq[-(U + e + 1) * ST];
+                dn[e] = bq[-(U + e + 1) * ST];
+            }
+#pragma unroll
+            for (int e = 0; e < U; ++e) { y = fma(c[e], y, d[e]); bq[-(e + 1) * ST] = y; }
+            gq -= U * ST;
+            bq -= U * ST;
+        }
+#pragma unroll
+        for (int e = 0; e < U; ++e) { y = fma(cn[e], y, dn[e]); bq[-(e + 1) * ST] = y; }
+        gq -= U * ST;
+        bq -= U * ST;
+        q -= U;
+    }
+    for (; q > 0; --q)
+    {
+        gq -= ST;
+        bq -= ST;
+        y = fma(*gq, y, *bq);
+        *bq = y;
+    }
+    return y;
+}
+
+template <class S, bool FIRST, int LL>
+__global__ __launch_bounds__(1024) void k_hevi_solve(const MemberArgs* __restrict__ ma, const int2* __restrict__ map,
+                                                     int s)
+{
+    constexpr int V = 16 / int(sizeof(S)), CW = LL * V;
+    constexpr unsigned es = sizeof(S);
     const Work wk = work_of(map);
     const MemberArgs& A = ma[wk.m];
-    const DevGrid& g = A.g;
-    const int NX = g.nx, NY = g.ny, NZ = g.nz;
     // uniform over the block (one member per block): no barrier is skipped by part of it
-    if (s >= A.p.substeps || !A.p.hevi_seg || NZ > kSegMaxNz) return;
-    extern __shared__ double s_prof[];
-    const LProf pr = stage_profiles(s_prof, A.f.base, NZ);
-    double* const ex = s_prof + kLdsProfiles * NZ;         // [11][kBlock]: run ends and reduced rows
-    double* const lv = ex + 11 * kBlock;                   // [kBlock]: last unknown of each run
-    int* const okv = reinterpret_cast<int*>(lv + kBlock);  // [2][kBlock]: run and reduction verdicts
-
-    const int tid = int(threadIdx.x);
-    const int col = tid & (kSegCols - 1), p = tid / kSegCols;
-    const int row_blocks = (NX + kSegCols - 1) / kSegCols;
-    const int j = wk.local / row_blocks;
-    const int i = (wk.local - j * row_blocks) * kSegCols + col;
-    const bool interior = i >= 1 && i < NX - 1 && j >= 1 && j < NY - 1;
-    const int n = NZ - 1;  // unknown faces 0 .. NZ-2
-    const int ls = (n + kSegments - 1) / kSegments;
-    const int runs = (n + ls - 1) / ls;
-    const int s0 = p * ls;
-    const int m = interior && p < runs ? min(ls, n - s0) : 0;
-
+    if (s >= A.p.substeps || A.geo.solve_lanes != LL) return;
+    const DevGrid& g = A.g;
+    const int NX = g.nx, NY = g.ny, NZ = g.nz;
     const DevFields& f = A.f;
-    const int par = s & 1;
-    const gptr<S> __restrict__ w = P<S>(f.w);
-    const gptr<const S> __restrict__ rp_in = P<S>(par ? f.rp2 : f.rp);
-    const gptr<S> __restrict__ rp_out = P<S>(par ? f.rp : f.rp2);
-    const gptr<S> __restrict__ pp = P<S>(f.pp);
-    const gptr<const S> __restrict__ psb = P<S>(f.u2);
-    const gptr<const S> __restrict__ th = P<S>(f.th);
-    const gptr<S> __restrict__ mfz = P<S>(f.mfz);
-    const Bounds bd = A.p.bounds;
+    const int tid = int(threadIdx.x);
+    const unsigned first_col = unsigned(wk.local) * CW;  // of the padded plane; the pitch is a multiple of CW
+    const int j = int(first_col / unsigned(g.px));
+    const int i0 = int(first_col - unsigned(j) * unsigned(g.px)) + (tid % LL) * V;
+    const int kk = tid / LL, k = min(kk, NZ - 1);
+    const bool active = kk < NZ;
+    const unsigned plane = unsigned(g.plane()) * es, sy = unsigned(g.px) * es;  // bytes
+    const unsigned c = unsigned(k) * plane + unsigned(j) * sy + unsigned(i0) * es;
+    void* const rp_in = (s & 1) ? f.rp2 : f.rp;
+    void* const rp_out = (s & 1) ? f.rp : f.rp2;
+    const bool solve = j >= 1 && j < NY - 1;  // uniform: a workgroup's columns share one row
+
+    // the operands of the horizontal part, in flight before the profiles are
+    // staged (rows of y ghosts read themselves in the place of a missing
+    // neighbour row); those of the column follow it, which keeps the register count down
+    const unsigned yp = solve || j == 0 ? c + sy : c, ym = solve ? c - sy : c;
+    const Vec<S> r = ldv<S>(rp_in, c), ryp = ldv<S>(rp_in, yp), rym = ldv<S>(rp_in, ym);
+    const Vec<S> u = ldv<S>(f.u, c), v = ldv<S>(f.v, c), vm = ldv<S>(f.v, ym);
+    const Vec<S> th = ldv<S>(f.th, c);
+    const Vec<S> mx = FIRST ? Vec<S>(S(0)) : ldv<S>(f.mfx, c);
+    const Vec<S> my = FIRST ? Vec<S>(S(0)) : ldv<S>(f.mfy, c);
+    // the neighbours beyond the lane's cells (clamped at the first and last element of the row)
+    const unsigned xr = i0 + V < int(g.px) ? c + 16u : c, xl = i0 > 0 ? c - es : c;
+    const S rr = ld<S>(P<S>(rp_in), xr), rl = ld<S>(P<S>(rp_in), xl);
+    const S ul = ld<S>(P<S>(f.u), xl);
+
+    extern __shared__ double s_prof[];
+    const LProf pr = stage_profiles(s_prof, f.base, NZ);
+    double* const gs = s_prof + kLdsProfiles * NZ;  // [NZ][CW] g, later c', later the new mass flux
+    double* const bs = gs + NZ * CW;                // [NZ][CW] H, later the right-hand side, d' and Y
+    double* const xs = bs + NZ * CW;                // [5][CW] c', d' where the halves meet, Y of the middle row
+    int* const bad = reinterpret_cast<int*>(xs + 5 * CW);  // [2][CW] pivot verdicts of the halves
+    const Bounds& bd = A.p.bounds;
     const double dts = A.p.dts, alpha = A.p.hevi_alpha, weight = A.p.mf_weight;
-    const bool acc = accumulate != 0, first = init != 0 && s == 0;
-    const double idz = g.idz;
-    const double a1 = 1.0 - alpha;
-    const std::size_t c0 = m > 0 ? g.at(i, j, 0) : 0, sz = g.plane();
+    const double a1 = 1.0 - alpha, cdt = dts * g.idz;
+    const double bc = alpha * cdt, bc2g = bc * bc * kGamma, a1oa = a1 / alpha;
+    const double hw = 0.5 * weight, hix = 0.5 * g.idx, hiy = 0.5 * g.idy;
+    const int cell = k * CW + (tid % LL) * V;
 
-    // 1. level q is level s0 - 1 + q (clamped to the column for the load)
-    S rp[NQ], wo_s[NQ], rs[NQ], ps[NQ], pn[NQ], tq[NQ], mq[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
+    // 1.
+    const double r0 = pr.rho0(k), r0u = pr.rho0(min(k + 1, NZ - 1));
+    Vec<S> rs;
+    double gk[V], H[V];
     {
-        rp[q] = wo_s[q] = rs[q] = ps[q] = pn[q] = tq[q] = mq[q] = S(0);
-        if (q <= m + 2 && m > 0)
+        Vec<S> mxn, myn;
+#pragma unroll
+        for (int e = 0; e < V; ++e)
         {
-            const std::size_t c = c0 + std::size_t(clampi(s0 - 1 + q, 0, NZ - 1)) * sz;
-            rp[q] = rp_in[c];
-            wo_s[q] = w[c];
-            if (q >= 1 && q <= m + 1)
+            const int i = i0 + e;
+            const bool in = solve && i >= 1 && i < NX - 1;
+            const double rc = r0 + double(r[e]);
+            const S rxp = e + 1 < V ? r[e + 1 < V ? e + 1 : 0] : rr, rxm = e > 0 ? r[e > 0 ? e - 1 : 0] : rl;
+            const S um = e > 0 ? u[e > 0 ? e - 1 : 0] : ul;
+            // twice the face fluxes (the factor 1/2 is in the constants)
+            const double fxp = (rc + (r0 + double(rxp))) * double(u[e]);
+            const double fyp = (rc + (r0 + double(ryp[e]))) * double(v[e]);
+            mxn[e] = i < NX - 1 ? S(double(mx[e]) + hw * fxp) : mx[e];
+            myn[e] = i < NX && j < NY - 1 ? S(double(my[e]) + hw * fyp) : my[e];
+            const double dxf = fma(-((r0 + double(rxm)) + rc), double(um), fxp);
+            const double dyf = fma(-((r0 + double(rym[e])) + rc), double(vm[e]), fyp);
+            const double dh = -(dxf * hix + dyf * hiy);
+            const double rstar = in ? rc + dts * finite0(dh) : rc;
+            rs[e] = S(rstar - r0);
+            // linearisation point p* = EOS(rho*), as a perturbation
+            const double psf = solve ? eos_full_pressure<S>(pr, k, rstar, double(th[e])) : 0.0;
+            gk[e] = in ? bc2g * psf * rcp_nr(r0 + double(rs[e])) : 0.0;
+            H[e] = in ? cdt * alpha * (psf - pr.p0(k)) : 0.0;
+        }
+        if (active)
+        {
+            stv<S>(f.mfx, c, mxn);
+            stv<S>(f.mfy, c, myn);
+            if (FIRST) stv<S>(f.rb, c, r);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned zp = k < NZ - 1 ? c + plane : c, zm = k > 0 ? c - plane : c;
+    const Vec<S> pn = ldv<S>(f.pp, c), wo = ldv<S>(f.w, c), rzp = ldv<S>(rp_in, zp);
+    double b[V];
+    if (solve)
+    {
+        const Vec<S> rzm = ldv<S>(rp_in, zm), wm = ldv<S>(f.w, zm);
+        const double r0d = pr.rho0(max(k - 1, 0));
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+        {
+            const int i = i0 + e;
+            const double rc = r0 + double(r[e]);
+            const double fo = k < NZ - 1 ? 0.5 * (rc + (r0u + double(rzp[e]))) * double(wo[e]) : 0.0;
+            const double fl = k > 0 ? 0.5 * ((r0d + double(rzm[e])) + rc) * double(wm[e]) : 0.0;
+            const bool in = i >= 1 && i < NX - 1;
+            H[e] = in ? H[e] + (cdt * a1 * double(pn[e]) - a1oa * gk[e] * (fo - fl)) : 0.0;
+            b[e] = in ? fo + H[e] : 0.0;
+        }
+    }
+    if (solve)
+    {
+        if (active)
+        {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
             {
-                rs[q] = rp_out[c];
-                ps[q] = psb[c];
-                pn[q] = pp[c];
+                gs[cell + e] = gk[e];
+                bs[cell + e] = H[e];
             }
         }
-    }
-    auto lev = [&](int q) { return clampi(s0 - 1 + q, 0, NZ - 1); };
-    // old w of face s0 - 1 + q (none below the ground face)
-    auto wo = [&](int q) { return s0 - 1 + q >= 0 ? double(wo_s[q]) : 0.0; };
-    // full density of cell s0 - 1 + q
-    auto rc_at = [&](int q) { return pr.rho0(lev(q)) + double(rp[q]); };
-    // density of face s0 - 1 + q between cells q and q + 1 (zero below the ground face and at the lid)
-    auto rb_of = [&](int q, double rc_lo, double rc_hi) {
-        const int fq = s0 - 1 + q;
-        return fq >= 0 && fq < NZ - 1 ? 0.5 * (rc_lo + rc_hi) : 0.0;
-    };
-    // cell s0 - 1 + q: C = gamma p* / rho* and the full p*
-    auto cell_c = [&](int q, double& Cq, double& psq) {
-        const int k = lev(q);
-        const double rstar = pr.rho0(k) + double(rs[q]);
-        psq = pr.p0(k) + double(ps[q]);
-        Cq = kGamma * psq * rcp_nr(rstar);
-    };
-
-    // 2. forward elimination of rows r = s0 + t (cells r, r + 1; faces r - 1, r, r + 1),
-    // C, the old-w divergence e and the face densities rolled along as in the sequential sweep
-    double c1[kSegRows], a1s[kSegRows], d1[kSegRows];
-    bool ok = true;
-    double rb_lo = 0.0, rb_mid = 0.0, rc_nx = 0.0, C_lo = 0.0, ps_lo = 0.0, e_lo = 0.0;
-    if (m > 0)
-    {
-        const double r0 = rc_at(0), r1 = rc_at(1);
-        rc_nx = rc_at(2);
-        rb_lo = rb_of(0, r0, r1);
-        rb_mid = rb_of(1, r1, rc_nx);
-        cell_c(1, C_lo, ps_lo);
-        e_lo = -a1 * dts * idz * (rb_mid * wo(1) - rb_lo * wo(0));
-    }
-    const double Bc = alpha * dts * idz;
-    double cp = 0.0, ap = 0.0, dp = 0.0;  // the last eliminated row
-#pragma unroll
-    for (int t = 0; t < kSegRows; ++t)
-    {
-        if (t < m)
-        {
-            const int r = s0 + t;
-            const double rc_hi = rc_at(t + 3);
-            const double rb_hi = rb_of(t + 2, rc_nx, rc_hi);
-            rc_nx = rc_hi;
-            double C_hi, ps_hi;
-            cell_c(t + 2, C_hi, ps_hi);
-            const double e_hi = -a1 * dts * idz * (rb_hi * wo(t + 2) - rb_mid * wo(t + 1));
-            const double rbr = rb_mid;
-            const double inv_rbr = rcp_nr(rbr);
-            const double Ak = Bc * inv_rbr;
-            const double Aa = r > 0 ? -Ak * Bc * C_lo * rb_lo : 0.0;
-            const double U = r < NZ - 2 ? -Ak * Bc * C_hi * rb_hi : 0.0;
-            const double D = 1.0 + Ak * Bc * (C_hi + C_lo) * rbr;
-            const double G_ = (alpha * ((ps_hi - ps_lo) - (pr.p0(r + 1) - pr.p0(r))) +
-                               a1 * (double(pn[t + 2]) - double(pn[t + 1]))) *
-                              idz;
-            const double R = wo(t + 1) - dts * inv_rbr * G_ - Ak * (C_hi * e_hi - C_lo * e_lo);
-            const double piv = D - Aa * cp;
-            if (!(piv > 0.0) || !isfinite(piv)) ok = false;
-            const double inv_piv = rcp_nr(piv);
-            c1[t] = U * inv_piv;
-            a1s[t] = (t == 0 ? Aa : -Aa * ap) * inv_piv;
-            d1[t] = (R - Aa * dp) * inv_piv;
-            cp = c1[t];
-            ap = a1s[t];
-            dp = d1[t];
-            rb_lo = rb_mid;
-            rb_mid = rb_hi;
-            C_lo = C_hi;
-            ps_lo = ps_hi;
-            e_lo = e_hi;
-        }
-        else
-        {
-            c1[t] = a1s[t] = d1[t] = 0.0;
-        }
-    }
-    // the first row back-eliminated: x_{s0} = dt0 - at0 L' - ct0 L (the last row is L itself)
-    double dt0 = 0.0, at0 = 0.0, ct0 = -1.0;
-#pragma unroll
-    for (int t = kSegRows - 2; t >= 0; --t)
-    {
-        if (t < m - 1)
-        {
-            dt0 = d1[t] - c1[t] * dt0;
-            at0 = a1s[t] - c1[t] * at0;
-            ct0 = -c1[t] * ct0;
-        }
-    }
-
-    // 3. the system of the runs' last unknowns L_p, one row per run thread:
-    // a1 L_{p-1} + (1 - c1 at') L_p - c1 ct' L_{p+1} = d1 - c1 dt' (primes:
-    // run p + 1's first row), solved by cyclic reduction over the kSegments
-    // run threads of the column in LDS (log2(kSegments) steps of stride 1, 2,
-    // 4, ..., double buffered so one barrier per step suffices). Runs past the
-    // column and non-interior columns carry identity rows.
-    double* const nb = ex;                 // [3][kBlock]: at0, ct0, dt0 of each run
-    double* const rbuf = ex + 3 * kBlock;  // [2][4][kBlock]: reduced rows (sub, dia, sup, rhs)
-    nb[0 * kBlock + tid] = at0;
-    nb[1 * kBlock + tid] = ct0;
-    nb[2 * kBlock + tid] = dt0;
-    okv[tid] = ok ? 1 : 0;
-    __syncthreads();
-    double sub = 0.0, dia = 1.0, sup = 0.0, rhs = 0.0;
-    if (m > 0)
-    {
-        const int un = tid + kSegCols;
-        const bool more = p + 1 < runs;
-        const double aN = more ? nb[0 * kBlock + un] : 0.0;
-        const double cN = more ? nb[1 * kBlock + un] : 0.0;
-        const double dN = more ? nb[2 * kBlock + un] : 0.0;
-        sub = ap;
-        dia = 1.0 - cp * aN;
-        sup = -cp * cN;
-        rhs = dp - cp * dN;
-    }
-    bool col_ok = true;
-    for (int q = 0; q < runs; ++q) col_ok = col_ok && okv[q * kSegCols + col] != 0;
-#pragma unroll
-    for (int st = 0; st < kSegSteps; ++st)
-    {
-        const int stride = 1 << st;
-        double* const b = rbuf + (st & 1) * 4 * kBlock;
-        b[0 * kBlock + tid] = sub;
-        b[1 * kBlock + tid] = dia;
-        b[2 * kBlock + tid] = sup;
-        b[3 * kBlock + tid] = rhs;
         __syncthreads();
-        double k1 = 0.0, k2 = 0.0, nsub = 0.0, nsup = 0.0, ndia = dia, nrhs = rhs;
-        if (p - stride >= 0)
+        if (kk < NZ - 1)
         {
-            const int u = tid - stride * kSegCols;
-            k1 = sub * rcp_nr(b[1 * kBlock + u]);
-            nsub = -k1 * b[0 * kBlock + u];
-            ndia -= k1 * b[2 * kBlock + u];
-            nrhs -= k1 * b[3 * kBlock + u];
+#pragma unroll
+            for (int e = 0; e < V; ++e) b[e] -= bs[cell + CW + e];
         }
-        if (p + stride < kSegments)
+        __syncthreads();
+        if (active)
         {
-            const int u = tid + stride * kSegCols;
-            k2 = sup * rcp_nr(b[1 * kBlock + u]);
-            nsup = -k2 * b[2 * kBlock + u];
-            ndia -= k2 * b[0 * kBlock + u];
-            nrhs -= k2 * b[3 * kBlock + u];
+#pragma unroll
+            for (int e = 0; e < V; ++e) bs[cell + e] = b[e];
         }
-        sub = nsub;
-        sup = nsup;
-        dia = ndia;
-        rhs = nrhs;
-        if (m > 0 && (!(dia > 0.0) || !isfinite(dia))) col_ok = false;
-    }
-    const double Lp = rhs * rcp_nr(dia);
-    lv[tid] = Lp;
-    okv[kBlock + tid] = col_ok ? 1 : 0;
-    __syncthreads();
-    if (m <= 0) return;  // no barrier after this point
-    for (int q = 0; q < runs; ++q) col_ok = col_ok && okv[kBlock + q * kSegCols + col] != 0;
+        __syncthreads();
 
-    // 4. back substitution from the top of the run down; each cell s0 + t + 1 is
-    // finalised once both of its faces are known (the face above the run is
-    // run p + 1's first unknown, the same expression and operands as there)
-    // theta and the mass flux of the cells this run finalises (no other run
-    // writes them) are loaded only now to keep them out of the elimination's
-    // registers; rho' and rho* of levels s0 .. s0 + m + 1 are read again here rather than
-    // kept: rho' is not written by this kernel, and rho* of a cell is
-    // overwritten only by the run that finalises it, after this read
-#pragma unroll
-    for (int q = 1; q < NQ; ++q)
-    {
-        if (q <= m + 2)
+        // 2. rows 0 .. h-1 upwards (first wave) and n-1 .. n-h downwards (second); an odd one is left between
+        const int n = NZ - 1, h = n / 2, lane = tid & 63, half = tid >> 6;
+        const bool chain = half < 2 && lane < CW;
+        double cp = 0.0, dp = 0.0, least = 1.0;
+        if (chain)
         {
-            const std::size_t c = c0 + std::size_t(lev(q)) * sz;
-            rp[q] = rp_in[c];
-            if (q >= (p == 0 ? 1 : 2) && q <= m + 1)
+            __builtin_amdgcn_s_setprio(3);  // the workgroup's other waves wait for these
+            if (half == 0) eliminate<CW>(gs + lane, bs + lane, h, cp, dp, least);
+            else eliminate<-CW>(gs + n * CW + lane, bs + (n - 1) * CW + lane, h, cp, dp, least);
+            xs[(2 * half) * CW + lane] = cp;
+            xs[(2 * half + 1) * CW + lane] = dp;
+        }
+        __syncthreads();
+        if (chain)
+        {
+            const double co = xs[(2 - 2 * half) * CW + lane], dpo = xs[(3 - 2 * half) * CW + lane];
+            double y;
+            if (n & 1)
             {
-                rs[q] = rp_out[c];
-                tq[q] = th[c];
-                if (acc && !first) mq[q] = mfz[c];
+                // the middle row, between the last rows of both halves
+                const double gl = gs[h * CW + lane], gu = gs[(h + 1) * CW + lane];
+                const double cl = half ? co : cp, dl = half ? dpo : dp, cu = half ? cp : co, du = half ? dp : dpo;
+                const double piv = 1.0 + gl + gu - fma(gl, cl, gu * cu);
+                least = fmin(least, piv);
+                y = (bs[h * CW + lane] + fma(gl, dl, gu * du)) * rcp_nr(piv);
+                xs[4 * CW + lane] = y;  // both halves do the same operations, so store the same value
+                y = fma(cp, y, dp);
             }
+            else
+            {
+                const double det = fma(-cp, co, 1.0);
+                least = fmin(least, det);
+                y = fma(cp, dpo, dp) * rcp_nr(det);
+            }
+            if (half == 0)
+            {
+                bs[(h - 1) * CW + lane] = y;
+                y = substitute<CW>(gs + (h - 1) * CW + lane, bs + (h - 1) * CW + lane, h, y);
+            }
+            else
+            {
+                bs[(n - h) * CW + lane] = y;
+                y = substitute<-CW>(gs + (n - h + 1) * CW + lane, bs + (n - h) * CW + lane, h, y);
+            }
+            // stored by every lane: a branch here would be the last of the enclosing one
+            bad[half * CW + lane] = least > 0.0 && isfinite(y) ? 0 : 1;
+            __builtin_amdgcn_s_setprio(0);
         }
+        __syncthreads();
     }
-    const double Lm = p > 0 ? lv[tid - kSegCols] : 0.0;
-    // old w, density and stored new w of the face above the run (face s0 + m)
-    double wo_e = 0.0, rc_e = 0.0, rc_e1 = 0.0;
+    const Vec<S> mz = FIRST ? Vec<S>(S(0)) : ldv<S>(f.mfz, c);
+    // 3. w and the off-centred mass flux of the upper face, then the cells
 #pragma unroll
-    for (int q = 1; q < NQ - 1; ++q)
-        if (q == m + 1)
-        {
-            wo_e = wo(q);
-            rc_e = rc_at(q);
-            rc_e1 = rc_at(q + 1);
-        }
-    double rb_up = rb_of(m + 1, rc_e, rc_e1);
-    double rc_up = rc_e;  // density of the cell above the current face
-    double w_up = 0.0;
-    if (s0 + m < n)
+    for (int e = 0; e < V; ++e) b[e] = 0.0;
+    if (solve)
     {
-        const int u = tid + kSegCols;
-        const double x = col_ok ? nb[2 * kBlock + u] - nb[0 * kBlock + u] * Lp - nb[1 * kBlock + u] * lv[u] : wo_e;
-        w_up = double(S(clamp_store<S>(x, 0.0, -bd.wind_v, bd.wind_v)));
-    }
-    auto finalise = [&](int q, double rb_top, double w_top, double rb_bot, double w_bot) {
-        // cell s0 - 1 + q: upper face q, lower face q - 1
-        const int kc = s0 - 1 + q;
-        const std::size_t cc = c0 + std::size_t(kc) * sz;
-        const double ft = kc < NZ - 1 ? rb_top * (alpha * w_top + a1 * wo(q)) : 0.0;
-        const double fb = kc >= 1 ? rb_bot * (alpha * w_bot + a1 * wo(q - 1)) : 0.0;
-        if (acc) mfz[cc] = S((first ? 0.0 : double(mq[q])) + weight * ft);
-        const double rstar = pr.rho0(kc) + double(rs[q]);
-        const RhoP<S> o = density_eos<S>(bd, pr, kc, rstar - dts * idz * (ft - fb), double(tq[q]));
-        rp_out[cc] = o.r;
-        pp[cc] = o.p;
-    };
-    double x_up = Lp;  // unclamped solution of the face above
+        if (kk < NZ - 1)
+        {
+            const bool mid = ((NZ - 1) & 1) && k == (NZ - 1) / 2;
+            Vec<S> wn = wo;
 #pragma unroll
-    for (int t = kSegRows - 1; t >= 0; --t)
-    {
-        if (t < m)
-        {
-            double x = t == m - 1 ? Lp : t == 0 ? dt0 - at0 * Lm - ct0 * Lp : d1[t] - c1[t] * x_up - a1s[t] * Lm;
-            x_up = x;
-            if (!col_ok) x = wo(t + 1);
-            const double c = clamp_store<S>(x, 0.0, -bd.wind_v, bd.wind_v);
-            w[c0 + std::size_t(s0 + t) * sz] = S(c);
-            const double wn = double(S(c));
-            const double rc_lo = rc_at(t + 1);
-            const double rb = rb_of(t + 1, rc_lo, rc_up);
-            finalise(t + 2, rb_up, w_up, rb, wn);
-            w_up = wn;
-            rb_up = rb;
-            rc_up = rc_lo;
+            for (int e = 0; e < V; ++e)
+            {
+                const int i = i0 + e, col = (tid % LL) * V + e;
+                if (i >= 1 && i < NX - 1)
+                {
+                    const bool ok = (bad[col] | bad[CW + col]) == 0;
+                    const double rb = 0.5 * ((r0 + double(r[e])) + (r0u + double(rzp[e])));
+                    const double y = mid ? xs[4 * CW + col] : bs[cell + e];
+                    const double x = ok ? y * rcp_nr(rb) : double(wo[e]);
+                    wn[e] = S(clamp_store<S>(x, 0.0, -bd.wind_v, bd.wind_v));
+                    b[e] = rb * (alpha * double(wn[e]) + a1 * double(wo[e]));
+                }
+                gs[cell + e] = b[e];
+            }
+            stv<S>(f.w, c, wn);
         }
+        __syncthreads();
     }
-    if (p == 0) finalise(1, rb_up, w_up, 0.0, 0.0);  // cell 0 above the ground face
+    if (!active) return;  // no barrier after this point
+    Vec<S> rn, pw, mzn;
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+    {
+        const double fl = solve && k > 0 ? gs[cell - CW + e] : 0.0;
+        mzn[e] = S(double(mz[e]) + weight * b[e]);
+        const double rstar = r0 + double(rs[e]);
+        const RhoP<S> o = density_eos<S>(bd, pr, k, rstar - cdt * (b[e] - fl), double(th[e]));
+        rn[e] = o.r;
+        pw[e] = o.p;
+    }
+    stv<S>(f.mfz, c, mzn);
+    stv<S>(rp_out, c, rn);
+    stv<S>(f.pp, c, pw);
 }
 
 // Backward momentum update of substep s with the new rho' (buffer
@@ -3033,6 +2898,7 @@ void fill_geometry(MemberArgs& a, int tile_w, int k_chunks, int xcd_remap)
     G.tiles_y = (a.g.ny + G.tile_h - 1) / G.tile_h;
     G.k_chunks = std::max(1, std::min(k_chunks, a.g.nz));
     G.xcd_remap = xcd_remap ? 1 : 0;
+    G.solve_lanes = solve_lanes(a.g.nz);
 }
 
 int work_items(const MemberArgs& a, WorkKind kind)
@@ -3049,7 +2915,7 @@ int work_items(const MemberArgs& a, WorkKind kind)
     case W_SN: return lin(std::size_t(a.g.nx) * a.g.nz);
     case W_SEED: return lin(std::size_t(std::max(a.g.nx, a.g.ny)) * a.g.nz);
     case W_DIAG: return kDiagBlocksPerMember;
-    case W_SEGCOL: return ((a.g.nx + kSegCols - 1) / kSegCols) * a.g.ny;
+    case W_SOLVE: return int(a.g.plane() / std::size_t(G.solve_lanes * G.vec));
     case W_TILECELL: return tiles * G.k_chunks * ((a.g.nz + G.k_chunks - 1) / G.k_chunks);
     default: return 0;
     }
@@ -3093,33 +2959,34 @@ namespace
 {
 
 template <class K, class... Args>
-void launch_map_lds(Launcher& L, const char* name, K kernel, const BatchView& b, int subset, WorkKind kind,
-                    std::size_t lds_bytes, Args... args)
+void launch_map(Launcher& L, const char* name, K kernel, const BatchView& b, int subset, WorkKind kind,
+                Args... args)
 {
     const BlockMap& m = b.maps[subset][kind];
     if (m.blocks <= 0) return;
     hipEvent_t ev;
     L.begin(name, ev);
-    hipLaunchKernelGGL(kernel, dim3(unsigned(m.blocks)), dim3(kBlock), lds_bytes, L.stream, b.args, m.entries,
-                       args...);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(m.blocks)), dim3(kBlock), 0, L.stream, b.args, m.entries, args...);
     L.end(name, ev);
 }
 
-template <class K, class... Args>
-void launch_map(Launcher& L, const char* name, K kernel, const BatchView& b, int subset, WorkKind kind,
-                Args... args)
+// The column solve of the members with LL lanes per level, whose deepest has
+// nz levels: one thread per LL-th of a level (at least two waves), the staged
+// profiles, two doubles per cell and the meeting rows in LDS.
+template <class S, int LL>
+void launch_hevi_solve(Launcher& L, const BatchView& b, int s, bool first, int nz)
 {
-    launch_map_lds(L, name, kernel, b, subset, kind, 0, args...);
-}
-
-// LDS bytes of the staged base-state profiles for the deepest member of a batch.
-std::size_t profile_lds_bytes(const BatchView& b) { return std::size_t(kLdsProfiles) * b.max_nz * sizeof(double); }
-
-// LDS of the partitioned column solve: the profiles, 12 doubles per thread
-// (run ends, two buffers of reduced rows, last unknowns) and 2 pivot verdicts.
-std::size_t segment_lds_bytes(const BatchView& b)
-{
-    return profile_lds_bytes(b) + std::size_t(12) * kBlock * sizeof(double) + std::size_t(2) * kBlock * sizeof(int);
+    constexpr int CW = LL * 16 / int(sizeof(S));
+    const BlockMap& m = b.maps[S_HEVI][W_SOLVE];
+    if (m.blocks <= 0) return;
+    const unsigned threads = std::max(128u, unsigned(LL * nz + 63) / 64u * 64u);
+    const std::size_t lds = std::size_t(nz) * (kLdsProfiles + 2 * CW) * sizeof(double) + 5 * CW * sizeof(double) +
+                            2 * CW * sizeof(int);
+    const auto kernel = first ? k_hevi_solve<S, true, LL> : k_hevi_solve<S, false, LL>;
+    hipEvent_t ev;
+    L.begin("acoustic_hevi_solve", ev);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(m.blocks)), dim3(threads), lds, L.stream, b.args, m.entries, s);
+    L.end("acoustic_hevi_solve", ev);
 }
 
 template <class S>
@@ -3148,14 +3015,10 @@ void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumu
 {
     launch_map(L, "acoustic_forward", k_acoustic_forward<S>, b, S_EXPLICIT, W_CELL, s, int(accumulate),
                int(init_at_first));
-    launch_map(L, "acoustic_hevi_explicit", k_hevi_explicit<S>, b, S_HEVI, W_CELL, s, int(accumulate),
-               int(init_at_first));
-    if (b.any_hevi_seg)
-        launch_map_lds(L, "acoustic_hevi_column_seg", k_hevi_column_seg<S>, b, S_HEVI, W_SEGCOL,
-                       segment_lds_bytes(b), s, int(accumulate), int(init_at_first));
-    if (b.any_hevi_serial)
-        launch_map_lds(L, "acoustic_hevi_column", k_hevi_column<S>, b, S_HEVI, W_COLUMN, profile_lds_bytes(b), s,
-                       int(accumulate), int(init_at_first));
+    const bool first = init_at_first && s == 0;
+    if (b.hevi_nz[0] > 0) launch_hevi_solve<S, 4>(L, b, s, first, b.hevi_nz[0]);
+    if (b.hevi_nz[1] > 0) launch_hevi_solve<S, 2>(L, b, s, first, b.hevi_nz[1]);
+    if (b.hevi_nz[2] > 0) launch_hevi_solve<S, 1>(L, b, s, first, b.hevi_nz[2]);
     launch_map(L, "acoustic_momentum", k_momentum<S>, b, S_ALL, W_CELL, s);
 }
 

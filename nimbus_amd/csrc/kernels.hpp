@@ -47,7 +47,6 @@ struct DevFields
     void *tth, *tqv, *tqc, *tqr;                         // transported scalars before microphysics
     void* flux[12];                                      // per scalar: x, y, z face fluxes (7 alias dead slots)
     float *rl_qv, *rl_qc, *rl_qr;                        // PD limiter factors
-    double *tri_c, *tri_r;                               // HE-VI Thomas coefficients (FP64)
     float *rad_w, *rad_e, *rad_s, *rad_n;                // KW78 radiative stashes
     double* rain;                                        // accumulated surface rain [ny][nx]
     double* base;                                        // kBaseCount * nz FP64 profiles
@@ -63,7 +62,7 @@ struct StepParams
     double mf_weight;   // retained mass-flux weight per substep (dts / dt in the large step)
     int substeps;
     int acoustic_mode;
-    int hevi_seg;       // the member's HE-VI columns are solved in the partitioned form (fixed per member)
+    int hevi_seg;       // the member's column-solve form reads PARTITIONED (fixed per member)
     double hevi_alpha;  // (1 + beta) / 2
     double coriolis_f;
     int bc_west, bc_east, bc_south, bc_north, bc_bottom, bc_top;
@@ -105,6 +104,9 @@ struct MemberGeom
     // padded [j][i] plane (`runs` per level) instead of column tiles at one
     // level, per-column work in runs of kBlock consecutive columns
     int linear, runs;
+    // HE-VI solve: 16-byte lanes per level of a workgroup (solve_lanes(nz)) and
+    // elements per 16 bytes (fixed by the storage type at creation)
+    int solve_lanes, vec;
 };
 
 struct MemberArgs
@@ -124,42 +126,28 @@ enum WorkKind
     W_SN = 3,      // 256 (i, k) rows of the south/north faces
     W_SEED = 4,    // 256 entries of the radiative stashes
     W_DIAG = 5,    // one of kDiagBlocksPerMember reduction blocks
-    W_SEGCOL = 6,  // kSegCols consecutive columns of one row, kSegments runs of faces each
+    W_SOLVE = 6,   // solve_lanes x 16 bytes consecutive columns of one row, whole columns (HE-VI solve)
     W_TILECELL = 7,  // one tile of columns at one level whatever the geometry (wide stencils)
     W_KINDS = 8
 };
 
-// Partitioned HE-VI column solve: a column of nz - 1 unknown faces is split
-// into kSegments runs of at most kSegRows faces, one thread per run, for
-// columns of at most kSegMaxNz levels. The form is a property of the member,
-// fixed at creation (StepParams::hevi_seg, default from the member's own
-// shape, nimbus_hip_member_set_column_solve to override), so a member's
-// arithmetic never depends on the batch it runs in. Default: FP64 members
-// always (measured faster than the sequential sweep, which is memory-bound
-// on its FP64 coefficient arrays); FP32-storage members with fewer than
-// kSegSmallMemberColumns columns, which alone cannot fill the GPU with one
-// thread per column (measured: 64x64x40 0.49 -> 0.36 ms per large step,
-// 160x160x80 1.29 -> 1.23; by 255x255 columns the partitioned form's
-// latency-bound FP64 elimination is the slower one, and at 400x400x100
-// 9.06 against 8.04). Deeper columns take the sequential sweep, which keeps
-// its FP64 coefficients in two cell-sized scratch arrays (allocated for every
-// member that may be solved by it: FP32 storage or more than kSegMaxNz levels).
-#ifndef NIMBUS_SEG_ROWS
-#define NIMBUS_SEG_ROWS 8
-#endif
-constexpr int kSegRows = NIMBUS_SEG_ROWS;        // faces per run (one thread)
-constexpr int kSegments = 128 / kSegRows;        // runs per column: columns of up to 129 levels
-constexpr int kSegCols = 256 / kSegments;        // columns per 256-thread workgroup
-constexpr int kSegSteps = kSegments == 64 ? 6 : kSegments == 32 ? 5 : kSegments == 16 ? 4 : kSegments == 8 ? 3 : 0;
-static_assert(kSegSteps > 0 && (1 << kSegSteps) == kSegments, "runs per column must be 8, 16, 32 or 64");
-constexpr int kSegMaxNz = kSegments * kSegRows + 1;
-constexpr int kSegSmallMemberColumns = 32768;
+// Column-solve form of a member (nimbus_hip_member_set_column_solve), fixed at
+// creation: PARTITIONED for FP64 members and for FP32 members of fewer than
+// kSweepColumns columns, both up to kSegMaxNz levels. A name that is accepted,
+// refused and reported; k_hevi_solve solves the columns of either form with
+// the same operations.
+constexpr int kSegMaxNz = 129;
+constexpr int kSweepColumns = 32768;
 constexpr bool hevi_partitioned_always(int elem, int nz) { return elem == 8 && nz <= kSegMaxNz; }
-// Default column-solve form of a member: 1 = partitioned, 0 = sequential sweep.
 constexpr int hevi_default_seg(int elem, int nx, int ny, int nz)
 {
-    return nz <= kSegMaxNz && (elem == 8 || long(nx) * long(ny) < long(kSegSmallMemberColumns)) ? 1 : 0;
+    return nz <= kSegMaxNz && (elem == 8 || long(nx) * long(ny) < long(kSweepColumns)) ? 1 : 0;
 }
+
+// HE-VI solve: lanes of 16 bytes per level, so that a workgroup of one thread
+// per lane holds a whole column of up to 1,024 levels (runtime grid check) in
+// at most 1,024 threads.
+constexpr int solve_lanes(int nz) { return nz <= 256 ? 4 : nz <= 512 ? 2 : 1; }
 
 // Member subsets a launch can be restricted to.
 enum MemberSubset
@@ -191,9 +179,8 @@ struct BatchView
     int any_sponge_unfused = 0;  // a member with sponges and no SGS or diffusion pass to apply them in
     int any_diffusion = 0;       // a member with explicit diffusion
     int any_kessler_adaptive = 0; // a member whose microphysics subcycles follow its sedimentation limit
-    int any_hevi_seg = 0;        // HE-VI members solved in the partitioned form
-    int any_hevi_serial = 0;     // HE-VI members solved by the sequential sweep
     int max_nz = 0;
+    int hevi_nz[3] = {0, 0, 0};  // deepest of the HE-VI members with 4, 2 and 1 lanes per level
     int elem = 4;
     BlockMap maps[S_SUBSETS][W_KINDS];
 };

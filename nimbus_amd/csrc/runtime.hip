@@ -82,7 +82,8 @@ Layout layout_for(const DevGrid& g, int elem, bool hevi, int lateral = 0)
     Layout L{};
     L.field = align256(g.cells() * std::size_t(elem));
     L.rl = align256(g.cells() * sizeof(float));
-    // FP64 Thomas coefficients: only the sequential sweep keeps them in memory
+    // two FP64 arrays that a member whose form may be SEQUENTIAL holds: part of
+    // its published size, which admission counts on; no kernel uses them
     L.tri = hevi && !hevi_partitioned_always(elem, g.nz) ? align256(g.cells() * sizeof(double)) : 0;
     L.rad_w = align256(std::size_t(g.ny) * g.nz * sizeof(float));
     L.rad_s = align256(std::size_t(g.nx) * g.nz * sizeof(float));
@@ -303,7 +304,7 @@ int set_column_solve(Member& m, int form)
         seg = 1;
         break;
     case NIMBUS_COLUMN_SOLVE_SEQUENTIAL:
-        if (!m.args.f.tri_c)
+        if (hevi_partitioned_always(m.elem, nz))
             return fail(NIMBUS_EINVAL, "set_column_solve: FP64 members of at most 129 levels hold no scratch for the "
                                        "sequential sweep");
         seg = 0;
@@ -319,6 +320,7 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
     m.desc = desc;
     m.elem = desc.precision == NIMBUS_PRECISION_MIXED ? 4 : 8;
     m.args.g = dev_grid(desc.grid, m.elem);
+    m.args.geo.vec = 16 / m.elem;
     const int nz = desc.grid.nz;
     const bool hevi = desc.config.acoustic_mode == NIMBUS_ACOUSTIC_HEVI;
     m.host_base.assign(std::size_t(kBaseCount) * nz, 0.0);
@@ -415,13 +417,7 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
     f.rl_qv = reinterpret_cast<float*>(p); p += L.rl;
     f.rl_qc = reinterpret_cast<float*>(p); p += L.rl;
     f.rl_qr = reinterpret_cast<float*>(p); p += L.rl;
-    f.tri_c = nullptr;
-    f.tri_r = nullptr;
-    if (L.tri)
-    {
-        f.tri_c = reinterpret_cast<double*>(p); p += L.tri;
-        f.tri_r = reinterpret_cast<double*>(p); p += L.tri;
-    }
+    p += 2 * L.tri;
     f.rad_w = reinterpret_cast<float*>(p); p += L.rad_w;
     f.rad_e = reinterpret_cast<float*>(p); p += L.rad_w;
     f.rad_s = reinterpret_cast<float*>(p); p += L.rad_s;
@@ -563,9 +559,8 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
         b.view.any_kessler_adaptive |= m->args.p.kessler_adaptive;
         if (m->args.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI)
         {
-            const bool part = m->args.p.hevi_seg != 0;
-            b.view.any_hevi_seg |= part;
-            b.view.any_hevi_serial |= !part;
+            int& nz = b.view.hevi_nz[m->args.geo.solve_lanes == 4 ? 0 : m->args.geo.solve_lanes == 2 ? 1 : 2];
+            nz = std::max(nz, m->args.g.nz);
         }
         remap = remap && m->xcd_remap;
     }

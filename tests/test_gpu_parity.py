@@ -404,6 +404,23 @@ def test_mixed_deep_columns_sequential_match_fp64_oracle(hip_ctx):
     check_mixed(out, ref, "deep mixed")
 
 
+@pytest.mark.parametrize("nx, ny, nz", [(5, 5, 4), (18, 5, 5), (15, 6, 40), (33, 7, 129), (5, 6, 130), (17, 5, 256),
+                                        (9, 5, 257), (6, 5, 513), (5, 5, 1024)])
+def test_column_solve_depths_match_fp64_oracle(hip_ctx, nx, ny, nz):
+    """The in-LDS column solve at the edges of its workgroup shapes (4, 2 and 1
+    lanes per level; odd and even middle rows; rows that fill no whole
+    workgroup), of FP64 and FP32-storage members, against the FP64 oracle."""
+    g, base, st64 = small_case(nx=nx, ny=ny, nz=nz, dz=min(500.0, 20000.0 / nz), cloudy=True, wind_noise=1.0,
+                               dtype=np.float64)
+    cfg = L.step_config(3.0, 6, acoustic_mode=L.ACOUSTIC_HEVI, lateral=L.BC_RIGID_SLIP)
+    ref, _ = O.large_steps(oracle_grid(g), base, O.from_step_config(cfg), st64, 2, np.float64)
+    out, _ = _run_member(hip_ctx, g, base, cfg, st64, L.PRECISION_FP64, 2)
+    check_fp64(out, ref, f"column {nx}x{ny}x{nz}", False)
+    st = {k: (v.astype(np.float32) if k in L.FIELDS else v) for k, v in st64.items()}
+    out, _ = _run_member(hip_ctx, g, base, cfg, st, L.PRECISION_MIXED, 2)
+    check_mixed(out, ref, f"mixed column {nx}x{ny}x{nz}")
+
+
 # Sponge settings scaled to the 7 km deep test domain: upper sponge from 4 km,
 # 4-cell w absorber, 3-cell lateral band.
 SMALL_SPONGE = {"z_d": 4000.0, "alpha": 0.05, "w_cells": 4, "w_alpha": 0.2, "lateral_cells": 3,
