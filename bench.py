@@ -49,7 +49,7 @@ HBM_PEAK_GBS = 8000.0
 PHASES = {
     "acoustic_substep": {"bytes_s": 17, "per_step": "substeps",
                          "kernels": ("acoustic_forward", "acoustic_hevi_solve", "acoustic_momentum", "acoustic_commit",
-                                     "bc_west_east", "bc_south_north", "bc_vertical", "seed_radiation")},
+                                     "boundary_closure")},
     "slow_rk2_apply": {"bytes_s": 44, "per_step": 1, "kernels": ("slow_stage1", "slow_stage2")},
     "scalar_transport": {"bytes_s": 13, "per_step": 1,
                          "kernels": ("transport_flux", "transport_limiter", "transport_update")},
@@ -95,8 +95,8 @@ def phase_table(tab, cells, elem, n_sub, steps, traffic=None):
 ALGO_PER_CELL = {
     # read u v w rho' theta mfx mfy mfz; write rho'(new) p' mfx mfy mfz
     "acoustic_forward": (13, 0),
-    # read rho'(new) p' u v w; write u v, and w for explicit members
-    "acoustic_momentum": {"explicit": (8, 0), "hevi": (7, 0)},
+    # read rho'(new) p' u v; write u v, and read and write w for explicit members
+    "acoustic_momentum": {"explicit": (8, 0), "hevi": (6, 0)},
     # HE-VI horizontal part and column solve: read rho' u v theta mfx mfy p' w mfz;
     # write mfx mfy w mfz rho' p'
     "acoustic_hevi_solve": (15, 0),

@@ -167,30 +167,6 @@ __device__ __forceinline__ Work work_of(const int2* __restrict__ map)
     return Work{e.x, e.y};
 }
 
-// One thread per (i, j) column: of a tile_w x tile_h tile of columns, or of
-// a run of kBlock consecutive columns in the linear geometry.
-struct Column
-{
-    int i, j;
-};
-
-__device__ __forceinline__ Column column_of(const MemberArgs& A, int local)
-{
-    const MemberGeom& geo = A.geo;
-    if (geo.linear)
-    {
-        // run `local` of kBlock consecutive columns in row-major order: a
-        // level's loads of a workgroup are one or two contiguous segments
-        const unsigned col = unsigned(local) * unsigned(kBlock) + threadIdx.x;
-        const unsigned nx = unsigned(A.g.nx);
-        const unsigned j = col / nx;
-        return Column{int(col - j * nx), int(j)};
-    }
-    const int ty = local / geo.tiles_x, tx = local - ty * geo.tiles_x;
-    const int tid = int(threadIdx.x);
-    return Column{tx * geo.tile_w + (tid & (geo.tile_w - 1)), ty * geo.tile_h + tid / geo.tile_w};
-}
-
 // One cell per thread. Column tiles (tile_cell_of): tile t of the member at
 // level k; the local work index runs k fastest within a vertical chunk
 // (k_chunks chunks of kz levels), then over the column tiles, then over the
@@ -692,44 +668,21 @@ __device__ __forceinline__ RhoP<S> acoustic_forward(const DevGrid& g, const Acou
     return o;
 }
 
-// Backward momentum update of one cell with the new rho' and p' of the cell
-// and its +x, +y, +z neighbours (acoustic_cgrid_fast.cpp:159-215).
+// Pressure-gradient tendency of the face between a cell and its upper
+// neighbour in one direction (acoustic_cgrid_fast.cpp:159-215): new p' of both,
+// the face density, 1 / spacing. FP32 storage forms it in FP32, as the
+// reference rounds it to FP32 before the update.
 template <class S>
-__device__ __forceinline__ void momentum_update(const DevGrid& g, double r0, double r0p, const Bounds& bd,
-                                                double dts, int i, int j, int k, RhoP<S> cc, RhoP<S> xp, RhoP<S> yp,
-                                                RhoP<S> zp, double u, double v, double w, bool skip_w, gptr<S> un,
-                                                gptr<S> vn, gptr<S> wn, std::size_t c)
+__device__ __forceinline__ double pressure_gradient(S lo, S hi, double rho_face, double inv_d)
 {
-    const int NX = g.nx, NY = g.ny, NZ = g.nz;
-    double du = 0.0, dv = 0.0, dw = 0.0;
-    const bool interior = i >= 1 && i < NX - 1 && j >= 1 && j < NY - 1 && k < NZ - 1;
-    if (interior)
+    if constexpr (sizeof(S) == sizeof(float))
     {
-        const double rc = r0 + double(cc.r);
-        const double rx = 0.5 * (rc + (r0 + double(xp.r)));
-        const double ry = 0.5 * (rc + (r0 + double(yp.r)));
-        const double rz = 0.5 * (rc + (r0p + double(zp.r)));
-        if constexpr (sizeof(S) == sizeof(float))
-        {
-            // FP32 tendency, as the reference rounds it to FP32 before the update
-            auto safe_f = [](float r) { return isfinite(r) && r > 1.0e-6f ? r : 1.0f; };
-            auto fin = [](float x) { return isfinite(x) ? x : 0.0f; };
-            const float pc = float(cc.p);
-            du = double(fin(-(float(xp.p) - pc) * float(g.idx) / safe_f(float(rx))));
-            dv = double(fin(-(float(yp.p) - pc) * float(g.idy) / safe_f(float(ry))));
-            dw = double(fin(-((float(zp.p) - pc) * float(g.idz)) / safe_f(float(rz))));
-        }
-        else
-        {
-            const double pc = double(cc.p);
-            du = finite0(-(double(xp.p) - pc) * g.idx / safe_rho(rx));
-            dv = finite0(-(double(yp.p) - pc) * g.idy / safe_rho(ry));
-            dw = finite0(-((double(zp.p) - pc) * g.idz) / safe_rho(rz));
-        }
+        const float r = float(rho_face);
+        const float t = -(float(hi) - float(lo)) * float(inv_d) / (isfinite(r) && r > 1.0e-6f ? r : 1.0f);
+        return double(isfinite(t) ? t : 0.0f);
     }
-    un[c] = S(clamp_store<S>(u + du * dts, 0.0, -bd.wind_h, bd.wind_h));
-    vn[c] = S(clamp_store<S>(v + dv * dts, 0.0, -bd.wind_h, bd.wind_h));
-    if (!(skip_w && interior)) wn[c] = S(clamp_store<S>(w + dw * dts, 0.0, -bd.wind_v, bd.wind_v));
+    else
+        return finite0(-(double(hi) - double(lo)) * inv_d / safe_rho(rho_face));
 }
 
 template <class S>
@@ -1147,45 +1100,19 @@ __global__ __launch_bounds__(1024) void k_hevi_solve(const MemberArgs* __restric
     stv<S>(f.pp, c, pw);
 }
 
-// Backward momentum update of substep s with the new rho' (buffer
-// (s + 1) & 1) and pressure, in place. HE-VI members keep the interior w the
-// column solve set; their ghost-column and lid w get the clamp only.
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_momentum(const MemberArgs* __restrict__ ma,
-                                                     const int2* __restrict__ map, int s)
-{
-    const Work wk = work_of(map);
-    const MemberArgs& A = ma[wk.m];
-    if (s >= A.p.substeps) return;
-    const Cell cl = cell_of(A, wk.local);
-    if (!cl.valid) return;
-    const DevGrid& g = A.g;
-    const int NX = g.nx, NY = g.ny, NZ = g.nz;
-    const int i = cl.i, j = cl.j, k = cl.k;
-    const DevFields& f = A.f;
-    const gptr<const S> __restrict__ rn = P<S>((s & 1) ? f.rp : f.rp2);
-    const gptr<const S> __restrict__ pp = P<S>(f.pp);
-    const auto u = P<S>(f.u);
-    const auto v = P<S>(f.v);
-    const auto w = P<S>(f.w);
-    const std::size_t sy = std::size_t(g.px), sz = g.plane();
-    const std::size_t c = g.at(i, j, k);
-    // neighbours clamped to the domain (the cell itself stands in for a missing one)
-    const std::size_t cxp = i < NX - 1 ? c + 1 : c, cyp = j < NY - 1 ? c + sy : c, czp = k < NZ - 1 ? c + sz : c;
-    RhoP<S> cc{rn[c], pp[c]}, xp{rn[cxp], pp[cxp]}, yp{rn[cyp], pp[cyp]}, zp{rn[czp], pp[czp]};
-    S uc = u[c], vc = v[c], wc = w[c];
-    const auto rho0 = slot(f.base, kBaseRho0, NZ);
-    double r0 = rho0[k], r0p = rho0[k < NZ - 1 ? k + 1 : k];
-    pin(cc.r); pin(cc.p); pin(xp.r); pin(xp.p); pin(yp.r); pin(yp.p); pin(zp.r); pin(zp.p);
-    pin(uc); pin(vc); pin(wc); pin(r0); pin(r0p);
-    momentum_update<S>(g, r0, r0p, A.p.bounds, A.p.dts, i, j, k, cc, xp, yp, zp, double(uc), double(vc), double(wc),
-                       A.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI, u, v, w, c);
-}
-
 // ---------------------------------------------------------------------
 // Boundary closure (boundary_conditions_cartesian_cgrid.cpp:798-1175):
 // west/east faces, then south/north, then the vertical closure; KW78
 // radiative faces integrate their FP32 stash when radiating.
+//
+// Every closed value depends on one cell between the lateral ghosts, so the
+// thread of that cell stores it everywhere it goes: into the ghost columns,
+// through them into the ghost rows, and from level NZ - 2 into the lid. The
+// momentum update closes the substep in its own stores that way, which takes
+// three launches (and their trips through memory) out of every substep.
+// Cells at coordinate 1, n - 3 or n - 2 of either axis are the edge cells,
+// the only ones whose values go into ghosts or onto another face; they are
+// taken by workgroups of their own, one wind component each.
 // ---------------------------------------------------------------------
 __device__ __forceinline__ float kw78_face(float prev, float phase, float grad, float dt, float inv_d, bool west_like)
 {
@@ -1196,187 +1123,308 @@ __device__ __forceinline__ float kw78_face(float prev, float phase, float grad, 
     return __fsub_rn(prev, c);
 }
 
-template <class S>
-struct BcBufs
+// One axis of an edge cell: coordinate q of n (never a ghost), the sides'
+// conditions, the stride. Tangential values go from low() and high() cells to
+// the ghosts; the face-normal wind also onto the high face n - 2, which an
+// open high side sets from n - 3.
+struct Axis
 {
-    gptr<S> u, v, w, rp, pp;
-    float dt_rad;
+    int n, q, lo, hi;
+    unsigned stride;  // bytes
+    __device__ __forceinline__ bool edge() const { return q == 1 || q >= n - 3; }
+    __device__ __forceinline__ bool open() const { return hi == NIMBUS_BC_RADIATIVE || hi == NIMBUS_BC_ZERO_GRADIENT; }
+    __device__ __forceinline__ bool wall() const { return hi == NIMBUS_BC_RIGID || hi == NIMBUS_BC_RIGID_SLIP; }
+    __device__ __forceinline__ bool low() const { return lo == NIMBUS_BC_PERIODIC ? q == n - 2 : q == 1; }
+    __device__ __forceinline__ bool high() const { return hi == NIMBUS_BC_PERIODIC ? q == 1 : q == n - 2; }
+    // the cell that stores the normal wind of the low ghost (an open high
+    // side's own where the ghost is the copy of that side's face) and of the
+    // high ghost, and whether a cell stores its own
+    __device__ __forceinline__ bool normal_low() const
+    {
+        return lo == NIMBUS_BC_PERIODIC && open() ? q == n - 3 : low();
+    }
+    __device__ __forceinline__ bool normal_high() const { return open() ? q == n - 3 : high(); }
+    __device__ __forceinline__ bool normal_self() const { return !(open() && q == n - 2); }
 };
 
-// Buffers current after substep s (s < 0: home buffers, no radiation):
-// u, v, w live in their home buffers, rho' in buffer (s + 1) & 1.
-template <class S>
-__device__ __forceinline__ bool bc_buffers(const MemberArgs& A, int s, BcBufs<S>& b)
-{
-    const DevFields& f = A.f;
-    if (s >= 0 && s >= A.p.substeps) return false;
-    const int par = s >= 0 ? ((s + 1) & 1) : 0;
-    b.u = P<S>(f.u);
-    b.v = P<S>(f.v);
-    b.w = P<S>(f.w);
-    b.rp = P<S>(par ? f.rp2 : f.rp);
-    b.pp = P<S>(f.pp);
-    b.dt_rad = s >= 0 ? float(A.p.dts) : 0.0f;
-    return true;
-}
+// Edge cells, level by level: the rows first, then what is left of the
+// columns, a row's three together.
+__host__ __device__ inline int edge_cells(int nx, int ny) { return 3 * (nx - 2) + 3 * (ny - 5); }
 
-// One lateral boundary pair of one row: the low face (ghost cell c, first
-// interior cell in) and the high face (interior face cell a, the one inside
-// it am, ghost cell gi) for the face-normal velocity n and the tangential
-// t1, t2. Every value is loaded before anything is stored, so the row costs
-// one round trip (periodic copies read a and in, which the other face does
-// not modify before, in the reference's order, they are read).
-template <class S>
-__device__ __forceinline__ void lateral_pair(gptr<S> n, gptr<S> t1, gptr<S> t2, gptr<S> rp, gptr<S> pp,
-                                             gptr<float> stash_lo, gptr<float> stash_hi, int bc_lo, int bc_hi,
-                                             bool radiate, float dt_rad, float inv_d, std::size_t c,
-                                             std::size_t in, std::size_t am, std::size_t a, std::size_t gi)
+__device__ __forceinline__ Cell edge_cell(const DevGrid& g, int t)
 {
-    const float cstar = 30.0f;
-    S n_in = n[in], t1_in = t1[in], t2_in = t2[in], rp_in = rp[in], pp_in = pp[in];
-    S n_a = n[a], t1_a = t1[a], t2_a = t2[a], rp_a = rp[a], pp_a = pp[a], n_am = n[am];
-    float s_lo = *stash_lo, s_hi = *stash_hi;
-    pin(n_in); pin(t1_in); pin(t2_in); pin(rp_in); pin(pp_in);
-    pin(n_a); pin(t1_a); pin(t2_a); pin(rp_a); pin(pp_a); pin(n_am); pin(s_lo); pin(s_hi);
-    // low face
-    if (bc_lo == NIMBUS_BC_PERIODIC)
+    auto third = [](int e, int n) { return e == 0 ? 1 : n - 4 + e; };  // 1, n - 3, n - 2
+    const int NX = g.nx, NY = g.ny, edges = edge_cells(NX, NY), rows = 3 * (NX - 2);
+    Cell c;
+    c.k = t / edges;
+    c.valid = c.k < g.nz;
+    t -= c.k * edges;
+    const int e = t / (NX - 2);
+    if (t < rows)
     {
-        n[c] = n_a; t1[c] = t1_a; t2[c] = t2_a; rp[c] = rp_a; pp[c] = pp_a;
+        c.i = 1 + (t - e * (NX - 2));
+        c.j = third(e, NY);
     }
     else
     {
-        if (bc_lo == NIMBUS_BC_RADIATIVE)
+        t -= rows;
+        c.j = 2 + t / 3;
+        c.i = third(t % 3, NX);
+    }
+    return c;
+}
+
+// Edge workgroup b of a member: wind component b % 3 (uniform) of 256 edge
+// cells, after the momentum update (MOM: of substep s, new rho' in rp) or as
+// stored; closed wherever it goes. The code is one loop over the lines
+// (coordinates of the tangential axis) that the value goes to, because a wave
+// comes through here once: unrolled over targets and components it was 2,000
+// instructions, whose fetch was most of the 4 us that it added to the update
+// of 48 x 48 x 40 cells.
+// s < 0: radiative faces stay as they are; s == 0 of an update that closes:
+// they start from the winds stored.
+template <class S, bool MOM>
+__device__ __forceinline__ void close_edges(const MemberArgs& A, int b, int s, gptr<S> rp)
+{
+    constexpr unsigned es = sizeof(S);
+    const DevGrid& g = A.g;
+    const StepParams& p = A.p;
+    const int q3 = b / 3, comp = b - 3 * q3;
+    const Cell cl = edge_cell(g, q3 * kBlock + int(threadIdx.x));
+    if (!cl.valid) return;
+    const int k = cl.k, NZ = g.nz;
+    const unsigned row = unsigned(g.px) * es, plane = unsigned(g.plane()) * es;
+    const Axis x{g.nx, cl.i, p.bc_west, p.bc_east, es}, y{g.ny, cl.j, p.bc_south, p.bc_north, row};
+    // N: the axis of the component (y for w, where it is tangential too), T: the other
+    const Axis N = comp == 0 ? x : y, T = comp == 0 ? y : x;
+    const auto f = P<S>(comp == 0 ? A.f.u : comp == 1 ? A.f.v : A.f.w);
+    const auto pp = P<S>(A.f.pp);
+    float* const lo_stash = comp == 0 ? A.f.rad_w : A.f.rad_s;
+    float* const hi_stash = comp == 0 ? A.f.rad_e : A.f.rad_n;
+    const unsigned level = unsigned(k) * plane, c = level + unsigned(N.q) * N.stride + unsigned(T.q) * T.stride;
+    const bool radiate = s >= 0, first = MOM && s == 0;
+    const bool gN = N.q == 1 || N.q == N.n - 2, gT = T.q == 1 || T.q == T.n - 2;
+    const bool perN = (N.q == 1 ? N.lo : N.hi) == NIMBUS_BC_PERIODIC, perT = (T.q == 1 ? T.lo : T.hi) == NIMBUS_BC_PERIODIC;
+    const bool low = comp < 2 ? N.normal_low() : N.low(), high = comp < 2 ? N.normal_high() : N.high();
+
+    // the faces at 0 and n - 2 of the cell's own line, stored (f) and radiative
+    auto face = [&](int q, int t) { return ld<S>(f, level + unsigned(q) * N.stride + unsigned(t) * T.stride); };
+    const std::size_t own_line = std::size_t(T.q) * NZ + k;
+    const unsigned cn = c + (MOM && comp == 2 ? (k < NZ - 1 ? plane : 0u) : N.stride);
+    S own = ld<S>(f, c), rc = ld<S>(rp, c), pc = ld<S>(pp, c), rn = S(0), pn = S(0), f0 = S(0), fa = S(0);
+    float s0 = 0.0f, sa = 0.0f;
+    if (MOM) { rn = ld<S>(rp, cn); pn = ld<S>(pp, cn); }
+    if (comp < 2)
+    {
+        if (low) { f0 = face(0, T.q); s0 = G(lo_stash)[own_line]; }
+        if (low || high) fa = face(N.n - 2, T.q);
+        if (high) sa = G(hi_stash)[own_line];
+    }
+    pin(own); pin(rc); pin(pc); pin(rn); pin(pn); pin(f0); pin(fa); pin(s0); pin(sa);
+
+    // density and pressure of the ghosts next to the cell: the component's own
+    // axis here, which its update has read above, the corner with w
+    if (comp < 2 ? gN : gN && gT)
+    {
+        const unsigned ghost = comp < 2 ? c : level + unsigned(T.q == 1 ? 0 : T.n - 1) * T.stride + unsigned(N.q) * N.stride;
+        const unsigned to = N.q == 1 ? ghost - N.stride : ghost + N.stride;
+        S r = rc, pr = pc;
+        if (perN || (comp == 2 && perT))
         {
-            if (radiate)
+            const int sn = perN ? N.n - 1 - N.q : N.q, st = comp == 2 && perT ? T.n - 1 - T.q : T.q;
+            const unsigned from = level + unsigned(sn) * N.stride + unsigned(st) * T.stride;
+            r = ld<S>(rp, from);
+            pr = ld<S>(pp, from);
+        }
+        st<S>(rp, to, r);
+        st<S>(pp, to, pr);
+    }
+    if (k == NZ - 1) return;  // the lid's winds are closed from the level below
+    if (MOM && !(comp == 2 && p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI))
+    {
+        const auto rho0 = slot(A.f.base, kBaseRho0, NZ);
+        const double r = rho0[k] + double(rc), rq = rho0[comp == 2 ? k + 1 : k] + double(rn);
+        const double d = pressure_gradient<S>(pc, pn, 0.5 * (r + rq), comp == 0 ? g.idx : comp == 1 ? g.idy : g.idz);
+        const double lim = comp == 2 ? p.bounds.wind_v : p.bounds.wind_h;
+        own = S(clamp_store<S>(double(own) + d * p.dts, 0.0, -lim, lim));
+    }
+
+    const float dt = float(p.dts), inv_d = 1.0f / float(comp == 0 ? g.dx : g.dy), cstar = 30.0f;
+#pragma unroll 1
+    for (int e = 0; e < 3; ++e)
+    {
+        // line t of the tangential axis: the cell's own, the low and the high ghost's
+        if ((e == 1 && !T.low()) || (e == 2 && !T.high())) continue;
+        const int t = e == 0 ? T.q : e == 1 ? 0 : T.n - 1;
+        const bool rigid = e != 0 && (e == 1 ? T.lo : T.hi) == NIMBUS_BC_RIGID;
+        auto put = [&](int q, S val) {
+            const unsigned o = level + unsigned(q) * N.stride + unsigned(t) * T.stride;
+            if (comp == 0 && rigid) val = S(0);
+            st<S>(f, o, comp < 2 && k == 0 && p.bc_bottom == NIMBUS_BOTTOM_NO_SLIP ? S(0) : val);
+            if (k == NZ - 2) st<S>(f, o + plane, comp < 2 || p.bc_top == NIMBUS_TOP_OPEN ? val : S(0));
+        };
+        // u: west/east is closed first and its rows spread then; v and w come through the columns
+        const bool zero = comp > 0 && rigid;
+        const S in = zero ? S(0) : own;
+        S vl = in, vh = in;
+        if (comp < 2)
+        {
+            const std::size_t line = std::size_t(comp == 0 ? T.q : t) * NZ + k;
+            const bool other = comp == 1 && e != 0;  // a line with radiative faces of its own
+            if (N.lo == NIMBUS_BC_PERIODIC) { if (N.open()) vl = zero ? S(0) : fa; }
+            else if (N.lo == NIMBUS_BC_RADIATIVE)
             {
-                const float nn = kw78_face(s_lo, s_lo - 0.0f - cstar, float(n_in) - s_lo, dt_rad, inv_d, true);
-                n[c] = S(nn);
-                *stash_lo = nn;
+                vl = zero ? S(0) : f0;
+                if (radiate && low)
+                {
+                    const float prev = first ? float(other ? face(0, t) : f0) : other ? G(lo_stash)[line] : s0;
+                    const float nn = kw78_face(prev, prev - 0.0f - cstar, float(in) - prev, dt, inv_d, true);
+                    G(lo_stash)[line] = nn;
+                    vl = S(nn);
+                }
             }
+            else if (N.lo != NIMBUS_BC_ZERO_GRADIENT) vl = S(0);
+            if (N.hi == NIMBUS_BC_RADIATIVE)
+            {
+                vh = zero ? S(0) : fa;
+                if (radiate && high)
+                {
+                    const float prev = first ? float(other ? face(N.n - 2, t) : fa) : other ? G(hi_stash)[line] : sa;
+                    const float nn = kw78_face(prev, prev - 0.0f + cstar, prev - float(in), dt, inv_d, false);
+                    G(hi_stash)[line] = nn;
+                    vh = S(nn);
+                }
+            }
+            else if (N.wall()) vh = S(0);
         }
-        else n[c] = bc_lo == NIMBUS_BC_ZERO_GRADIENT ? n_in : S(0);
-        const bool rigid = bc_lo == NIMBUS_BC_RIGID;
-        t1[c] = rigid ? S(0) : t1_in;
-        t2[c] = rigid ? S(0) : t2_in;
-        rp[c] = rp_in;
-        pp[c] = pp_in;
-    }
-    // high face
-    if (bc_hi == NIMBUS_BC_PERIODIC)
-    {
-        n[gi] = n_in; t1[gi] = t1_in; t2[gi] = t2_in; rp[gi] = rp_in; pp[gi] = pp_in;
-    }
-    else
-    {
-        S na = n_a;
-        if (bc_hi == NIMBUS_BC_RIGID || bc_hi == NIMBUS_BC_RIGID_SLIP) na = S(0);
-        if (bc_hi == NIMBUS_BC_RADIATIVE && radiate)
+        else
         {
-            const float nn = kw78_face(s_hi, s_hi - 0.0f + cstar, s_hi - float(n_am), dt_rad, inv_d, false);
-            na = S(nn);
-            *stash_hi = nn;
+            if (N.lo == NIMBUS_BC_RIGID) vl = S(0);
+            if (N.hi == NIMBUS_BC_RIGID) vh = S(0);
         }
-        else if (bc_hi == NIMBUS_BC_ZERO_GRADIENT) na = n_am;
-        if (bc_hi == NIMBUS_BC_RIGID || bc_hi == NIMBUS_BC_RIGID_SLIP || (bc_hi == NIMBUS_BC_RADIATIVE && radiate) ||
-            bc_hi == NIMBUS_BC_ZERO_GRADIENT)
-            n[a] = na;
-        n[gi] = (bc_hi == NIMBUS_BC_RADIATIVE || bc_hi == NIMBUS_BC_ZERO_GRADIENT) ? na : S(0);
-        const bool rigid = bc_hi == NIMBUS_BC_RIGID;
-        t1[gi] = rigid ? S(0) : t1_a;
-        t2[gi] = rigid ? S(0) : t2_a;
-        rp[gi] = rp_a;
-        pp[gi] = pp_a;
+        if (comp == 2 || N.normal_self()) put(N.q, comp < 2 && N.wall() && N.q == N.n - 2 ? S(0) : in);
+        if (low) put(0, vl);
+        if (high)
+        {
+            put(N.n - 1, vh);
+            if (comp < 2 && N.open()) put(N.n - 2, vh);
+        }
     }
 }
 
+// Backward momentum update of substep s with the new rho' (buffer
+// (s + 1) & 1) and pressure, in place, and (close) the boundary closure of the
+// new state: edge workgroups, then the others. HE-VI members keep the
+// interior w the column solve set. Members that are not closed here (bc_split,
+// or a single substep) update the ghost cells as every other, which clamps them.
+//
+// Bound by HBM (24 B per cell of a HE-VI member with FP32 storage). Edge cells
+// in the lanes of the row runs doubled the life of a fourth of all waves (148
+// us per substep at 400 x 400 x 100 mixed), in workgroups of their own they
+// run beside the others. us per substep, the update and three closure
+// kernels -> this one: 400 x 400 x 100 mixed 106 + 34 -> 123, 160 x 160 x 80
+// 16 + 24 -> 22, 48 x 48 x 40 6 + 21 -> 8, 64 x 64 x 40 FP64 7 + 22 -> 9.
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_bc_west_east(const MemberArgs* __restrict__ ma,
-                                                         const int2* __restrict__ map, int s)
+__global__ __launch_bounds__(kBlock) void k_momentum(const MemberArgs* __restrict__ ma,
+                                                     const int2* __restrict__ map, int s, int close)
 {
     const Work wk = work_of(map);
     const MemberArgs& A = ma[wk.m];
-    BcBufs<S> b;
-    if (!bc_buffers<S>(A, s, b)) return;
+    if (s >= A.p.substeps) return;
+    const bool closes = close != 0 && !bc_split(A.p);
+    const DevFields& f = A.f;
+    const auto rn = P<S>((s & 1) ? f.rp : f.rp2);
+    if (wk.local < A.geo.edge_blocks)
+    {
+        if (closes) close_edges<S, true>(A, wk.local, s, rn);
+        return;
+    }
+    const Cell cl = cell_of(A, wk.local - A.geo.edge_blocks);
+    if (!cl.valid) return;
     const DevGrid& g = A.g;
-    const int t = wk.local * kBlock + int(threadIdx.x);
-    if (t >= g.ny * g.nz) return;
-    const int k = t / g.ny, j = t - k * g.ny;
-    const int NX = g.nx, NZ = g.nz;
-    const std::size_t row = g.at(0, j, k);
-    const std::size_t st = std::size_t(j) * NZ + k;
-    lateral_pair<S>(b.u, b.v, b.w, b.rp, b.pp, G(A.f.rad_w) + st, G(A.f.rad_e) + st, A.p.bc_west, A.p.bc_east,
-                    b.dt_rad > 0.0f, b.dt_rad, 1.0f / float(g.dx), row, row + 1, row + (NX - 3), row + (NX - 2),
-                    row + (NX - 1));
+    const int NX = g.nx, NY = g.ny, NZ = g.nz;
+    const int i = cl.i, j = cl.j, k = cl.k;
+    // the edge workgroups close the ghosts, the level below the lid closes the lid
+    if (closes && (i < 2 || i >= NX - 3 || j < 2 || j >= NY - 3 || k == NZ - 1)) return;
+    const auto pp = P<S>(f.pp), u = P<S>(f.u), v = P<S>(f.v), w = P<S>(f.w);
+    const bool lateral = i >= 1 && i < NX - 1 && j >= 1 && j < NY - 1;
+    const bool interior = lateral && k < NZ - 1, hevi = A.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI;
+    const std::size_t sy = std::size_t(g.px), sz = g.plane();
+    const std::size_t c = g.at(i, j, k);
+    // neighbours clamped to the domain (the cell itself stands in for a missing one)
+    const std::size_t cxp = i < NX - 1 ? c + 1 : c, cyp = j < NY - 1 ? c + sy : c, czp = k < NZ - 1 ? c + sz : c;
+    RhoP<S> cc{rn[c], pp[c]}, xp{rn[cxp], pp[cxp]}, yp{rn[cyp], pp[cyp]}, zp{S(0), S(0)};
+    S uc = u[c], vc = v[c], wc = S(0);
+    if (!hevi) zp = RhoP<S>{rn[czp], pp[czp]};
+    if (!(hevi && closes)) wc = w[c];
+    const auto rho0 = slot(f.base, kBaseRho0, NZ);
+    double r0 = rho0[k], r0p = rho0[k < NZ - 1 ? k + 1 : k];
+    pin(cc.r); pin(cc.p); pin(xp.r); pin(xp.p); pin(yp.r); pin(yp.p); pin(zp.r); pin(zp.p);
+    pin(uc); pin(vc); pin(wc); pin(r0); pin(r0p);
+    const Bounds& bd = A.p.bounds;
+    const double dts = A.p.dts;
+    double du = 0.0, dv = 0.0, dw = 0.0;
+    if (interior)
+    {
+        const double rc = r0 + double(cc.r);
+        du = pressure_gradient<S>(cc.p, xp.p, 0.5 * (rc + (r0 + double(xp.r))), g.idx);
+        dv = pressure_gradient<S>(cc.p, yp.p, 0.5 * (rc + (r0 + double(yp.r))), g.idy);
+        if (!hevi) dw = pressure_gradient<S>(cc.p, zp.p, 0.5 * (rc + (r0p + double(zp.r))), g.idz);
+    }
+    const S un = S(clamp_store<S>(double(uc) + du * dts, 0.0, -bd.wind_h, bd.wind_h));
+    const S vn = S(clamp_store<S>(double(vc) + dv * dts, 0.0, -bd.wind_h, bd.wind_h));
+    const S wn = hevi && interior ? wc : S(clamp_store<S>(double(wc) + dw * dts, 0.0, -bd.wind_v, bd.wind_v));
+    const bool ground = closes && k == 0 && A.p.bc_bottom == NIMBUS_BOTTOM_NO_SLIP;
+    u[c] = ground ? S(0) : un;
+    v[c] = ground ? S(0) : vn;
+    if (!(hevi && interior)) w[c] = wn;
+    if (closes && k == NZ - 2)
+    {
+        u[c + sz] = un;
+        v[c + sz] = vn;
+        w[c + sz] = A.p.bc_top == NIMBUS_TOP_OPEN ? wn : S(0);  // (HE-VI members have a rigid lid)
+    }
+    if (!closes && s == 0 && bc_split(A.p))
+    {
+        // the radiative faces start from the winds before the first update
+        if (i == 0) G(f.rad_w)[std::size_t(j) * NZ + k] = float(uc);
+        if (i == NX - 2) G(f.rad_e)[std::size_t(j) * NZ + k] = float(uc);
+        if (j == 0) G(f.rad_s)[std::size_t(i) * NZ + k] = float(vc);
+        if (j == NY - 2) G(f.rad_n)[std::size_t(i) * NZ + k] = float(vc);
+    }
 }
 
+// The closure alone: of the home buffers, without radiation (s < 0), and of
+// substep s of the members whose momentum update cannot close it (bc_split).
+// Edge workgroups, then the other columns of the lid and the ground.
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_bc_south_north(const MemberArgs* __restrict__ ma,
-                                                           const int2* __restrict__ map, int s)
+__global__ __launch_bounds__(kBlock) void k_close(const MemberArgs* __restrict__ ma, const int2* __restrict__ map,
+                                                  int s)
 {
     const Work wk = work_of(map);
     const MemberArgs& A = ma[wk.m];
-    BcBufs<S> b;
-    if (!bc_buffers<S>(A, s, b)) return;
+    if (s >= 0 && (s >= A.p.substeps || !bc_split(A.p))) return;
     const DevGrid& g = A.g;
-    const int t = wk.local * kBlock + int(threadIdx.x);
-    if (t >= g.nx * g.nz) return;
-    const int k = t / g.nx, i = t - k * g.nx;
-    const int NY = g.ny, NZ = g.nz;
-    const std::size_t sy = std::size_t(g.px);
-    const std::size_t c = g.at(i, 0, k);
-    const std::size_t st = std::size_t(i) * NZ + k;
-    lateral_pair<S>(b.v, b.u, b.w, b.rp, b.pp, G(A.f.rad_s) + st, G(A.f.rad_n) + st, A.p.bc_south, A.p.bc_north,
-                    b.dt_rad > 0.0f, b.dt_rad, 1.0f / float(g.dy), c, c + sy, c + (NY - 3) * sy, c + (NY - 2) * sy,
-                    c + (NY - 1) * sy);
-}
-
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_bc_vertical(const MemberArgs* __restrict__ ma,
-                                                        const int2* __restrict__ map, int s)
-{
-    const Work wk = work_of(map);
-    const MemberArgs& A = ma[wk.m];
-    BcBufs<S> b;
-    if (!bc_buffers<S>(A, s, b)) return;
-    const DevGrid& g = A.g;
-    const Column t = column_of(A, wk.local);
-    if (t.i >= g.nx || t.j >= g.ny) return;
-    const int NZ = g.nz;
-    const std::size_t top = g.at(t.i, t.j, NZ - 1), tm = g.at(t.i, t.j, NZ - 2);
-    const S wt = b.w[tm], ut = b.u[tm], vt = b.v[tm];  // loads before the stores
+    if (wk.local < A.geo.edge_blocks)
+    {
+        close_edges<S, false>(A, wk.local, s, P<S>(s >= 0 && !(s & 1) ? A.f.rp2 : A.f.rp));
+        return;
+    }
+    const int t = (wk.local - A.geo.edge_blocks) * kBlock + int(threadIdx.x), wx = g.nx - 5;
+    if (t >= wx * (g.ny - 5)) return;
+    const int jj = t / wx;
+    const std::size_t ground = g.at(2 + t - jj * wx, 2 + jj, 0), top = ground + g.plane() * (g.nz - 1);
+    const std::size_t tm = top - g.plane();
+    const auto u = P<S>(A.f.u), v = P<S>(A.f.v), w = P<S>(A.f.w);
+    const S ut = u[tm], vt = v[tm], wt = w[tm];
     if (A.p.bc_bottom == NIMBUS_BOTTOM_NO_SLIP)
     {
-        b.u[g.at(t.i, t.j, 0)] = S(0);
-        b.v[g.at(t.i, t.j, 0)] = S(0);
+        u[ground] = S(0);
+        v[ground] = S(0);
     }
-    b.w[top] = A.p.bc_top == NIMBUS_TOP_OPEN ? wt : S(0);
-    b.u[top] = ut;
-    b.v[top] = vt;
-}
-
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_seed_radiation(const MemberArgs* __restrict__ ma,
-                                                           const int2* __restrict__ map)
-{
-    const Work wk = work_of(map);
-    const MemberArgs& A = ma[wk.m];
-    const DevGrid& g = A.g;
-    const int t = wk.local * kBlock + int(threadIdx.x);
-    const int NZ = g.nz;
-    const auto u = P<S>(A.f.u);
-    const auto v = P<S>(A.f.v);
-    if (t < g.ny * NZ)
-    {
-        const int j = t / NZ, k = t - j * NZ;
-        G(A.f.rad_w)[t] = float(u[g.at(0, j, k)]);
-        G(A.f.rad_e)[t] = float(u[g.at(g.nx - 2, j, k)]);
-    }
-    if (t < g.nx * NZ)
-    {
-        const int i = t / NZ, k = t - i * NZ;
-        G(A.f.rad_s)[t] = float(v[g.at(i, 0, k)]);
-        G(A.f.rad_n)[t] = float(v[g.at(i, g.ny - 2, k)]);
-    }
+    u[top] = ut;
+    v[top] = vt;
+    w[top] = A.p.bc_top == NIMBUS_TOP_OPEN ? wt : S(0);
 }
 
 // Moves rho' from buffer 1 to buffer 0 when the member's substep count
@@ -2899,22 +2947,20 @@ void fill_geometry(MemberArgs& a, int tile_w, int k_chunks, int xcd_remap)
     G.k_chunks = std::max(1, std::min(k_chunks, a.g.nz));
     G.xcd_remap = xcd_remap ? 1 : 0;
     G.solve_lanes = solve_lanes(a.g.nz);
+    G.edge_blocks = 3 * ((edge_cells(a.g.nx, a.g.ny) * a.g.nz + kBlock - 1) / kBlock);
 }
 
 int work_items(const MemberArgs& a, WorkKind kind)
 {
     const MemberGeom& G = a.geo;
     const int tiles = G.tiles_x * G.tiles_y;
-    const auto lin = [](std::size_t n) { return int((n + kBlock - 1) / kBlock); };
     switch (kind)
     {
     case W_CELL:
         return G.linear ? G.runs * a.g.nz : tiles * G.k_chunks * ((a.g.nz + G.k_chunks - 1) / G.k_chunks);
-    case W_COLUMN: return G.linear ? int((std::size_t(a.g.nx) * a.g.ny + kBlock - 1) / kBlock) : tiles;
-    case W_WE: return lin(std::size_t(a.g.ny) * a.g.nz);
-    case W_SN: return lin(std::size_t(a.g.nx) * a.g.nz);
-    case W_SEED: return lin(std::size_t(std::max(a.g.nx, a.g.ny)) * a.g.nz);
     case W_DIAG: return kDiagBlocksPerMember;
+    case W_MOMENTUM: return G.edge_blocks + work_items(a, W_CELL);
+    case W_SHELL: return G.edge_blocks + ((a.g.nx - 5) * (a.g.ny - 5) + kBlock - 1) / kBlock;
     case W_SOLVE: return int(a.g.plane() / std::size_t(G.solve_lanes * G.vec));
     case W_TILECELL: return tiles * G.k_chunks * ((a.g.nz + G.k_chunks - 1) / G.k_chunks);
     default: return 0;
@@ -3011,7 +3057,7 @@ void launch_slow_tendencies(Launcher& L, const BatchView& b, void* du, void* dv,
 }
 
 template <class S>
-void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumulate, bool init_at_first)
+void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumulate, bool init_at_first, bool close)
 {
     launch_map(L, "acoustic_forward", k_acoustic_forward<S>, b, S_EXPLICIT, W_CELL, s, int(accumulate),
                int(init_at_first));
@@ -3019,21 +3065,14 @@ void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumu
     if (b.hevi_nz[0] > 0) launch_hevi_solve<S, 4>(L, b, s, first, b.hevi_nz[0]);
     if (b.hevi_nz[1] > 0) launch_hevi_solve<S, 2>(L, b, s, first, b.hevi_nz[1]);
     if (b.hevi_nz[2] > 0) launch_hevi_solve<S, 1>(L, b, s, first, b.hevi_nz[2]);
-    launch_map(L, "acoustic_momentum", k_momentum<S>, b, S_ALL, W_CELL, s);
+    launch_map(L, "acoustic_momentum", k_momentum<S>, b, S_ALL, W_MOMENTUM, s, int(close));
+    if (close && b.any_bc_split) launch_map(L, "boundary_closure", k_close<S>, b, S_ALL, W_SHELL, s);
 }
 
 template <class S>
-void launch_boundaries(Launcher& L, const BatchView& b, int s)
+void launch_boundaries(Launcher& L, const BatchView& b)
 {
-    launch_map(L, "bc_west_east", k_bc_west_east<S>, b, S_ALL, W_WE, s);
-    launch_map(L, "bc_south_north", k_bc_south_north<S>, b, S_ALL, W_SN, s);
-    launch_map(L, "bc_vertical", k_bc_vertical<S>, b, S_ALL, W_COLUMN, s);
-}
-
-template <class S>
-void launch_seed_radiation(Launcher& L, const BatchView& b)
-{
-    launch_map(L, "seed_radiation", k_seed_radiation<S>, b, S_ALL, W_SEED);
+    launch_map(L, "boundary_closure", k_close<S>, b, S_ALL, W_SHELL, -1);
 }
 
 template <class S>
@@ -3066,13 +3105,8 @@ template <class S>
 void launch_large_step(Launcher& L, const BatchView& b)
 {
     launch_slow_rk2<S>(L, b);
-    launch_boundaries<S>(L, b, -1);
-    launch_seed_radiation<S>(L, b);
-    for (int s = 0; s < b.max_substeps; ++s)
-    {
-        launch_acoustic_substep<S>(L, b, s, true, true);
-        launch_boundaries<S>(L, b, s);
-    }
+    launch_boundaries<S>(L, b);
+    for (int s = 0; s < b.max_substeps; ++s) launch_acoustic_substep<S>(L, b, s, true, true, true);
     launch_commit<S>(L, b, -1);
     const int pd[4] = {0, 1, 1, 1};
     launch_transport<S>(L, b, 4, pd, true);
@@ -3103,7 +3137,7 @@ void launch_large_step(Launcher& L, const BatchView& b)
         launch_map(L, "diffusion_commit", k_diffusion_commit<S>, b, S_ALL, W_CELL);
     }
     if (b.any_sponge_unfused) launch_map(L, "sponge", k_sponge<S>, b, S_ALL, W_CELL);
-    launch_boundaries<S>(L, b, -1);
+    launch_boundaries<S>(L, b);
 }
 
 template <class S>
@@ -3140,9 +3174,8 @@ void launch_dev_to_host(Launcher& L, const DevGrid& g, const void* src, void* ds
     template void launch_large_step<S>(Launcher&, const BatchView&);                                            \
     template void launch_slow_rk2<S>(Launcher&, const BatchView&);                                              \
     template void launch_slow_tendencies<S>(Launcher&, const BatchView&, void*, void*, void*);                  \
-    template void launch_acoustic_substep<S>(Launcher&, const BatchView&, int, bool, bool);                     \
-    template void launch_boundaries<S>(Launcher&, const BatchView&, int);                                       \
-    template void launch_seed_radiation<S>(Launcher&, const BatchView&);                                        \
+    template void launch_acoustic_substep<S>(Launcher&, const BatchView&, int, bool, bool, bool);                     \
+    template void launch_boundaries<S>(Launcher&, const BatchView&);                                            \
     template void launch_commit<S>(Launcher&, const BatchView&, int);                                           \
     template void launch_transport<S>(Launcher&, const BatchView&, int, const int*, bool);                      \
     template void launch_kessler_tendencies<S>(Launcher&, const BatchView&, double, void*, void*, void*, void*); \

@@ -101,13 +101,24 @@ struct MemberGeom
     int k_chunks;
     int xcd_remap;
     // per-cell work in runs of kBlock consecutive elements of one level's
-    // padded [j][i] plane (`runs` per level) instead of column tiles at one
-    // level, per-column work in runs of kBlock consecutive columns
+    // padded [j][i] plane (`runs` per level) instead of column tiles at one level
     int linear, runs;
     // HE-VI solve: 16-byte lanes per level of a workgroup (solve_lanes(nz)) and
     // elements per 16 bytes (fixed by the storage type at creation)
     int solve_lanes, vec;
+    // workgroups of the edge cells (close_edges), which the boundary closure spreads
+    int edge_blocks;
 };
+
+// A low side that copies an open high side's face periodically needs that
+// face before and after its closure, so the momentum update cannot close it.
+__host__ __device__ inline bool bc_split(const StepParams& p)
+{
+    auto split = [](int lo, int hi) {
+        return lo == NIMBUS_BC_PERIODIC && (hi == NIMBUS_BC_RADIATIVE || hi == NIMBUS_BC_ZERO_GRADIENT);
+    };
+    return split(p.bc_west, p.bc_east) || split(p.bc_south, p.bc_north);
+}
 
 struct MemberArgs
 {
@@ -121,14 +132,12 @@ struct MemberArgs
 enum WorkKind
 {
     W_CELL = 0,    // one tile of columns at one level, or one run of a level (one cell per thread)
-    W_COLUMN = 1,  // one tile, whole columns (one column per thread)
-    W_WE = 2,      // 256 (j, k) rows of the west/east faces
-    W_SN = 3,      // 256 (i, k) rows of the south/north faces
-    W_SEED = 4,    // 256 entries of the radiative stashes
-    W_DIAG = 5,    // one of kDiagBlocksPerMember reduction blocks
-    W_SOLVE = 6,   // solve_lanes x 16 bytes consecutive columns of one row, whole columns (HE-VI solve)
-    W_TILECELL = 7,  // one tile of columns at one level whatever the geometry (wide stencils)
-    W_KINDS = 8
+    W_DIAG = 1,    // one of kDiagBlocksPerMember reduction blocks
+    W_SOLVE = 2,   // solve_lanes x 16 bytes consecutive columns of one row, whole columns (HE-VI solve)
+    W_TILECELL = 3,  // one tile of columns at one level whatever the geometry (wide stencils)
+    W_MOMENTUM = 4,  // a wind component of 256 edge cells (edge_blocks of them), then as W_CELL
+    W_SHELL = 5,     // a wind component of 256 edge cells (edge_blocks of them), then 256 other columns
+    W_KINDS = 6
 };
 
 // Column-solve form of a member (nimbus_hip_member_set_column_solve), fixed at
@@ -179,6 +188,7 @@ struct BatchView
     int any_sponge_unfused = 0;  // a member with sponges and no SGS or diffusion pass to apply them in
     int any_diffusion = 0;       // a member with explicit diffusion
     int any_kessler_adaptive = 0; // a member whose microphysics subcycles follow its sedimentation limit
+    int any_bc_split = 0;        // a member whose substeps are closed by k_close
     int max_nz = 0;
     int hevi_nz[3] = {0, 0, 0};  // deepest of the HE-VI members with 4, 2 and 1 lanes per level
     int elem = 4;
@@ -198,15 +208,14 @@ template <class S>
 void launch_slow_rk2(Launcher& L, const BatchView& b);
 template <class S>
 void launch_slow_tendencies(Launcher& L, const BatchView& b, void* du, void* dv, void* dw);
-// Substep s of the acoustic loop (0-based): reads buffer s & 1, writes (s + 1) & 1.
+// Substep s of the acoustic loop (0-based): reads buffer s & 1, writes (s + 1) & 1;
+// close: with its boundary closure, which radiates with the member's dts (the
+// radiative faces start from the winds stored at substep 0).
 template <class S>
-void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumulate, bool init_at_first);
-// Boundary closure; s >= 0 selects the buffers after substep s and radiates
-// with the member's dts; s < 0 closes the home buffers without radiation.
+void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumulate, bool init_at_first, bool close);
+// Boundary closure of the home buffers, without radiation.
 template <class S>
-void launch_boundaries(Launcher& L, const BatchView& b, int s);
-template <class S>
-void launch_seed_radiation(Launcher& L, const BatchView& b);
+void launch_boundaries(Launcher& L, const BatchView& b);
 // Moves rho' from buffer 1 to buffer 0 for members whose last substep (n_done - 1) left it there.
 template <class S>
 void launch_commit(Launcher& L, const BatchView& b, int n_done);

@@ -557,6 +557,7 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
         b.view.any_sponge_unfused |= m->args.p.sponge && m->args.p.sgs_n == 0 && m->args.p.dif_apply == 0;
         b.view.any_diffusion |= m->args.p.dif_apply != 0;
         b.view.any_kessler_adaptive |= m->args.p.kessler_adaptive;
+        b.view.any_bc_split |= bc_split(m->args.p);
         if (m->args.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI)
         {
             int& nz = b.view.hevi_nz[m->args.geo.solve_lanes == 4 ? 0 : m->args.geo.solve_lanes == 2 ? 1 : 2];
@@ -577,7 +578,15 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
                 if (s == S_EXPLICIT && mode != NIMBUS_ACOUSTIC_EXPLICIT) continue;
                 if (s == S_HEVI && mode != NIMBUS_ACOUSTIC_HEVI) continue;
                 const int n = work_items(ms[q]->args, WorkKind(k));
-                for (int l = 0; l < n; ++l) logical.push_back(int2{int(q), l});
+                // edge workgroups evenly among the others: the XCDs share them, and
+                // each runs beside the levels it belongs to
+                const long e = k == W_MOMENTUM || k == W_SHELL ? ms[q]->args.geo.edge_blocks : 0;
+                for (long l = 0, edges = 0; l < n; ++l)
+                {
+                    const bool edge = edges < (l + 1) * e / n;
+                    logical.push_back(int2{int(q), int(edge ? edges : e + l - edges)});
+                    edges += edge;
+                }
             }
             const int n = int(logical.size());
             offsets[s][k] = all.size();
@@ -1533,7 +1542,7 @@ int nimbus_hip_dispatch_acoustic_substep_fused(nimbus_hip_ctx* ctx, const nimbus
     rc = upload_state<float>(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
     Launcher L = make_launcher(ctx);
-    launch_acoustic_substep<float>(L, sm.batch.view, 0, false, false);
+    launch_acoustic_substep<float>(L, sm.batch.view, 0, false, false, false);
     launch_commit<float>(L, sm.batch.view, 1);
     if (L.error != hipSuccess) return hip_fail(L.error, "acoustic launch");
     nimbus_host_state out{d->u, d->v, d->w, d->rho, d->p, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -1596,12 +1605,8 @@ int nimbus_hip_dispatch_acoustic_substeps_batched(nimbus_hip_ctx* ctx,
         }
     }
     Launcher L = make_launcher(ctx);
-    launch_seed_radiation<float>(L, sm.batch.view);
     for (int s = 0; s < d->n_substeps; ++s)
-    {
-        launch_acoustic_substep<float>(L, sm.batch.view, s, d->accumulate_mass_flux != 0, false);
-        launch_boundaries<float>(L, sm.batch.view, s);
-    }
+        launch_acoustic_substep<float>(L, sm.batch.view, s, d->accumulate_mass_flux != 0, false, true);
     launch_commit<float>(L, sm.batch.view, d->n_substeps);
     if (L.error != hipSuccess) return hip_fail(L.error, "batched acoustic launch");
     nimbus_host_state out{d->u, d->v, d->w, d->rho, d->p, nullptr, nullptr, nullptr, nullptr, nullptr};

@@ -332,6 +332,30 @@ def test_mixed_lateral_pairings_fp64_match_fp64_oracle(hip_ctx, lateral):
         check_fp64(out, ref, f"lateral {lateral} mode {mode}", rad, diffusive=rad)
 
 
+BC_SIDES = [L.BC_PERIODIC, L.BC_RADIATIVE, L.BC_ZERO_GRADIENT, L.BC_RIGID, L.BC_RIGID_SLIP]
+
+
+@pytest.mark.parametrize("mode", [L.ACOUSTIC_EXPLICIT, L.ACOUSTIC_HEVI])
+@pytest.mark.parametrize("shape", [(5, 5, 4), (70, 6, 5)])
+@pytest.mark.parametrize("bottom, top", [(L.BOTTOM_NO_SLIP, L.TOP_OPEN), (L.BOTTOM_FREE_SLIP, L.TOP_RIGID)])
+def test_every_pair_of_sides_fp64_matches_fp64_oracle(hip_ctx, mode, shape, bottom, top):
+    """The closure in the momentum update's stores: every pair of conditions on
+    opposite sides (also a periodic low side with an open high one, which is
+    closed by its own kernel), the ground and lid conditions, on the smallest
+    grid (every cell between the ghosts is an edge) and on rows that span more
+    than one workgroup."""
+    nx, ny, nz = shape
+    g, base, st = small_case(nx=nx, ny=ny, nz=nz, dz=2000.0, cloudy=True, wind_noise=0.5, dtype=np.float64)
+    for lo in BC_SIDES:
+        for hi in BC_SIDES:
+            lateral = (lo, hi, hi, BC_SIDES[(BC_SIDES.index(lo) + 1) % 5])
+            cfg = L.step_config(3.0, 3, acoustic_mode=mode, lateral=lateral, bottom=bottom,
+                                top=top if mode == L.ACOUSTIC_EXPLICIT else L.TOP_RIGID)
+            ref, _ = O.large_steps(oracle_grid(g), base, O.from_step_config(cfg), st, 2, np.float64)
+            out, _ = _run_member(hip_ctx, g, base, cfg, st, L.PRECISION_FP64, 2)
+            check_fp64(out, ref, f"sides {lateral} mode {mode} {shape}", L.BC_RADIATIVE in lateral, diffusive=True)
+
+
 MIXED_TOL_SCALE = {"u": 30.0, "v": 30.0, "w": 30.0, "rho": 1.0, "p": 1e5, "theta": 300.0, "qv": 0.014,
                    "qc": 0.014, "qr": 0.014}
 
