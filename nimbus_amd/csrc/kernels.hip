@@ -2911,23 +2911,62 @@ __global__ void k_diag_final(const MemberArgs* __restrict__ ma, int n_members)
 }
 
 // Host layout [i][j][k] <-> device [k][j][i], subtracting / adding a base slot.
-// Grid: (ceil(nx / 64), ny, nz) workgroups of 64 threads.
-template <class H, class S>
-__global__ __launch_bounds__(64) void k_host_to_dev(DevGrid g, const H* src, S* dst, const double* base_slot)
-{
-    const int i = int(blockIdx.x) * 64 + int(threadIdx.x), j = int(blockIdx.y), k = int(blockIdx.z);
-    if (i >= g.nx) return;
-    const std::size_t h = (std::size_t(i) * g.ny + j) * g.nz + k;
-    dst[g.at(i, j, k)] = S(double(src[h]) - (base_slot ? base_slot[k] : 0.0));
-}
+// A chunk of a host array: the elements [r0, r0 + nr) of the (j, k) planes
+// (r = j nz + k, contiguous on the host) of columns i0 .. i0 + ni - 1, one
+// after the other (nr is a whole plane where ni > 1).
+// The host array's fastest axis is the device's slowest, so a workgroup turns
+// a tile of kTurnI x kTurnR through LDS: rows of 64 B or more on the device
+// side, 256 B or more on the host side, which for the slots of HostTransfer is
+// the host link, the bound (49 GB/s written, 53 read).
+constexpr int kTurnI = 16, kTurnR = 128;
 
-template <class S, class H>
-__global__ __launch_bounds__(64) void k_dev_to_host(DevGrid g, const S* src, H* dst, const double* base_slot)
+template <class S, class H, bool TO_HOST>
+__global__ __launch_bounds__(kBlock) void k_turn(DevGrid g, S* dev, H* host, const double* __restrict__ base, int i0,
+                                                 int ni, int r0, int nr)
 {
-    const int i = int(blockIdx.x) * 64 + int(threadIdx.x), j = int(blockIdx.y), k = int(blockIdx.z);
-    if (i >= g.nx) return;
-    const std::size_t h = (std::size_t(i) * g.ny + j) * g.nz + k;
-    dst[h] = H(double(src[g.at(i, j, k)]) + (base_slot ? base_slot[k] : 0.0));
+    __shared__ H tile[kTurnI][kTurnR + 1];
+    constexpr int N = kTurnI * kTurnR / kBlock;
+    const int nz = g.nz, ti = int(blockIdx.y) * kTurnI, tr = int(blockIdx.x) * kTurnR;
+    const int tid = int(threadIdx.x);
+    // device side: column a of the tile and elements q + e; host side: element b and columns h + e
+    const int a = tid % kTurnI, q = tid / kTurnI * N, b = tid % kTurnR, h = tid / kTurnR * N;
+    std::size_t c[N];
+    double sub[N];
+    bool in_d[N], in_h[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+    {
+        in_d[e] = ti + a < ni && tr + q + e < nr;
+        in_h[e] = ti + h + e < ni && tr + b < nr;
+        const int r = min(r0 + tr + q + e, g.ny * nz - 1), j = r / nz, k = r - j * nz;
+        c[e] = g.at(min(i0 + ti + a, g.nx - 1), j, k);
+        sub[e] = base ? base[k] : 0.0;
+    }
+    if (TO_HOST)
+    {
+        S v[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = dev[c[e]];  // in bounds also outside the part
+#pragma unroll
+        for (int e = 0; e < N; ++e) tile[a][q + e] = H(double(v[e]) + sub[e]);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+            if (in_h[e]) host[std::size_t(ti + h + e) * nr + (tr + b)] = tile[h + e][b];
+    }
+    else
+    {
+        H v[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+            v[e] = host[std::size_t(min(ti + h + e, ni - 1)) * nr + min(tr + b, nr - 1)];
+#pragma unroll
+        for (int e = 0; e < N; ++e) tile[h + e][b] = v[e];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+            if (in_d[e]) dev[c[e]] = S(double(tile[a][q + e]) - sub[e]);
+    }
 }
 
 }  // namespace
@@ -3150,24 +3189,17 @@ void launch_diagnostics(Launcher& L, const BatchView& b)
     L.end("diag_final", ev);
 }
 
-template <class H, class S>
-void launch_host_to_dev(Launcher& L, const DevGrid& g, const void* src, void* dst, const double* base_slot)
-{
-    hipEvent_t ev;
-    L.begin("host_to_dev", ev);
-    hipLaunchKernelGGL((k_host_to_dev<H, S>), dim3(unsigned((g.nx + 63) / 64), unsigned(g.ny), unsigned(g.nz)),
-                       dim3(64), 0, L.stream, g, static_cast<const H*>(src), PS<S>(dst), base_slot);
-    L.end("host_to_dev", ev);
-}
-
 template <class S, class H>
-void launch_dev_to_host(Launcher& L, const DevGrid& g, const void* src, void* dst, const double* base_slot)
+void launch_turn(Launcher& L, const DevGrid& g, void* dev, void* host, const double* base_slot, bool to_host,
+                 const HostPart& part)
 {
+    const dim3 grid(unsigned((part.nr + kTurnR - 1) / kTurnR), unsigned((part.ni + kTurnI - 1) / kTurnI));
+    const auto kernel = to_host ? k_turn<S, H, true> : k_turn<S, H, false>;
     hipEvent_t ev;
-    L.begin("dev_to_host", ev);
-    hipLaunchKernelGGL((k_dev_to_host<S, H>), dim3(unsigned((g.nx + 63) / 64), unsigned(g.ny), unsigned(g.nz)),
-                       dim3(64), 0, L.stream, g, static_cast<const S*>(src), static_cast<H*>(dst), base_slot);
-    L.end("dev_to_host", ev);
+    L.begin("host_transfer", ev);
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, L.stream, g, PS<S>(dev), static_cast<H*>(host), base_slot, part.i0,
+                       part.ni, part.r0, part.nr);
+    L.end("host_transfer", ev);
 }
 
 #define NIMBUS_INSTANTIATE(S)                                                                                    \
@@ -3180,10 +3212,8 @@ void launch_dev_to_host(Launcher& L, const DevGrid& g, const void* src, void* ds
     template void launch_transport<S>(Launcher&, const BatchView&, int, const int*, bool);                      \
     template void launch_kessler_tendencies<S>(Launcher&, const BatchView&, double, void*, void*, void*, void*); \
     template void launch_diagnostics<S>(Launcher&, const BatchView&);                                           \
-    template void launch_host_to_dev<float, S>(Launcher&, const DevGrid&, const void*, void*, const double*);   \
-    template void launch_host_to_dev<double, S>(Launcher&, const DevGrid&, const void*, void*, const double*);  \
-    template void launch_dev_to_host<S, float>(Launcher&, const DevGrid&, const void*, void*, const double*);   \
-    template void launch_dev_to_host<S, double>(Launcher&, const DevGrid&, const void*, void*, const double*);
+    template void launch_turn<S, float>(Launcher&, const DevGrid&, void*, void*, const double*, bool, const HostPart&); \
+    template void launch_turn<S, double>(Launcher&, const DevGrid&, void*, void*, const double*, bool, const HostPart&);
 
 NIMBUS_INSTANTIATE(float)
 NIMBUS_INSTANTIATE(double)

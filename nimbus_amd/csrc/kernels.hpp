@@ -226,10 +226,17 @@ void launch_kessler_tendencies(Launcher& L, const BatchView& b, double dt, void*
                                void* dqr);
 template <class S>
 void launch_diagnostics(Launcher& L, const BatchView& b);
-template <class H, class S>
-void launch_host_to_dev(Launcher& L, const DevGrid& g, const void* src, void* dst, const double* base_slot);
+// Elements [r0, r0 + nr) of the (j, k) planes of columns i0 .. i0 + ni - 1 of a
+// host array [i][j][k], packed; nr is a whole plane where ni > 1.
+struct HostPart
+{
+    int i0, ni, r0, nr;
+};
+// Device field (elements S, base profile subtracted) from or to such a part of
+// a host array (elements H), at an address that the device can reach.
 template <class S, class H>
-void launch_dev_to_host(Launcher& L, const DevGrid& g, const void* src, void* dst, const double* base_slot);
+void launch_turn(Launcher& L, const DevGrid& g, void* dev, void* host, const double* base_slot, bool to_host,
+                 const HostPart& part);
 
 constexpr int kDiagValues = 8;
 constexpr int kDiagBlocksPerMember = 64;

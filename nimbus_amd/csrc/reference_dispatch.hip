@@ -33,44 +33,45 @@ constexpr int kThreads = 256;
         if (e_ != hipSuccess) return set_error(NIMBUS_EHIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// Device copies of the call's arrays, released when the call returns.
+// Device copies of the call's arrays, released when the call returns. take()
+// names them, upload() fills those that have a host array.
 struct DeviceArrays
 {
     std::vector<void*> ptrs;
+    std::vector<ArrayCopy> in;
     ~DeviceArrays()
     {
         for (void* p : ptrs) hipFree(p);
     }
-    // Device array of n floats, a copy of host (or zero when host is null).
+    // Device array of n floats, to be a copy of host (or zero when host is null).
     int take(const float* host, std::size_t n, hipStream_t s, float** out)
     {
         void* p = nullptr;
         const hipError_t e = hipMalloc(&p, std::max<std::size_t>(n, 1) * sizeof(float));
         if (e != hipSuccess) return set_error(NIMBUS_ENOMEM, std::string("dispatch staging: ") + hipGetErrorString(e));
         ptrs.push_back(p);
-        const hipError_t c = host ? hipMemcpyAsync(p, host, n * sizeof(float), hipMemcpyHostToDevice, s)
-                                  : hipMemsetAsync(p, 0, n * sizeof(float), s);
-        if (c != hipSuccess) return set_error(NIMBUS_EHIP, std::string("dispatch staging: ") + hipGetErrorString(c));
+        if (host) in.push_back(ArrayCopy{p, const_cast<float*>(host), n * sizeof(float)});
+        else
+        {
+            const hipError_t c = hipMemsetAsync(p, 0, n * sizeof(float), s);
+            if (c != hipSuccess) return set_error(NIMBUS_EHIP, std::string("dispatch staging: ") + hipGetErrorString(c));
+        }
         *out = static_cast<float*>(p);
         return NIMBUS_OK;
     }
+    int upload(nimbus_hip_ctx* ctx) const { return copy_arrays(ctx, true, in); }
 };
-
-int back(float* host, const float* dev, std::size_t n, hipStream_t s)
-{
-    REF_TRY(hipMemcpyAsync(host, dev, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    return NIMBUS_OK;
-}
 
 // Four committed fields: copied to host staging, shown to the observer (if
 // any) while the caller's arrays still hold the old state, then published.
-int commit_four(float* const* host, float* const* dev, std::size_t n, hipStream_t s,
+int commit_four(nimbus_hip_ctx* ctx, float* const* host, float* const* dev, std::size_t n,
                 nimbus_four_field_observer observer, void* context)
 {
     std::vector<float> stage(4 * n);
-    for (int q = 0; q < 4; ++q)
-        REF_TRY(hipMemcpyAsync(stage.data() + q * n, dev[q], n * sizeof(float), hipMemcpyDeviceToHost, s));
-    REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> out;
+    for (int q = 0; q < 4; ++q) out.push_back(ArrayCopy{dev[q], stage.data() + q * n, n * sizeof(float)});
+    const int rc = copy_arrays(ctx, false, out);
+    if (rc != NIMBUS_OK) return rc;
     if (observer) observer(context, stage.data(), stage.data() + n, stage.data() + 2 * n, stage.data() + 3 * n);
     for (int q = 0; q < 4; ++q) std::memcpy(host[q], stage.data() + q * n, n * sizeof(float));
     return NIMBUS_OK;
@@ -932,6 +933,7 @@ int nimbus_hip_dispatch_cartesian_cgrid_slow_tendencies(nimbus_hip_ctx* ctx,
         rc = A.take(hin[q], hin[q] ? len[q] : std::max<std::size_t>(len[q], 1), s, &w_[q]);
     for (int q = 11; q < 19 && rc == NIMBUS_OK; ++q)
         if (q < 16 || adv) rc = A.take(nullptr, n, s, &w_[q]);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     v.u = w_[0]; v.v = w_[1]; v.w = w_[2]; v.rho = w_[3]; v.p = w_[4]; v.rho0 = w_[5]; v.qv0 = w_[6];
     v.u0 = w_[7]; v.v0 = w_[8]; v.qv = w_[9]; v.load = w_[10];
@@ -946,8 +948,9 @@ int nimbus_hip_dispatch_cartesian_cgrid_slow_tendencies(nimbus_hip_ctx* ctx,
     REF_TRY(hipStreamSynchronize(s));
     float* outs[8] = {d->du_dt_data, d->dv_dt_data, d->dw_dt_data, d->drho_dt_data, d->dp_dt_data,
                       d->du_advection_dt_data, d->dv_advection_dt_data, d->dw_advection_dt_data};
-    for (int q = 0; q < (adv ? 8 : 5) && rc == NIMBUS_OK; ++q) rc = back(outs[q], w_[11 + q], n, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> out;
+    for (int q = 0; q < (adv ? 8 : 5); ++q) out.push_back(ArrayCopy{w_[11 + q], outs[q], n * sizeof(float)});
+    rc = copy_arrays(ctx, false, out);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "cartesian_cgrid_slow_tendencies");
     return rc;
 }
@@ -967,13 +970,14 @@ int nimbus_hip_dispatch_slow_apply(nimbus_hip_ctx* ctx, const nimbus_slow_apply_
                             d->dv_dt_pbl};
     int rc = NIMBUS_OK;
     for (int q = 0; q < 10 && rc == NIMBUS_OK; ++q) rc = A.take(hin[q], n, s, &a[q]);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     hipLaunchKernelGGL(k_ref_slow_apply, dim3(blocks_for(n)), dim3(kThreads), 0, s, n, a[0], a[1], a[2], a[3], a[4],
                        a[5], a[6], a[7], a[8], a[9], double(d->dt_large), d->sanitize ? 1 : 0);
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
     float* outs[4] = {d->u, d->v, d->w, d->p_data};
-    rc = commit_four(outs, a, n, s, d->completed_observer, d->completed_observer_context);
+    rc = commit_four(ctx, outs, a, n, d->completed_observer, d->completed_observer_context);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "slow_apply");
     return rc;
 }
@@ -995,6 +999,7 @@ int nimbus_hip_dispatch_state_relaxation_cartesian(nimbus_hip_ctx* ctx, const ni
     int rc = NIMBUS_OK;
     for (int q = 0; q < 4 && rc == NIMBUS_OK; ++q) rc = A.take(hin[q], n, s, &a[q]);
     if (rc == NIMBUS_OK) rc = A.take(d->profiles, std::size_t(d->profiles_len), s, &a[4]);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     hipLaunchKernelGGL(k_ref_relax, dim3(blocks_for(n)), dim3(kThreads), 0, s, d->nx, d->ny, d->nz, a[0], a[1], a[2],
                        a[3], a[4], d->lateral_width, d->do_upper ? 1 : 0, d->do_w_only ? 1 : 0,
@@ -1002,7 +1007,7 @@ int nimbus_hip_dispatch_state_relaxation_cartesian(nimbus_hip_ctx* ctx, const ni
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
     float* outs[4] = {d->u, d->v, d->w, d->theta_data};
-    rc = commit_four(outs, a, n, s, d->completed_observer, d->completed_observer_context);
+    rc = commit_four(ctx, outs, a, n, d->completed_observer, d->completed_observer_context);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "state_relaxation_cartesian");
     return rc;
 }
@@ -1037,6 +1042,7 @@ int nimbus_hip_dispatch_microphysics_apply(nimbus_hip_ctx* ctx, const nimbus_mic
     if (rc == NIMBUS_OK) rc = A.take(d->dqv_pbl, n, s, &dqvp);
     if (rc == NIMBUS_OK && d->stats_out)
         rc = A.take(reinterpret_cast<const float*>(d->stats_out), std::size_t(d->stats_len), s, &st);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     v.drad = drad; v.dpbl = dpbl; v.dqvpbl = dqvp;
     v.stats = reinterpret_cast<unsigned*>(st);
@@ -1048,10 +1054,11 @@ int nimbus_hip_dispatch_microphysics_apply(nimbus_hip_ctx* ctx, const nimbus_mic
     hipLaunchKernelGGL(k_ref_micro_apply, dim3(blocks_for(n)), dim3(kThreads), 0, s, v);
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
-    for (int q = 0; q < 8 && rc == NIMBUS_OK; ++q)
-        if (fields[q]) rc = back(fields[q], v.q[q], n, s);
-    if (rc == NIMBUS_OK && d->stats_out) rc = back(reinterpret_cast<float*>(d->stats_out), st, d->stats_len, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> out;
+    for (int q = 0; q < 8; ++q)
+        if (fields[q]) out.push_back(ArrayCopy{v.q[q], fields[q], n * sizeof(float)});
+    if (d->stats_out) out.push_back(ArrayCopy{st, d->stats_out, std::size_t(d->stats_len) * sizeof(float)});
+    rc = copy_arrays(ctx, false, out);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "microphysics_apply");
     return rc;
 }
@@ -1072,6 +1079,7 @@ int nimbus_hip_dispatch_kessler_pointwise(nimbus_hip_ctx* ctx, const nimbus_kess
     const float* hin[6] = {d->temperature_data, d->p_data, d->qv_data, d->qc_data, d->qr_data, d->rho_d_data};
     int rc = NIMBUS_OK;
     for (int q = 0; q < 12 && rc == NIMBUS_OK; ++q) rc = A.take(q < 6 ? hin[q] : nullptr, n, s, &a[q]);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     KesslerPtView v{a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11],
                     d->nr, d->nth, d->nz, d->i_begin, d->i_end, d->j_begin, d->j_end, d->k_begin, d->k_end,
@@ -1081,9 +1089,10 @@ int nimbus_hip_dispatch_kessler_pointwise(nimbus_hip_ctx* ctx, const nimbus_kess
     REF_TRY(hipStreamSynchronize(s));
     float* outs[6] = {d->dtheta_dt_data, d->dqv_dt_data, d->dqc_dt_data, d->dqr_dt_data, d->dqg_dt_data,
                       d->dqh_dt_data};
-    for (int q = 0; q < 6 && rc == NIMBUS_OK; ++q)
-        if (outs[q]) rc = back(outs[q], a[6 + q], n, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> out;
+    for (int q = 0; q < 6; ++q)
+        if (outs[q]) out.push_back(ArrayCopy{a[6 + q], outs[q], n * sizeof(float)});
+    rc = copy_arrays(ctx, false, out);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "kessler_pointwise");
     return rc;
 }
@@ -1104,14 +1113,14 @@ int nimbus_hip_dispatch_kessler_sedimentation(nimbus_hip_ctx* ctx, const nimbus_
     if (rc == NIMBUS_OK && d->rho_d_data) rc = A.take(d->rho_d_data, n, s, &rho);
     if (rc == NIMBUS_OK && d->layer_thickness_m) rc = A.take(d->layer_thickness_m, n, s, &layer);
     if (rc == NIMBUS_OK) rc = A.take(d->dqr_dt_data, n, s, &dqr);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     KesslerSedView v{qr, rho, layer, dqr, d->nr, d->nth, d->nz, d->i_begin, d->i_end, d->j_begin, d->j_end,
                      d->k_begin, d->k_end, d->dz_val, d->Vt_max_rain, d->vt_cap};
     hipLaunchKernelGGL(k_ref_kessler_sed, dim3(blocks_for(std::size_t(d->nr) * d->nth)), dim3(kThreads), 0, s, v);
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
-    rc = back(d->dqr_dt_data, dqr, n, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    rc = copy_arrays(ctx, false, {ArrayCopy{dqr, d->dqr_dt_data, n * sizeof(float)}});
     if (rc == NIMBUS_OK) count_dispatch(ctx, "kessler_sedimentation");
     return rc;
 }
@@ -1143,6 +1152,7 @@ int nimbus_hip_dispatch_advect_scalars_conservative_cartesian_cgrid(
     }
     float* scratch = nullptr;
     if (rc == NIMBUS_OK) rc = A.take(nullptr, kTransportScratchFields * n, s, &scratch);
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
     if (rc != NIMBUS_OK) return rc;
     t.rho = rho;
     if (sup) { t.mfx = a; t.mfy = b; t.mfz = c; t.rho_begin = e; }
@@ -1152,8 +1162,9 @@ int nimbus_hip_dispatch_advect_scalars_conservative_cartesian_cgrid(
     enqueue_transport(*d, t, scratch, s);
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
-    for (int q = 0; q < d->n_scalars && rc == NIMBUS_OK; ++q) rc = back(d->q_out[q], qout[q], n, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> out;
+    for (int q = 0; q < d->n_scalars; ++q) out.push_back(ArrayCopy{qout[q], d->q_out[q], n * sizeof(float)});
+    rc = copy_arrays(ctx, false, out);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "advect_scalars_conservative_cartesian_cgrid");
     return rc;
 }
@@ -1170,26 +1181,29 @@ int nimbus_hip_dispatch_diffusion_batch(nimbus_hip_ctx* ctx, const nimbus_diffus
     float *rho = nullptr, *dz = nullptr;
     rc = A.take(d->rho, n, s, &rho);
     if (rc == NIMBUS_OK) rc = A.take(d->dz, std::size_t(d->nz), s, &dz);
-    std::vector<float*> out(d->count, nullptr);
+    std::vector<float*> f(d->count, nullptr), kv(d->count, nullptr), out(d->count, nullptr);
     for (int t = 0; t < d->count && rc == NIMBUS_OK; ++t)
     {
-        float *f = nullptr, *kv = nullptr;
-        rc = A.take(d->fields[t], n, s, &f);
+        rc = A.take(d->fields[t], n, s, &f[t]);
         const float* kvh = d->vertical_K ? d->vertical_K[t] : nullptr;
-        if (rc == NIMBUS_OK && kvh) rc = A.take(kvh, n, s, &kv);
+        if (rc == NIMBUS_OK && kvh) rc = A.take(kvh, n, s, &kv[t]);
         if (rc == NIMBUS_OK) rc = A.take(nullptr, n, s, &out[t]);
-        if (rc != NIMBUS_OK) break;
-        DiffusionView v{f, rho, dz, kv, out[t], d->nx, d->ny, d->nz, d->locations[t], d->c_grid != 0 ? 1 : 0,
+    }
+    if (rc == NIMBUS_OK) rc = A.upload(ctx);
+    if (rc != NIMBUS_OK) return rc;
+    for (int t = 0; t < d->count; ++t)
+    {
+        DiffusionView v{f[t], rho, dz, kv[t], out[t], d->nx, d->ny, d->nz, d->locations[t], d->c_grid != 0 ? 1 : 0,
                         d->periodic_x != 0 ? 1 : 0, d->periodic_y != 0 ? 1 : 0, double(d->dx), double(d->dy),
                         double(d->K_h), double(d->K_v)};
         hipLaunchKernelGGL(k_ref_diffusion, dim3(blocks_for(n)), dim3(kThreads), 0, s, v);
     }
-    if (rc != NIMBUS_OK) return rc;
     REF_TRY(hipGetLastError());
     REF_TRY(hipStreamSynchronize(s));
     // published only once every target has been computed
-    for (int t = 0; t < d->count && rc == NIMBUS_OK; ++t) rc = back(d->tendencies[t], out[t], n, s);
-    if (rc == NIMBUS_OK) REF_TRY(hipStreamSynchronize(s));
+    std::vector<ArrayCopy> tend;
+    for (int t = 0; t < d->count; ++t) tend.push_back(ArrayCopy{out[t], d->tendencies[t], n * sizeof(float)});
+    rc = copy_arrays(ctx, false, tend);
     if (rc == NIMBUS_OK) count_dispatch(ctx, "diffusion_batch");
     return rc;
 }

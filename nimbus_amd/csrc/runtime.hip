@@ -3,6 +3,7 @@
 // every kernel launch (device member table + block maps), hipGraph capture of
 // a batch's whole large step, per-kernel HIP-event timing and the C ABI
 // declared in nimbus_hip.h.
+#include "host_transfer.hpp"
 #include "kernels.hpp"
 #include "nimbus_internal.hpp"
 
@@ -224,6 +225,7 @@ struct nimbus_hip_ctx
     // captures (capture + instantiate), host wall clock
     std::uint64_t batch_builds = 0, graph_captures = 0;
     double batch_build_ms = 0.0, graph_capture_ms = 0.0;
+    nimbus::HostTransfer transfer;  // pinned slots of host array copies
 };
 
 namespace nimbus
@@ -724,91 +726,108 @@ int step_members(nimbus_hip_ctx* ctx, const std::uint32_t* ids, int n_ids, int n
     return NIMBUS_OK;
 }
 
-// Host field h (reference layout, element H) -> device field d via a staging buffer.
-template <class H>
-int upload_field(nimbus_hip_ctx* ctx, Member& m, const void* h, void* d, const double* subtract, void* staging)
+// Whether a kernel can reach the caller's array itself (it is device memory).
+bool device_array(const void* p)
 {
-    const std::size_t n = std::size_t(m.g().nx) * m.g().ny * m.g().nz;
-    NIMBUS_HIP_TRY(hipMemcpyAsync(staging, h, n * sizeof(H), hipMemcpyHostToDevice, ctx->stream));
-    Launcher L = make_launcher(ctx);
-    L.timing = false;
-    if (m.elem == 4) launch_host_to_dev<H, float>(L, m.g(), staging, d, subtract);
-    else launch_host_to_dev<H, double>(L, m.g(), staging, d, subtract);
-    if (L.error != hipSuccess) return hip_fail(L.error, "upload transpose");
-    return NIMBUS_OK;
+    hipPointerAttribute_t at{};
+    const bool yes = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
+    hipGetLastError();  // an ordinary host array is no error
+    return yes;
 }
 
-template <class H>
-int download_field(nimbus_hip_ctx* ctx, Member& m, const void* d, void* h, const double* add, void* staging)
+// A device field of a member and the host array it is read from or written to.
+struct FieldIo
 {
-    const std::size_t n = std::size_t(m.g().nx) * m.g().ny * m.g().nz;
-    Launcher L = make_launcher(ctx);
-    L.timing = false;
-    if (m.elem == 4) launch_dev_to_host<float, H>(L, m.g(), d, staging, add);
-    else launch_dev_to_host<double, H>(L, m.g(), d, staging, add);
-    if (L.error != hipSuccess) return hip_fail(L.error, "download transpose");
-    NIMBUS_HIP_TRY(hipMemcpyAsync(h, staging, n * sizeof(H), hipMemcpyDeviceToHost, ctx->stream));
-    NIMBUS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    return NIMBUS_OK;
-}
-
-struct Staging
-{
-    void* p = nullptr;
-    ~Staging()
-    {
-        if (p) hipFree(p);
-    }
+    void* dev;
+    const void* host;
+    const double* base;  // profile that the device field is the perturbation from
 };
+
+// Copies fields from (up) or to host arrays of elements H in the reference
+// layout, in parts of at most a slot: whole columns i where they fit.
+template <class H>
+int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::vector<FieldIo>& fields)
+{
+    const DevGrid& g = m.g();
+    const std::size_t rows = std::size_t(g.ny) * g.nz, slot = HostTransfer::kSlot / sizeof(H);
+    std::vector<HostChunk> chunks;
+    std::vector<HostPart> parts;
+    std::vector<std::size_t> of;
+    for (std::size_t q = 0; q < fields.size(); ++q)
+    {
+        char* const host = static_cast<char*>(const_cast<void*>(fields[q].host));
+        const bool direct = device_array(host);
+        std::size_t ni = std::max<std::size_t>(1, slot / rows);
+        if (ni >= 16) ni -= ni % 16;  // whole tiles of the kernel
+        const std::size_t nr = std::min(rows, slot);
+        for (std::size_t i = 0; i < std::size_t(g.nx); i += ni)
+            for (std::size_t r = 0; r < rows; r += nr)
+            {
+                const HostPart p{int(i), int(std::min(ni, g.nx - i)), int(r), int(std::min(nr, rows - r))};
+                chunks.push_back(HostChunk{host + (i * rows + r) * sizeof(H), std::size_t(p.ni) * p.nr * sizeof(H),
+                                           direct});
+                parts.push_back(p);
+                of.push_back(q);
+            }
+    }
+    Launcher L = make_launcher(ctx);
+    L.timing = false;
+    const hipError_t e = ctx->transfer.run(ctx->device, ctx->stream, up, chunks, [&](int c, char* p) {
+        const FieldIo& f = fields[of[c]];
+        if (m.elem == 4) launch_turn<float, H>(L, g, f.dev, p, f.base, !up, parts[c]);
+        else launch_turn<double, H>(L, g, f.dev, p, f.base, !up, parts[c]);
+        return L.error;
+    });
+    return e == hipSuccess ? NIMBUS_OK : hip_fail(e, up ? "upload" : "download");
+}
+
+// The state's nine fields; a field without a host array is left as it is.
+std::vector<FieldIo> state_fields(const Member& m, const nimbus_host_state& s)
+{
+    const void* hs[9] = {s.u, s.v, s.w, s.rho, s.p, s.theta, s.qv, s.qc, s.qr};
+    const DevFields& f = m.f();
+    void* ds[9] = {f.u, f.v, f.w, f.rp, f.pp, f.th, f.qv, f.qc, f.qr};
+    std::vector<FieldIo> io;
+    for (int q = 0; q < 9; ++q)
+        if (hs[q])
+            io.push_back(FieldIo{ds[q], hs[q],
+                                 q == 3 ? base_slot(m, kBaseRho0) : (q == 4 ? base_slot(m, kBaseP0) : nullptr)});
+    return io;
+}
 
 template <class H>
 int upload_state(nimbus_hip_ctx* ctx, Member& m, const nimbus_host_state& s)
 {
-    Staging st;
-    const std::size_t n = std::size_t(m.g().nx) * m.g().ny * m.g().nz;
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(H)));
-    const void* hs[9] = {s.u, s.v, s.w, s.rho, s.p, s.theta, s.qv, s.qc, s.qr};
-    const DevFields& f = m.f();
-    void* ds[9] = {f.u, f.v, f.w, f.rp, f.pp, f.th, f.qv, f.qc, f.qr};
-    for (int q = 0; q < 9; ++q)
-    {
-        if (!hs[q]) return fail(NIMBUS_EINVAL, "upload: null field");
-        const double* sub = q == 3 ? base_slot(m, kBaseRho0) : (q == 4 ? base_slot(m, kBaseP0) : nullptr);
-        const int rc = upload_field<H>(ctx, m, hs[q], ds[q], sub, st.p);
-        if (rc != NIMBUS_OK) return rc;
-        NIMBUS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    }
+    const std::vector<FieldIo> io = state_fields(m, s);
+    if (io.size() != 9) return fail(NIMBUS_EINVAL, "upload: null field");
+    const int rc = transfer_fields<H>(ctx, m, true, io);
+    if (rc != NIMBUS_OK) return rc;
     const std::size_t cols = std::size_t(m.g().nx) * m.g().ny;
     std::vector<double> rain(cols, 0.0);
     if (s.rain_mm)
         for (int i = 0; i < m.g().nx; ++i)
             for (int j = 0; j < m.g().ny; ++j)
                 rain[std::size_t(j) * m.g().nx + i] = s.rain_mm[std::size_t(i) * m.g().ny + j];
-    NIMBUS_HIP_TRY(hipMemcpy(f.rain, rain.data(), cols * sizeof(double), hipMemcpyHostToDevice));
+    NIMBUS_HIP_TRY(hipMemcpy(m.f().rain, rain.data(), cols * sizeof(double), hipMemcpyHostToDevice));
     return NIMBUS_OK;
+}
+
+// Fields of a new scratch member, which is zero where no array is given.
+int upload_scratch(nimbus_hip_ctx* ctx, const Member& m, const nimbus_host_state& s)
+{
+    return transfer_fields<float>(ctx, m, true, state_fields(m, s));
 }
 
 template <class H>
 int download_state(nimbus_hip_ctx* ctx, Member& m, const nimbus_host_state& s)
 {
-    Staging st;
-    const std::size_t n = std::size_t(m.g().nx) * m.g().ny * m.g().nz;
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(H)));
-    void* hs[9] = {s.u, s.v, s.w, s.rho, s.p, s.theta, s.qv, s.qc, s.qr};
-    const DevFields& f = m.f();
-    void* ds[9] = {f.u, f.v, f.w, f.rp, f.pp, f.th, f.qv, f.qc, f.qr};
-    for (int q = 0; q < 9; ++q)
-    {
-        if (!hs[q]) continue;
-        const double* add = q == 3 ? base_slot(m, kBaseRho0) : (q == 4 ? base_slot(m, kBaseP0) : nullptr);
-        const int rc = download_field<H>(ctx, m, ds[q], hs[q], add, st.p);
-        if (rc != NIMBUS_OK) return rc;
-    }
+    const int rc = transfer_fields<H>(ctx, m, false, state_fields(m, s));
+    if (rc != NIMBUS_OK) return rc;
     if (s.rain_mm)
     {
         const std::size_t cols = std::size_t(m.g().nx) * m.g().ny;
         std::vector<double> rain(cols);
-        NIMBUS_HIP_TRY(hipMemcpy(rain.data(), f.rain, cols * sizeof(double), hipMemcpyDeviceToHost));
+        NIMBUS_HIP_TRY(hipMemcpy(rain.data(), m.f().rain, cols * sizeof(double), hipMemcpyDeviceToHost));
         for (int i = 0; i < m.g().nx; ++i)
             for (int j = 0; j < m.g().ny; ++j)
                 s.rain_mm[std::size_t(i) * m.g().ny + j] = rain[std::size_t(j) * m.g().nx + i];
@@ -1536,10 +1555,9 @@ int nimbus_hip_dispatch_acoustic_substep_fused(nimbus_hip_ctx* ctx, const nimbus
     p.dt = d->dt_small_host;
     p.mf_weight = 0.0;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    std::vector<float> zero(std::size_t(d->nx) * d->ny * d->nz, 0.0f);
-    nimbus_host_state hs{d->u, d->v, d->w, d->rho, d->p, const_cast<float*>(d->theta_data), zero.data(), zero.data(),
-                         zero.data(), nullptr};
-    rc = upload_state<float>(ctx, m, hs);
+    nimbus_host_state hs{d->u, d->v, d->w, d->rho, d->p, const_cast<float*>(d->theta_data), nullptr, nullptr, nullptr,
+                         nullptr};
+    rc = upload_scratch(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
     Launcher L = make_launcher(ctx);
     launch_acoustic_substep<float>(L, sm.batch.view, 0, false, false, false);
@@ -1584,44 +1602,29 @@ int nimbus_hip_dispatch_acoustic_substeps_batched(nimbus_hip_ctx* ctx,
     p.dt = d->dt_small * d->n_substeps;
     p.mf_weight = d->mass_flux_weight;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    std::vector<float> zero(std::size_t(d->nx) * d->ny * d->nz, 0.0f);
-    nimbus_host_state hs{d->u, d->v, d->w, d->rho, d->p, const_cast<float*>(d->theta_data), zero.data(), zero.data(),
-                         zero.data(), nullptr};
-    rc = upload_state<float>(ctx, m, hs);
+    nimbus_host_state hs{d->u, d->v, d->w, d->rho, d->p, const_cast<float*>(d->theta_data), nullptr, nullptr, nullptr,
+                         nullptr};
+    rc = upload_scratch(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
-    Staging st;
-    const std::size_t n = zero.size();
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(float)));
     const DevFields& f = m.f();
     if (d->accumulate_mass_flux)
     {
-        const void* src[3] = {d->mass_flux_x, d->mass_flux_y, d->mass_flux_z};
-        void* dst[3] = {f.mfx, f.mfy, f.mfz};
-        for (int q = 0; q < 3; ++q)
-        {
-            rc = upload_field<float>(ctx, m, src[q], dst[q], nullptr, st.p);
-            if (rc != NIMBUS_OK) return rc;
-            NIMBUS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-        }
+        rc = transfer_fields<float>(ctx, m, true, {{f.mfx, d->mass_flux_x, nullptr}, {f.mfy, d->mass_flux_y, nullptr},
+                                                   {f.mfz, d->mass_flux_z, nullptr}});
+        if (rc != NIMBUS_OK) return rc;
     }
     Launcher L = make_launcher(ctx);
     for (int s = 0; s < d->n_substeps; ++s)
         launch_acoustic_substep<float>(L, sm.batch.view, s, d->accumulate_mass_flux != 0, false, true);
     launch_commit<float>(L, sm.batch.view, d->n_substeps);
     if (L.error != hipSuccess) return hip_fail(L.error, "batched acoustic launch");
-    nimbus_host_state out{d->u, d->v, d->w, d->rho, d->p, nullptr, nullptr, nullptr, nullptr, nullptr};
-    rc = download_state<float>(ctx, m, out);
-    if (rc != NIMBUS_OK) return rc;
+    const nimbus_host_state out{d->u, d->v, d->w, d->rho, d->p, nullptr, nullptr, nullptr, nullptr, nullptr};
+    std::vector<FieldIo> io = state_fields(m, out);
     if (d->accumulate_mass_flux)
-    {
-        void* dst[3] = {d->mass_flux_x, d->mass_flux_y, d->mass_flux_z};
-        const void* src[3] = {f.mfx, f.mfy, f.mfz};
-        for (int q = 0; q < 3; ++q)
-        {
-            rc = download_field<float>(ctx, m, src[q], dst[q], nullptr, st.p);
-            if (rc != NIMBUS_OK) return rc;
-        }
-    }
+        io.insert(io.end(), {{f.mfx, d->mass_flux_x, nullptr}, {f.mfy, d->mass_flux_y, nullptr},
+                             {f.mfz, d->mass_flux_z, nullptr}});
+    rc = transfer_fields<float>(ctx, m, false, io);
+    if (rc != NIMBUS_OK) return rc;
     harvest(ctx);
     return NIMBUS_OK;
 }
@@ -1643,25 +1646,18 @@ int nimbus_hip_dispatch_slow_tendencies(nimbus_hip_ctx* ctx, const nimbus_slow_t
     m.args.p.coriolis_f = d->coriolis_f;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
     const std::size_t n = std::size_t(d->nr) * d->nth * d->nz;
-    std::vector<float> zero(n, 0.0f);
     nimbus_host_state hs{const_cast<float*>(d->u_data), const_cast<float*>(d->v_data), const_cast<float*>(d->w_data),
-                         const_cast<float*>(d->rho_data), zero.data(), zero.data(), const_cast<float*>(d->qv_data),
+                         const_cast<float*>(d->rho_data), nullptr, nullptr, const_cast<float*>(d->qv_data),
                          const_cast<float*>(d->qc_data), const_cast<float*>(d->qr_data), nullptr};
-    rc = upload_state<float>(ctx, m, hs);
+    rc = upload_scratch(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
     const DevFields& f = m.f();
     Launcher L = make_launcher(ctx);
     launch_slow_tendencies<float>(L, sm.batch.view, f.k1u, f.k1v, f.k1w);
     if (L.error != hipSuccess) return hip_fail(L.error, "slow tendencies launch");
-    Staging st;
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(float)));
-    void* outs[3] = {d->du_dt_data, d->dv_dt_data, d->dw_dt_data};
-    void* srcs[3] = {f.k1u, f.k1v, f.k1w};
-    for (int q = 0; q < 3; ++q)
-    {
-        rc = download_field<float>(ctx, m, srcs[q], outs[q], nullptr, st.p);
-        if (rc != NIMBUS_OK) return rc;
-    }
+    rc = transfer_fields<float>(ctx, m, false, {{f.k1u, d->du_dt_data, nullptr}, {f.k1v, d->dv_dt_data, nullptr},
+                                                {f.k1w, d->dw_dt_data, nullptr}});
+    if (rc != NIMBUS_OK) return rc;
     harvest(ctx);
     return NIMBUS_OK;
 }
@@ -1683,10 +1679,9 @@ int nimbus_hip_dispatch_slow_rk2(nimbus_hip_ctx* ctx, const nimbus_slow_rk2_disp
     m.args.p.dt = d->dt_large;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
     const std::size_t n = std::size_t(d->nx) * d->ny * d->nz;
-    std::vector<float> zero(n, 0.0f);
-    nimbus_host_state hs{d->u, d->v, d->w, const_cast<float*>(d->rho), zero.data(), zero.data(),
+    nimbus_host_state hs{d->u, d->v, d->w, const_cast<float*>(d->rho), nullptr, nullptr,
                          const_cast<float*>(d->qv), const_cast<float*>(d->qc), const_cast<float*>(d->qr), nullptr};
-    rc = upload_state<float>(ctx, m, hs);
+    rc = upload_scratch(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
     Launcher L = make_launcher(ctx);
     launch_slow_rk2<float>(L, sm.batch.view);
@@ -1723,37 +1718,27 @@ int nimbus_hip_dispatch_advect_scalars(nimbus_hip_ctx* ctx, const nimbus_advect_
     m.args.p.dt = d->dt;
     m.args.p.bc_top = d->bc_top;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    const std::size_t n = std::size_t(d->nx) * d->ny * d->nz;
-    Staging st;
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(float)));
     const DevFields& f = m.f();
     // rho0 = 0 in the scratch member, so rho' slots hold the full densities.
-    const void* src[5] = {d->mass_flux_x, d->mass_flux_y, d->mass_flux_z, d->rho_begin, d->rho_end};
-    void* dst[5] = {f.mfx, f.mfy, f.mfz, f.rb, f.rp};
-    for (int q = 0; q < 5; ++q)
-    {
-        rc = upload_field<float>(ctx, m, src[q], dst[q], nullptr, st.p);
-        if (rc != NIMBUS_OK) return rc;
-        NIMBUS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    }
+    std::vector<FieldIo> in{{f.mfx, d->mass_flux_x, nullptr}, {f.mfy, d->mass_flux_y, nullptr},
+                            {f.mfz, d->mass_flux_z, nullptr}, {f.rb, d->rho_begin, nullptr}, {f.rp, d->rho_end, nullptr}};
+    std::vector<FieldIo> out;
     void* qin[4] = {f.th, f.qv, f.qc, f.qr};
     void* qout[4] = {f.tth, f.tqv, f.tqc, f.tqr};
     int pd[4] = {0, 0, 0, 0};
     for (int s = 0; s < d->n_scalars; ++s)
     {
-        rc = upload_field<float>(ctx, m, d->q[s], qin[s], nullptr, st.p);
-        if (rc != NIMBUS_OK) return rc;
-        NIMBUS_HIP_TRY(hipStreamSynchronize(ctx->stream));
+        in.push_back(FieldIo{qin[s], d->q[s], nullptr});
+        out.push_back(FieldIo{qout[s], d->q[s], nullptr});
         pd[s] = d->positive_definite[s] != 0;
     }
+    rc = transfer_fields<float>(ctx, m, true, in);
+    if (rc != NIMBUS_OK) return rc;
     Launcher L = make_launcher(ctx);
     launch_transport<float>(L, sm.batch.view, d->n_scalars, pd, true);
     if (L.error != hipSuccess) return hip_fail(L.error, "advect launch");
-    for (int s = 0; s < d->n_scalars; ++s)
-    {
-        rc = download_field<float>(ctx, m, qout[s], d->q[s], nullptr, st.p);
-        if (rc != NIMBUS_OK) return rc;
-    }
+    rc = transfer_fields<float>(ctx, m, false, out);
+    if (rc != NIMBUS_OK) return rc;
     harvest(ctx);
     return NIMBUS_OK;
 }
@@ -1785,27 +1770,44 @@ int nimbus_hip_dispatch_kessler(nimbus_hip_ctx* ctx, const nimbus_kessler_dispat
     m.args.p.kessler = KesslerConst{d->qc0, d->c_auto, d->c_accr, d->evap_eff, d->vt_max};
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
     const std::size_t n = std::size_t(d->nx) * d->ny * d->nz;
-    std::vector<float> zero(n, 0.0f);
-    nimbus_host_state hs{zero.data(), zero.data(), zero.data(), const_cast<float*>(d->rho), const_cast<float*>(d->p),
+    nimbus_host_state hs{nullptr, nullptr, nullptr, const_cast<float*>(d->rho), const_cast<float*>(d->p),
                          const_cast<float*>(d->theta), const_cast<float*>(d->qv), const_cast<float*>(d->qc),
                          const_cast<float*>(d->qr), nullptr};
-    // upload_state subtracts base slots that are zero here
-    rc = upload_state<float>(ctx, m, hs);
+    // the base slots that the upload subtracts are zero here
+    rc = upload_scratch(ctx, m, hs);
     if (rc != NIMBUS_OK) return rc;
     Launcher L = make_launcher(ctx);
     launch_kessler_tendencies<float>(L, sm.batch.view, d->dt, f.k1u, f.k1v, f.k1w, f.u2);
     if (L.error != hipSuccess) return hip_fail(L.error, "kessler launch");
-    Staging st;
-    NIMBUS_HIP_TRY(hipMalloc(&st.p, n * sizeof(float)));
-    void* outs[4] = {d->dtheta_dt, d->dqv_dt, d->dqc_dt, d->dqr_dt};
-    void* srcs[4] = {f.k1u, f.k1v, f.k1w, f.u2};
-    for (int q = 0; q < 4; ++q)
-    {
-        rc = download_field<float>(ctx, m, srcs[q], outs[q], nullptr, st.p);
-        if (rc != NIMBUS_OK) return rc;
-    }
+    rc = transfer_fields<float>(ctx, m, false, {{f.k1u, d->dtheta_dt, nullptr}, {f.k1v, d->dqv_dt, nullptr},
+                                                {f.k1w, d->dqc_dt, nullptr}, {f.u2, d->dqr_dt, nullptr}});
+    if (rc != NIMBUS_OK) return rc;
     harvest(ctx);
     return NIMBUS_OK;
 }
 
 }  // extern "C"
+
+namespace nimbus
+{
+int copy_arrays(nimbus_hip_ctx* ctx, bool up, const std::vector<ArrayCopy>& arrays)
+{
+    std::vector<HostChunk> chunks;
+    std::vector<char*> dev;
+    for (const ArrayCopy& a : arrays)
+    {
+        const bool direct = a.bytes != 0 && device_array(a.host);
+        for (std::size_t o = 0; o < a.bytes; o += HostTransfer::kSlot)
+        {
+            const std::size_t n = std::min(HostTransfer::kSlot, a.bytes - o);
+            chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, n, direct});
+            dev.push_back(static_cast<char*>(a.dev) + o);
+        }
+    }
+    const hipError_t e = ctx->transfer.run(ctx->device, ctx->stream, up, chunks, [&](int c, char* p) {
+        return up ? hipMemcpyAsync(dev[c], p, chunks[c].bytes, hipMemcpyDefault, ctx->stream)
+                  : hipMemcpyAsync(p, dev[c], chunks[c].bytes, hipMemcpyDefault, ctx->stream);
+    });
+    return e == hipSuccess ? NIMBUS_OK : hip_fail(e, up ? "upload" : "download");
+}
+}  // namespace nimbus

@@ -699,3 +699,35 @@ def test_accuracy_run_reports_the_fp32_rounding_control(hip_ctx):
           "control", c["w_pointwise_max_error"], c["theta_p_rms_difference"])
     assert c["theta_p_rms_difference"] < res["theta_p_rms_difference"]
     assert c["w_pointwise_max_error"] < 1e-3
+
+
+@pytest.mark.parametrize("precision", [L.PRECISION_MIXED, L.PRECISION_FP64])
+@pytest.mark.parametrize("shape", [(5, 5, 4), (17, 9, 129), (70, 300, 130), (5, 1031, 1024)])
+def test_upload_then_download_returns_the_fields(hip_ctx, shape, precision):
+    """Host arrays through the pinned slots: less than a slot, ragged tiles of
+    the transposition, more parts than slots, and planes larger than a slot.
+    Fields stored whole come back bitwise; rho and p, stored as perturbations,
+    within the two roundings of the storage type (x - base is below 2 x)."""
+    nx, ny, nz = shape
+    g = L.make_grid(nx, ny, nz, 1000.0, 1000.0, 20000.0 / nz)
+    base = L.base_state(g)
+    m = hip_ctx.member(g, L.step_config(3.0, 6), base, precision)
+    dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
+    eps = np.finfo(dtype).eps
+    r = np.random.default_rng(5)
+    try:
+        st = {f: r.random(shape, np.float32).astype(dtype) + dtype(0.25) for f in L.FIELDS}
+        st["p"] = st["p"] * dtype(1.0e5)
+        rain = r.random((nx, ny))
+        m.upload(dict(st, rain_mm=rain))
+        out = m.download()
+    finally:
+        m.destroy()
+    for f in L.FIELDS:
+        if f in ("rho", "p"):
+            slot = np.asarray(base["rho0" if f == "rho" else "p0"], np.float64)[None, None, :]
+            bound = 0.5 * eps * (np.abs(st[f] - slot) + 1.5 * np.abs(st[f]))
+            assert np.all(np.abs(out[f].astype(np.float64) - st[f]) <= bound), f
+        else:
+            assert np.array_equal(out[f], st[f]), f
+    assert np.array_equal(out["rain_mm"], rain)
