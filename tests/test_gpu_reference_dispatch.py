@@ -287,6 +287,28 @@ def test_conservative_transport_matches_oracle(hip_ctx, rng, supplied):
         assert nbad == 0, name
 
 
+@pytest.mark.parametrize("power", [20, 60, 110])
+def test_conservative_transport_scales_with_its_scalar(hip_ctx, rng, power):
+    """The reconstruction's weights do not depend on the scalar's unit: a scalar
+    times 2^power gives the result times 2^power (2^110 theta takes the weights
+    that are formed one by one). Two roundings of a result may differ by one in
+    the last place, and a face flux by one more."""
+    from tests.test_gpu_parity import _transport_inputs
+    g, base, st = small_case(nx=11, ny=9, nz=7, cloudy=True)
+    (mfx, mfy, mfz), rho_b, rho_e = _transport_inputs(g, base, st, 4.0, rng)
+    theta = np.ascontiguousarray(st["theta"], F32)
+    kap, pd, outs = np.zeros(1, F32), (ctypes.c_int * 1)(0), []
+    for q in (theta, theta * F32(2.0 ** power)):
+        out = np.zeros_like(q)
+        qin, qout = (ctypes.POINTER(ctypes.c_float) * 1)(fp(q)), (ctypes.POINTER(ctypes.c_float) * 1)(fp(out))
+        d = L.ConservativeTransportDispatch(None, None, None, fp(rho_e), qin, qout, fp(kap), pd, 1, g.nx, g.ny, g.nz,
+                                            1.0 / g.dx, 1.0 / g.dy, 1.0 / g.dz, 0.0, 0.0, 0.0, 4.0, 0.05, fp(rho_b),
+                                            fp(mfx), fp(mfy), fp(mfz), 1, 0.0, 0.0, 1, 0)
+        call(hip_ctx, "nimbus_hip_dispatch_advect_scalars_conservative_cartesian_cgrid", d)
+        outs.append(out.astype(np.float64))
+    assert np.all(np.abs(outs[1] * 2.0 ** -power - outs[0]) <= 2.0 ** -22 * np.abs(outs[0]))
+
+
 def test_reference_contract_refusals_leave_host_fields_untouched(hip_ctx):
     shape = (8, 7, 6)
     q = np.ones(shape, F32)
