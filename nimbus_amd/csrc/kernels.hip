@@ -756,6 +756,10 @@ __global__ __launch_bounds__(kBlock) void k_acoustic_forward(const MemberArgs* _
 // per 8 faces, for the vertical (us per substep): 400 x 400 x 100 mixed
 // 441 -> 417, 640 x 640 x 60 674 -> 463, 100 x 120 x 140 138 -> 78,
 // 160 x 160 x 80 82 -> 64, 48 x 48 x 40 21 -> 13, 256 x 256 x 80 FP64 262 -> 251.
+// At most 96 VGPRs (the launch bound): five waves per SIMD, so that four
+// workgroups of 80 levels share a CU instead of three: 160 x 160 x 80 62.6 ->
+// 53.1 us against 104 VGPRs, 400 x 400 x 100 426 -> 405, 100 x 120 x 140 78 ->
+// 74. The next step, 80 VGPRs, spills.
 template <class S>
 using Vec = __attribute__((ext_vector_type(16 / sizeof(S)))) S;
 
@@ -873,7 +877,7 @@ __device__ __forceinline__ double substitute(const double* gq, double* bq, int h
 }
 
 template <class S, bool FIRST, int LL>
-__global__ __launch_bounds__(1024) void k_hevi_solve(const MemberArgs* __restrict__ ma, const int2* __restrict__ map,
+__global__ __launch_bounds__(1024, 5) void k_hevi_solve(const MemberArgs* __restrict__ ma, const int2* __restrict__ map,
                                                      int s)
 {
     constexpr int V = 16 / int(sizeof(S)), CW = LL * V;
@@ -928,37 +932,53 @@ __global__ __launch_bounds__(1024) void k_hevi_solve(const MemberArgs* __restric
     const double r0 = pr.rho0(k), r0u = pr.rho0(min(k + 1, NZ - 1));
     Vec<S> rs;
     double gk[V], H[V];
+    // one axis after the other, so that an axis's operands are done with before
+    // the next one's results need registers (96 of them: five waves per SIMD)
+    double dh[V];
     {
-        Vec<S> mxn, myn;
+        Vec<S> mn;
 #pragma unroll
         for (int e = 0; e < V; ++e)
         {
-            const int i = i0 + e;
-            const bool in = solve && i >= 1 && i < NX - 1;
+            // twice the face fluxes (the factor 1/2 is in the constants)
             const double rc = r0 + double(r[e]);
             const S rxp = e + 1 < V ? r[e + 1 < V ? e + 1 : 0] : rr, rxm = e > 0 ? r[e > 0 ? e - 1 : 0] : rl;
             const S um = e > 0 ? u[e > 0 ? e - 1 : 0] : ul;
-            // twice the face fluxes (the factor 1/2 is in the constants)
             const double fxp = (rc + (r0 + double(rxp))) * double(u[e]);
+            mn[e] = i0 + e < NX - 1 ? S(double(mx[e]) + hw * fxp) : mx[e];
+            dh[e] = fma(-((r0 + double(rxm)) + rc), double(um), fxp) * hix;
+        }
+        if (active) stv<S>(f.mfx, c, mn);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        Vec<S> mn;
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+        {
+            const double rc = r0 + double(r[e]);
             const double fyp = (rc + (r0 + double(ryp[e]))) * double(v[e]);
-            mxn[e] = i < NX - 1 ? S(double(mx[e]) + hw * fxp) : mx[e];
-            myn[e] = i < NX && j < NY - 1 ? S(double(my[e]) + hw * fyp) : my[e];
-            const double dxf = fma(-((r0 + double(rxm)) + rc), double(um), fxp);
-            const double dyf = fma(-((r0 + double(rym[e])) + rc), double(vm[e]), fyp);
-            const double dh = -(dxf * hix + dyf * hiy);
-            const double rstar = in ? rc + dts * finite0(dh) : rc;
-            rs[e] = S(rstar - r0);
-            // linearisation point p* = EOS(rho*), as a perturbation
-            const double psf = solve ? eos_full_pressure<S>(pr, k, rstar, double(th[e])) : 0.0;
-            gk[e] = in ? bc2g * psf * rcp_nr(r0 + double(rs[e])) : 0.0;
-            H[e] = in ? cdt * alpha * (psf - pr.p0(k)) : 0.0;
+            mn[e] = i0 + e < NX && j < NY - 1 ? S(double(my[e]) + hw * fyp) : my[e];
+            dh[e] = -fma(fma(-((r0 + double(rym[e])) + rc), double(vm[e]), fyp), hiy, dh[e]);
         }
         if (active)
         {
-            stv<S>(f.mfx, c, mxn);
-            stv<S>(f.mfy, c, myn);
+            stv<S>(f.mfy, c, mn);
             if (FIRST) stv<S>(f.rb, c, r);
         }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+    {
+        const bool in = solve && i0 + e >= 1 && i0 + e < NX - 1;
+        const double rc = r0 + double(r[e]);
+        const double rstar = in ? rc + dts * finite0(dh[e]) : rc;
+        rs[e] = S(rstar - r0);
+        // linearisation point p* = EOS(rho*), as a perturbation
+        const double psf = solve ? eos_full_pressure<S>(pr, k, rstar, double(th[e])) : 0.0;
+        gk[e] = in ? bc2g * psf * rcp_nr(r0 + double(rs[e])) : 0.0;
+        H[e] = in ? cdt * alpha * (psf - pr.p0(k)) : 0.0;
     }
     __builtin_amdgcn_sched_barrier(0);
     const unsigned zp = k < NZ - 1 ? c + plane : c, zm = k > 0 ? c - plane : c;
