@@ -64,6 +64,7 @@ public:
         // a thread for each MB: below that starting one costs as much as it takes over
         const int want = int(std::min<std::size_t>({std::size_t(kThreads), chunks.size(), bytes >> 20}));
         std::vector<std::thread> team;
+        team.reserve(kThreads);  // no allocation once a thread runs
         try
         {
             for (int t = 1; t < want; ++t)
