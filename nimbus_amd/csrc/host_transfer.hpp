@@ -21,6 +21,14 @@
 namespace nimbus
 {
 
+// A whole array and its copy on the device. No bytes: no copy.
+struct ArrayCopy
+{
+    void* dev;
+    void* host;
+    std::size_t bytes;
+};
+
 // A contiguous piece of one of the caller's arrays; direct: the kernel can
 // reach the array itself (device memory), nothing is copied.
 struct HostChunk
@@ -36,6 +44,23 @@ public:
     static constexpr std::size_t kSlot = std::size_t(2) << 20;
     static constexpr int kSlots = 10;
     static constexpr int kThreads = 6;
+    // Whole arrays take the ring from these sizes of one direction on (down:
+    // and of an array on average). Below them the ring's threads and the copy,
+    // event and wait of every chunk cost more than they overlap. Plain copies
+    // against the ring, us: down (18 GB/s plain), 16 x 128 KB 246 to 297, 4 x 512 KB
+    // 116 to 133, 8 x 512 KB 258 to 225, 2 x 2 MB 230 to 180, 4 x 2 MB 461 to 318; up,
+    // where a plain copy reads warm pages at 35 GB/s and runs beside the caller's
+    // next allocation, whole calls with 9 arrays of 96 x 96 x 60 floats (20 MB)
+    // 1,850 to 2,120, of 112 x 112 x 60 (27 MB) 2,500 to 2,900, with 4 of
+    // 160 x 160 x 80 (33 MB) 3,840 to 3,530, with 5 of them 6,590 to 6,040.
+    static constexpr std::size_t kRingDown = std::size_t(4) << 20;
+    static constexpr std::size_t kRingArray = std::size_t(512) << 10;
+    static constexpr std::size_t kRingUp = std::size_t(32) << 20;
+    // Whether `count` arrays of `bytes` together take the ring.
+    static constexpr bool takes_ring(bool up, std::size_t bytes, std::size_t count)
+    {
+        return up ? bytes >= kRingUp : bytes >= kRingDown && bytes >= count * kRingArray;
+    }
 
     HostTransfer() = default;
     HostTransfer(const HostTransfer&) = delete;
@@ -61,8 +86,10 @@ public:
         st.copied.assign(chunks.size(), 0);
         std::size_t bytes = 0;
         for (const HostChunk& c : chunks) bytes += c.bytes;
-        // a thread for each MB: below that starting one costs as much as it takes over
-        const int want = int(std::min<std::size_t>({std::size_t(kThreads), chunks.size(), bytes >> 20}));
+        // a thread for each 4 MB: one for each MB took 2,040 us where this takes 1,910 (a contract
+        // call of 13 arrays of 96 x 96 x 60 floats) and 435 where this takes 408 (9 of 64 x 64 x 48
+        // doubles), in starting them and in the release of device memory beside them
+        const int want = int(std::min<std::size_t>({std::size_t(kThreads), chunks.size(), bytes >> 22}));
         std::vector<std::thread> team;
         team.reserve(kThreads);  // no allocation once a thread runs
         try
@@ -108,6 +135,53 @@ public:
         for (std::thread& t : team) t.join();
         e = hipStreamSynchronize(stream);
         return st.error != hipSuccess ? st.error : e;
+    }
+
+    // Copies whole arrays to (up) or from the device. Downloads are complete on
+    // return; uploads precede what is enqueued on `stream` next, and the arrays
+    // are read by the time that `stream` has run.
+    hipError_t copy(int device, hipStream_t stream, bool up, const std::vector<ArrayCopy>& arrays)
+    {
+        std::size_t bytes = 0, count = 0;
+        for (const ArrayCopy& a : arrays)
+        {
+            bytes += a.bytes;
+            count += a.bytes != 0;
+        }
+        const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+        if (!takes_ring(up, bytes, count))
+        {
+            for (const ArrayCopy& a : arrays)
+            {
+                if (a.bytes == 0) continue;
+                const hipError_t e = hipMemcpyAsync(up ? a.dev : a.host, up ? a.host : a.dev, a.bytes, kind, stream);
+                if (e != hipSuccess) return e;
+            }
+            return up ? hipSuccess : hipStreamSynchronize(stream);
+        }
+        std::vector<HostChunk> chunks;
+        std::vector<char*> dev;
+        for (const ArrayCopy& a : arrays)
+        {
+            const bool direct = a.bytes != 0 && device_array(a.host);
+            for (std::size_t o = 0; o < a.bytes; o += kSlot)
+            {
+                chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, std::min(kSlot, a.bytes - o), direct});
+                dev.push_back(static_cast<char*>(a.dev) + o);
+            }
+        }
+        return run(device, stream, up, chunks, [&](int c, char* p) {
+            return hipMemcpyAsync(up ? dev[c] : p, up ? p : dev[c], chunks[c].bytes, hipMemcpyDefault, stream);
+        });
+    }
+
+    // Whether a kernel can reach the caller's array itself (it is device memory).
+    static bool device_array(const void* p)
+    {
+        hipPointerAttribute_t at{};
+        const bool yes = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
+        hipGetLastError();  // an ordinary host array is no error
+        return yes;
     }
 
 private:

@@ -9,6 +9,7 @@
 #include <string>
 #include <vector>
 
+#include "host_transfer.hpp"
 #include "nimbus_hip.h"
 
 namespace nimbus
@@ -42,14 +43,7 @@ int resolve_substeps(const nimbus_grid& g, const double* rho0, const double* p0,
 int context_device(nimbus_hip_ctx* ctx);
 hipStream_t context_stream(nimbus_hip_ctx* ctx);
 void count_dispatch(nimbus_hip_ctx* ctx, const char* op);
-// Copies whole arrays from (up) or to the host through the context's pinned
-// slots and waits. A copy of no bytes is none.
-struct ArrayCopy
-{
-    void* dev;
-    void* host;
-    std::size_t bytes;
-};
+// HostTransfer::copy on a context's stream.
 int copy_arrays(nimbus_hip_ctx* ctx, bool up, const std::vector<ArrayCopy>& arrays);
 
 // Device grid descriptor. Device fields are stored [k][j][i] with i

@@ -3,7 +3,6 @@
 // every kernel launch (device member table + block maps), hipGraph capture of
 // a batch's whole large step, per-kernel HIP-event timing and the C ABI
 // declared in nimbus_hip.h.
-#include "host_transfer.hpp"
 #include "kernels.hpp"
 #include "nimbus_internal.hpp"
 
@@ -726,15 +725,6 @@ int step_members(nimbus_hip_ctx* ctx, const std::uint32_t* ids, int n_ids, int n
     return NIMBUS_OK;
 }
 
-// Whether a kernel can reach the caller's array itself (it is device memory).
-bool device_array(const void* p)
-{
-    hipPointerAttribute_t at{};
-    const bool yes = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
-    hipGetLastError();  // an ordinary host array is no error
-    return yes;
-}
-
 // A device field of a member and the host array it is read from or written to.
 struct FieldIo
 {
@@ -756,7 +746,7 @@ int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::ve
     for (std::size_t q = 0; q < fields.size(); ++q)
     {
         char* const host = static_cast<char*>(const_cast<void*>(fields[q].host));
-        const bool direct = device_array(host);
+        const bool direct = HostTransfer::device_array(host);
         std::size_t ni = std::max<std::size_t>(1, slot / rows);
         if (ni >= 16) ni -= ni % 16;  // whole tiles of the kernel
         const std::size_t nr = std::min(rows, slot);
@@ -1792,22 +1782,7 @@ namespace nimbus
 {
 int copy_arrays(nimbus_hip_ctx* ctx, bool up, const std::vector<ArrayCopy>& arrays)
 {
-    std::vector<HostChunk> chunks;
-    std::vector<char*> dev;
-    for (const ArrayCopy& a : arrays)
-    {
-        const bool direct = a.bytes != 0 && device_array(a.host);
-        for (std::size_t o = 0; o < a.bytes; o += HostTransfer::kSlot)
-        {
-            const std::size_t n = std::min(HostTransfer::kSlot, a.bytes - o);
-            chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, n, direct});
-            dev.push_back(static_cast<char*>(a.dev) + o);
-        }
-    }
-    const hipError_t e = ctx->transfer.run(ctx->device, ctx->stream, up, chunks, [&](int c, char* p) {
-        return up ? hipMemcpyAsync(dev[c], p, chunks[c].bytes, hipMemcpyDefault, ctx->stream)
-                  : hipMemcpyAsync(p, dev[c], chunks[c].bytes, hipMemcpyDefault, ctx->stream);
-    });
+    const hipError_t e = ctx->transfer.copy(ctx->device, ctx->stream, up, arrays);
     return e == hipSuccess ? NIMBUS_OK : hip_fail(e, up ? "upload" : "download");
 }
 }  // namespace nimbus

@@ -116,6 +116,22 @@ def test_slow_apply_follows_its_definition(hip_ctx, rng):
     assert np.array_equal(seen["u"], u_dev) and np.array_equal(seen["old_u"], u)
 
 
+@pytest.mark.parametrize("shape", [(8, 7, 6), (80, 80, 60), (128, 127, 61)])
+def test_slow_apply_is_whole_on_every_transfer_route(hip_ctx, shape):
+    """The ten arrays up and four down as plain copies, plain up and through
+    the ring down, and through the ring both ways, with lengths that are no
+    multiple of a slot: one rounding of u + t dt, bitwise."""
+    r = np.random.default_rng(3)
+    u, v, w, p, du, dv, dw, dp, dup, dvp = (r.standard_normal(shape).astype(F32) for _ in range(10))
+    out = [x.copy() for x in (u, v, w, p)]
+    d = L.SlowApplyDispatch(*[fp(x) for x in out], *[fp(x) for x in (du, dv, dw, dp, dup, dvp)], *shape, 6.0,
+                            L.FourFieldObserver(), None, 1)
+    call(hip_ctx, "nimbus_hip_dispatch_slow_apply", d)
+    f = np.float64
+    for got, x, t in zip(out, (u, v, w, p), (du.astype(f) + dup, dv.astype(f) + dvp, dw.astype(f), dp.astype(f))):
+        assert np.array_equal(got, (x.astype(f) + t * 6.0).astype(F32))
+
+
 def test_state_relaxation_follows_its_definition(hip_ctx, rng):
     nx, ny, nz = 12, 10, 9
     shape = (nx, ny, nz)
