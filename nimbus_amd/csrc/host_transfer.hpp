@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <condition_variable>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -29,13 +30,20 @@ struct ArrayCopy
     std::size_t bytes;
 };
 
-// A contiguous piece of one of the caller's arrays; direct: the kernel can
-// reach the array itself (device memory), nothing is copied.
+// How the device side of a transfer gets at one of the caller's arrays.
+enum class Reach
+{
+    Host,     // ordinary memory: std::memcpy to or from a slot
+    Runtime,  // memory of the runtime that a kernel here may not touch: hipMemcpy to or from a slot
+    Kernel    // a kernel on the context's device reads or writes the array itself
+};
+
+// A contiguous piece of one of the caller's arrays.
 struct HostChunk
 {
     char* host;
     std::size_t bytes;
-    bool direct;
+    Reach reach;
 };
 
 class HostTransfer
@@ -72,7 +80,7 @@ public:
     }
 
     // Moves the chunks to (up) or from the device; launch(c, p) enqueues the
-    // device side of chunk c on `stream` against p, its slot or (direct) its
+    // device side of chunk c on `stream` against p, its slot or (Reach::Kernel) its
     // array. Returns when the caller's arrays are read or written. Transfers of
     // one ring run one after the other.
     template <class Launch>
@@ -118,7 +126,7 @@ public:
                 if (up ? st.copied[c] : c < kSlots || st.copied[c - kSlots])
                 {
                     lock.unlock();
-                    hipError_t r = launch(c, chunks[c].direct ? chunks[c].host : slot(c));
+                    hipError_t r = launch(c, chunks[c].reach == Reach::Kernel ? chunks[c].host : slot(c));
                     if (r == hipSuccess) r = hipEventRecord(events_[c % kSlots], stream);
                     lock.lock();
                     if (r != hipSuccess) st.error = r;
@@ -163,10 +171,18 @@ public:
         std::vector<char*> dev;
         for (const ArrayCopy& a : arrays)
         {
-            const bool direct = a.bytes != 0 && device_array(a.host);
+            if (a.bytes == 0) continue;
+            // the runtime copies its own memory, whichever device's, without a slot
+            if (reach(device, a.host, a.bytes, 1) != Reach::Host)
+            {
+                const hipError_t e = hipMemcpyAsync(up ? a.dev : a.host, up ? a.host : a.dev, a.bytes,
+                                                    hipMemcpyDefault, stream);
+                if (e != hipSuccess) return e;
+                continue;
+            }
             for (std::size_t o = 0; o < a.bytes; o += kSlot)
             {
-                chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, std::min(kSlot, a.bytes - o), direct});
+                chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, std::min(kSlot, a.bytes - o), Reach::Host});
                 dev.push_back(static_cast<char*>(a.dev) + o);
             }
         }
@@ -175,13 +191,27 @@ public:
         });
     }
 
-    // Whether a kernel can reach the caller's array itself (it is device memory).
-    static bool device_array(const void* p)
+    // The reach of a caller's array of elements of `size` bytes from a kernel on
+    // `device`: the device's own memory, aligned and allocated over the whole array.
+    static Reach reach(int device, const void* p, std::size_t bytes, std::size_t size)
     {
         hipPointerAttribute_t at{};
-        const bool yes = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
+        const bool known = hipPointerGetAttributes(&at, p) == hipSuccess;
+        Reach r = Reach::Host;
+        if (known && (at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeUnified))
+        {
+            r = Reach::Runtime;
+            hipDeviceptr_t base = nullptr;
+            std::size_t n = 0;
+            if (at.type == hipMemoryTypeDevice && at.device == device && reinterpret_cast<std::uintptr_t>(p) % size == 0 &&
+                hipMemGetAddressRange(&base, &n, const_cast<void*>(p)) == hipSuccess)
+            {
+                const std::size_t o = std::size_t(static_cast<const char*>(p) - static_cast<const char*>(base));
+                if (o <= n && bytes <= n - o) r = Reach::Kernel;
+            }
+        }
         hipGetLastError();  // an ordinary host array is no error
-        return yes;
+        return r;
     }
 
 private:
@@ -207,10 +237,12 @@ private:
         hipError_t r = hipSuccess;
         if (!up || c >= kSlots) r = hipEventSynchronize(events_[c % kSlots]);
         const HostChunk& k = chunks[c];
-        if (r == hipSuccess && !k.direct)
+        if (r == hipSuccess && k.reach != Reach::Kernel)
         {
-            if (up) std::memcpy(slot(c), k.host, k.bytes);
-            else std::memcpy(k.host, slot(c), k.bytes);
+            void* const to = up ? slot(c) : k.host;
+            const void* const from = up ? k.host : slot(c);
+            if (k.reach == Reach::Runtime) r = hipMemcpy(to, from, k.bytes, hipMemcpyDefault);
+            else std::memcpy(to, from, k.bytes);
         }
         lock.lock();
         if (r != hipSuccess) st.error = r;

@@ -746,7 +746,7 @@ int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::ve
     for (std::size_t q = 0; q < fields.size(); ++q)
     {
         char* const host = static_cast<char*>(const_cast<void*>(fields[q].host));
-        const bool direct = HostTransfer::device_array(host);
+        const Reach reach = HostTransfer::reach(ctx->device, host, rows * g.nx * sizeof(H), sizeof(H));
         std::size_t ni = std::max<std::size_t>(1, slot / rows);
         if (ni >= 16) ni -= ni % 16;  // whole tiles of the kernel
         const std::size_t nr = std::min(rows, slot);
@@ -755,7 +755,7 @@ int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::ve
             {
                 const HostPart p{int(i), int(std::min(ni, g.nx - i)), int(r), int(std::min(nr, rows - r))};
                 chunks.push_back(HostChunk{host + (i * rows + r) * sizeof(H), std::size_t(p.ni) * p.nr * sizeof(H),
-                                           direct});
+                                           reach});
                 parts.push_back(p);
                 of.push_back(q);
             }

@@ -12,7 +12,7 @@
 
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 enum hipMemcpyKind { hipMemcpyHostToHost, hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipMemcpyDeviceToDevice, hipMemcpyDefault };
-enum hipMemoryType { hipMemoryTypeUnregistered, hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged };
+enum hipMemoryType { hipMemoryTypeUnregistered, hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged, hipMemoryTypeUnified };
 enum { hipEventDisableTiming = 2 };
 typedef struct fake_stream* hipStream_t;
 typedef struct fake_event* hipEvent_t;

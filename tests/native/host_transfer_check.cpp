@@ -74,6 +74,56 @@ int large()
     }
     return 0;
 }
+// A kernel on the context's device (0) touches only memory of that device, over
+// its whole allocation, aligned; what else the runtime knows it copies itself.
+int reach()
+{
+    std::vector<char> a(64 * KB);
+    char* const p = a.data();
+    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Host);
+    auto as = [&](hipMemoryType type, int device) { fake::ranges = {{p, fake::Range{64 * KB, type, device}}}; };
+    as(hipMemoryTypeDevice, 0);
+    CHECK(HostTransfer::reach(0, p, 64 * KB, 4) == Reach::Kernel);
+    CHECK(HostTransfer::reach(0, p + 4 * KB, 60 * KB, 8) == Reach::Kernel);
+    CHECK(HostTransfer::reach(0, p + 4 * KB, 60 * KB + 1, 4) == Reach::Runtime);
+    CHECK(HostTransfer::reach(0, p + 2, 4 * KB, 4) == Reach::Runtime);
+    CHECK(HostTransfer::reach(0, p + 4, 4 * KB, 8) == Reach::Runtime);
+    as(hipMemoryTypeDevice, 1);
+    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Runtime);
+    as(hipMemoryTypeManaged, 0);
+    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Runtime);
+    return 0;
+}
+
+// Another device's array goes through the slots with the runtime's copies, and
+// in a copy of whole arrays without them.
+int foreign()
+{
+    for (bool up : {true, false})
+    {
+        Arrays a(8, 7 * MB + 13);
+        fake::ranges = {{a.host[3].data(), fake::Range{a.host[3].size(), hipMemoryTypeDevice, 1}}};
+        {
+            HostTransfer t;
+            fake::reset();
+            CHECK(t.copy(0, nullptr, up, a.copies) == hipSuccess);
+            CHECK(a.equal());
+            CHECK(fake::events == 7 * 4 && fake::copies == 7 * 4 + 1 && fake::blocking_copies == 0);
+        }
+        HostTransfer t;
+        std::vector<char> from(3 * MB, 5), to(3 * MB, 6);
+        const std::vector<HostChunk> chunks{{(up ? from : to).data(), MB, Reach::Host},
+                                            {(up ? from : to).data() + MB, 2 * MB, Reach::Runtime}};
+        char* const dev = (up ? to : from).data();
+        fake::reset();
+        CHECK(t.run(0, nullptr, up, chunks, [&](int c, char* p) {
+            char* const d = dev + (c ? MB : 0);
+            return hipMemcpyAsync(up ? d : p, up ? p : d, chunks[c].bytes, hipMemcpyDefault, nullptr);
+        }) == hipSuccess);
+        CHECK(to == from && fake::blocking_copies == 1);
+    }
+    return 0;
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -81,6 +131,8 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "small") return small();
     if (what == "large") return large();
+    if (what == "reach") return reach();
+    if (what == "foreign") return foreign();
     std::printf("unknown check %s\n", what.c_str());
     return 2;
 }

@@ -763,3 +763,61 @@ def test_upload_then_download_returns_the_fields(hip_ctx, shape, precision):
         else:
             assert np.array_equal(out[f], st[f]), f
     assert np.array_equal(out["rain_mm"], rain)
+
+
+
+class RuntimeArray:
+    """`n` bytes from the HIP runtime that the library is bound to, `shift` into their allocation."""
+
+    def __init__(self, n, shift=0):
+        self.hip = ctypes.CDLL("libamdhip64.so.7")
+        self.hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+        self.hip.hipFree.argtypes = [ctypes.c_void_p]
+        self.hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+        self.base = ctypes.c_void_p()
+        assert self.hip.hipMalloc(ctypes.byref(self.base), n + shift) == 0
+        self.ptr = self.base.value + shift
+
+    def put(self, a):
+        assert self.hip.hipMemcpy(self.ptr, a.ctypes.data, a.nbytes, 4) == 0
+
+    def get(self, like):
+        a = np.empty_like(like)
+        assert self.hip.hipMemcpy(a.ctypes.data, self.ptr, a.nbytes, 4) == 0
+        return a
+
+    def free(self):
+        assert self.hip.hipFree(self.base) == 0
+
+
+@pytest.mark.parametrize("precision", [L.PRECISION_MIXED, L.PRECISION_FP64])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_state_in_device_arrays(hip_ctx, shift, precision):
+    """A member's state from and to device arrays, which the kernel reaches
+    itself, and ones at an address that is no multiple of the element size: as
+    with host arrays, bitwise."""
+    shape = (70, 190, 61)
+    g = L.make_grid(*shape, 1000.0, 1000.0, 20000.0 / shape[2])
+    m = hip_ctx.member(g, L.step_config(3.0, 6), L.base_state(g), precision)
+    dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
+    r = np.random.default_rng(6)
+    st = {f: r.random(shape, np.float32).astype(dtype) + dtype(0.25) for f in L.FIELDS}
+    arrays = {f: RuntimeArray(st[f].nbytes, shift) for f in L.FIELDS}
+    hs = L.HostState(**{f: a.ptr for f, a in arrays.items()})
+    try:
+        m.upload(dict(st, rain_mm=None))
+        ref = m.download()
+        m.upload(dict({f: np.zeros(shape, dtype) for f in L.FIELDS}, rain_mm=None))
+        for f, a in arrays.items():
+            a.put(st[f])
+        L.check(hip_ctx.lib.nimbus_hip_member_upload(hip_ctx.handle, m.id, ctypes.byref(hs)), "upload")
+        for a in arrays.values():
+            a.put(np.zeros(shape, dtype))
+        L.check(hip_ctx.lib.nimbus_hip_member_download(hip_ctx.handle, m.id, ctypes.byref(hs)), "download")
+        got = {f: a.get(st[f]) for f, a in arrays.items()}
+    finally:
+        for a in arrays.values():
+            a.free()
+        m.destroy()
+    for f in L.FIELDS:
+        assert np.array_equal(got[f], ref[f]), f
