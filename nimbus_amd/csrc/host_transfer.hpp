@@ -92,12 +92,17 @@ public:
         State st;
         st.n = int(chunks.size());
         st.copied.assign(chunks.size(), 0);
-        std::size_t bytes = 0;
-        for (const HostChunk& c : chunks) bytes += c.bytes;
+        std::size_t bytes = 0, copies = 0;
+        for (const HostChunk& c : chunks)
+            if (c.reach != Reach::Kernel)
+            {
+                bytes += c.bytes;
+                ++copies;
+            }
         // a thread for each 4 MB: one for each MB took 2,040 us where this takes 1,910 (a contract
         // call of 13 arrays of 96 x 96 x 60 floats) and 435 where this takes 408 (9 of 64 x 64 x 48
         // doubles), in starting them and in the release of device memory beside them
-        const int want = int(std::min<std::size_t>({std::size_t(kThreads), chunks.size(), bytes >> 22}));
+        const int want = int(std::min<std::size_t>({std::size_t(kThreads), copies, bytes >> 22}));
         std::vector<std::thread> team;
         team.reserve(kThreads);  // no allocation once a thread runs
         try

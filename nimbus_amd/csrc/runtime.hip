@@ -747,9 +747,11 @@ int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::ve
     {
         char* const host = static_cast<char*>(const_cast<void*>(fields[q].host));
         const Reach reach = HostTransfer::reach(ctx->device, host, rows * g.nx * sizeof(H), sizeof(H));
-        std::size_t ni = std::max<std::size_t>(1, slot / rows);
-        if (ni >= 16) ni -= ni % 16;  // whole tiles of the kernel
-        const std::size_t nr = std::min(rows, slot);
+        // no slot, no parts: the kernel takes the whole array
+        const bool whole = reach == Reach::Kernel;
+        std::size_t ni = whole ? std::size_t(g.nx) : std::max<std::size_t>(1, slot / rows);
+        if (!whole && ni >= 16) ni -= ni % 16;  // whole tiles of the kernel
+        const std::size_t nr = whole ? rows : std::min(rows, slot);
         for (std::size_t i = 0; i < std::size_t(g.nx); i += ni)
             for (std::size_t r = 0; r < rows; r += nr)
             {

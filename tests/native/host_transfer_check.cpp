@@ -124,6 +124,24 @@ int foreign()
     }
     return 0;
 }
+// Arrays that the kernel reaches itself need no copying thread.
+int no_threads()
+{
+    for (bool up : {true, false})
+    {
+        HostTransfer t;
+        std::vector<char> array(64 * MB, 1), dev(64 * MB, 2);
+        std::vector<HostChunk> chunks;
+        for (int c = 0; c < 4; ++c) chunks.push_back(HostChunk{array.data() + c * 16 * MB, 16 * MB, Reach::Kernel});
+        fake::reset();
+        CHECK(t.run(0, nullptr, up, chunks, [&](int c, char* p) {
+            char* const d = dev.data() + c * 16 * MB;
+            return hipMemcpyAsync(up ? d : p, up ? p : d, chunks[c].bytes, hipMemcpyDefault, nullptr);
+        }) == hipSuccess);
+        CHECK(array == dev && fake::copies == 4 && fake::threads_set == 0);
+    }
+    return 0;
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -131,6 +149,7 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "small") return small();
     if (what == "large") return large();
+    if (what == "no_threads") return no_threads();
     if (what == "reach") return reach();
     if (what == "foreign") return foreign();
     std::printf("unknown check %s\n", what.c_str());
