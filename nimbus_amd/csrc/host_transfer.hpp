@@ -87,8 +87,6 @@ public:
     hipError_t run(int device, hipStream_t stream, bool up, const std::vector<HostChunk>& chunks, Launch launch)
     {
         std::lock_guard<std::mutex> one(busy_);
-        hipError_t e = prepare();
-        if (e != hipSuccess) return e;
         State st;
         st.n = int(chunks.size());
         st.copied.assign(chunks.size(), 0);
@@ -99,6 +97,8 @@ public:
                 bytes += c.bytes;
                 ++copies;
             }
+        hipError_t e = prepare(copies != 0);
+        if (e != hipSuccess) return e;
         // a thread for each 4 MB: one for each MB took 2,040 us where this takes 1,910 (a contract
         // call of 13 arrays of 96 x 96 x 60 floats) and 435 where this takes 408 (9 of 64 x 64 x 48
         // doubles), in starting them and in the release of device memory beside them
@@ -153,70 +153,85 @@ public:
     // Copies whole arrays to (up) or from the device. Downloads are complete on
     // return; uploads precede what is enqueued on `stream` next, and the arrays
     // are read by the time that `stream` has run.
-    hipError_t copy(int device, hipStream_t stream, bool up, const std::vector<ArrayCopy>& arrays)
+    hipError_t copy(int device, hipStream_t stream, bool up, std::vector<ArrayCopy> arrays)
     {
-        std::size_t bytes = 0, count = 0;
-        for (const ArrayCopy& a : arrays)
-        {
-            bytes += a.bytes;
-            count += a.bytes != 0;
-        }
-        const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-        if (!takes_ring(up, bytes, count))
-        {
-            for (const ArrayCopy& a : arrays)
+        auto rings = [up](auto first, auto last) {
+            std::size_t bytes = 0, count = 0;
+            for (; first != last; ++first)
             {
-                if (a.bytes == 0) continue;
-                const hipError_t e = hipMemcpyAsync(up ? a.dev : a.host, up ? a.host : a.dev, a.bytes, kind, stream);
-                if (e != hipSuccess) return e;
+                bytes += first->bytes;
+                count += first->bytes != 0;
             }
-            return up ? hipSuccess : hipStreamSynchronize(stream);
+            return takes_ring(up, bytes, count);
+        };
+        // first what is copied plainly: everything below the ring's sizes, and memory
+        // of the runtime, pinned or any device's, which its copies move without a slot
+        auto staged = arrays.end();
+        if (rings(arrays.begin(), arrays.end()))
+        {
+            staged = std::stable_partition(arrays.begin(), arrays.end(), [&](const ArrayCopy& a) {
+                return a.bytes == 0 || of_runtime(a.host);
+            });
+            if (!rings(staged, arrays.end())) staged = arrays.end();
         }
+        for (auto a = arrays.begin(); a != staged; ++a)
+        {
+            if (a->bytes == 0) continue;
+            const hipError_t e = hipMemcpyAsync(up ? a->dev : a->host, up ? a->host : a->dev, a->bytes,
+                                                hipMemcpyDefault, stream);
+            if (e != hipSuccess) return e;
+        }
+        if (staged == arrays.end()) return up ? hipSuccess : hipStreamSynchronize(stream);
         std::vector<HostChunk> chunks;
         std::vector<char*> dev;
-        for (const ArrayCopy& a : arrays)
-        {
-            if (a.bytes == 0) continue;
-            // the runtime copies its own memory, whichever device's, without a slot
-            if (reach(device, a.host, a.bytes, 1) != Reach::Host)
+        for (auto a = staged; a != arrays.end(); ++a)
+            for (std::size_t o = 0; o < a->bytes; o += kSlot)
             {
-                const hipError_t e = hipMemcpyAsync(up ? a.dev : a.host, up ? a.host : a.dev, a.bytes,
-                                                    hipMemcpyDefault, stream);
-                if (e != hipSuccess) return e;
-                continue;
+                chunks.push_back(HostChunk{static_cast<char*>(a->host) + o, std::min(kSlot, a->bytes - o), Reach::Host});
+                dev.push_back(static_cast<char*>(a->dev) + o);
             }
-            for (std::size_t o = 0; o < a.bytes; o += kSlot)
-            {
-                chunks.push_back(HostChunk{static_cast<char*>(a.host) + o, std::min(kSlot, a.bytes - o), Reach::Host});
-                dev.push_back(static_cast<char*>(a.dev) + o);
-            }
-        }
         return run(device, stream, up, chunks, [&](int c, char* p) {
             return hipMemcpyAsync(up ? dev[c] : p, up ? p : dev[c], chunks[c].bytes, hipMemcpyDefault, stream);
         });
     }
 
-    // The reach of a caller's array of elements of `size` bytes from a kernel on
-    // `device`: the device's own memory, aligned and allocated over the whole array.
-    static Reach reach(int device, const void* p, std::size_t bytes, std::size_t size)
+    // How a kernel on `device` reaches a caller's array of elements of `size`
+    // bytes, and at which address: memory of its own device and host memory
+    // pinned for it, aligned and allocated over the whole array.
+    struct Place
+    {
+        Reach reach;
+        char* at;
+    };
+    static Place place(int device, const void* p, std::size_t bytes, std::size_t size)
     {
         hipPointerAttribute_t at{};
-        const bool known = hipPointerGetAttributes(&at, p) == hipSuccess;
-        Reach r = Reach::Host;
-        if (known && (at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeUnified))
+        Place r{Reach::Host, static_cast<char*>(const_cast<void*>(p))};
+        if (!of_runtime(p, &at)) return r;
+        if (at.type != hipMemoryTypeHost) r.reach = Reach::Runtime;
+        char* const q = static_cast<char*>(at.type == hipMemoryTypeHost ? at.devicePointer : r.at);
+        if (!q || (at.type != hipMemoryTypeHost && at.type != hipMemoryTypeDevice) || at.device != device ||
+            reinterpret_cast<std::uintptr_t>(q) % size != 0)
+            return r;
+        hipDeviceptr_t base = nullptr;
+        std::size_t n = 0;
+        if (hipMemGetAddressRange(&base, &n, q) == hipSuccess)
         {
-            r = Reach::Runtime;
-            hipDeviceptr_t base = nullptr;
-            std::size_t n = 0;
-            if (at.type == hipMemoryTypeDevice && at.device == device && reinterpret_cast<std::uintptr_t>(p) % size == 0 &&
-                hipMemGetAddressRange(&base, &n, const_cast<void*>(p)) == hipSuccess)
-            {
-                const std::size_t o = std::size_t(static_cast<const char*>(p) - static_cast<const char*>(base));
-                if (o <= n && bytes <= n - o) r = Reach::Kernel;
-            }
+            const std::size_t o = std::size_t(q - static_cast<char*>(base));
+            if (o <= n && bytes <= n - o) return Place{Reach::Kernel, q};
         }
-        hipGetLastError();  // an ordinary host array is no error
+        hipGetLastError();
         return r;
+    }
+
+    // Whether the runtime knows an array's memory (pinned, or any device's).
+    static bool of_runtime(const void* p, hipPointerAttribute_t* at = nullptr)
+    {
+        hipPointerAttribute_t own{};
+        if (!at) at = &own;
+        const bool known = hipPointerGetAttributes(at, p) == hipSuccess && at->type != hipMemoryTypeUnregistered;
+        hipGetLastError();  // an ordinary host array is no error
+        return known;
     }
 
 private:
@@ -255,7 +270,7 @@ private:
         st.cv.notify_all();
     }
 
-    hipError_t prepare()
+    hipError_t prepare(bool slots)
     {
         while (int(events_.size()) < kSlots)
         {
@@ -264,7 +279,7 @@ private:
             if (e != hipSuccess) return e;
             events_.push_back(ev);
         }
-        if (slots_) return hipSuccess;
+        if (slots_ || !slots) return hipSuccess;
         const hipError_t e = hipHostMalloc(&slots_, kSlot * kSlots, 0);
         if (e != hipSuccess) slots_ = nullptr;
         return e;

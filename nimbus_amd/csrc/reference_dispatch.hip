@@ -34,10 +34,11 @@ constexpr int kThreads = 256;
     } while (0)
 
 // Device copies of the call's arrays, released when the call returns. take()
-// names them, upload() fills those that have a host array. Where these (at
-// most `floats` together) don't take the transfer ring, take() copies at once:
-// the copies run beside the allocations that follow, which is 8 % of a call of
-// 19 arrays of 64 x 64 x 48 cells.
+// names them, upload() fills those that have a host array. Arrays that don't
+// take the transfer ring (all where they are at most `floats` together, memory
+// of the runtime at any size) are copied by take() at once: the copies run
+// beside the allocations that follow, which is 8 % of a call of 19 arrays of
+// 64 x 64 x 48 cells.
 struct DeviceArrays
 {
     const bool at_once;
@@ -56,10 +57,10 @@ struct DeviceArrays
         if (e != hipSuccess) return set_error(NIMBUS_ENOMEM, std::string("dispatch staging: ") + hipGetErrorString(e));
         ptrs.push_back(p);
         const std::size_t bytes = n * sizeof(float);
-        if (host && !at_once) in.push_back(ArrayCopy{p, const_cast<float*>(host), bytes});
+        if (host && !at_once && !HostTransfer::of_runtime(host)) in.push_back(ArrayCopy{p, const_cast<float*>(host), bytes});
         else
         {
-            const hipError_t c = host ? hipMemcpyAsync(p, host, bytes, hipMemcpyHostToDevice, s)
+            const hipError_t c = host ? hipMemcpyAsync(p, host, bytes, hipMemcpyDefault, s)
                                       : hipMemsetAsync(p, 0, bytes, s);
             if (c != hipSuccess) return set_error(NIMBUS_EHIP, std::string("dispatch staging: ") + hipGetErrorString(c));
         }

@@ -745,8 +745,8 @@ int transfer_fields(nimbus_hip_ctx* ctx, const Member& m, bool up, const std::ve
     std::vector<std::size_t> of;
     for (std::size_t q = 0; q < fields.size(); ++q)
     {
-        char* const host = static_cast<char*>(const_cast<void*>(fields[q].host));
-        const Reach reach = HostTransfer::reach(ctx->device, host, rows * g.nx * sizeof(H), sizeof(H));
+        const auto [reach, host] =
+            HostTransfer::place(ctx->device, fields[q].host, rows * g.nx * sizeof(H), sizeof(H));
         // no slot, no parts: the kernel takes the whole array
         const bool whole = reach == Reach::Kernel;
         std::size_t ni = whole ? std::size_t(g.nx) : std::max<std::size_t>(1, slot / rows);

@@ -37,6 +37,7 @@ struct Range
 inline std::map<char*, Range> ranges;  // what the runtime knows of; set up before a transfer starts
 inline std::atomic<int> copies, blocking_copies, events, pinned, threads_set, queries;
 inline bool no_pinned = false;
+inline std::ptrdiff_t mapped = 0;  // distance of an array's address on the device
 
 inline void reset() { copies = blocking_copies = events = pinned = threads_set = queries = 0; }
 inline const Range* range_of(const void* p, char** base = nullptr)
@@ -83,15 +84,16 @@ inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* at, const void*
     ++fake::queries;
     const fake::Range* r = fake::range_of(p);
     if (!r) return hipErrorInvalidValue;
-    *at = hipPointerAttribute_t{r->type, r->device, const_cast<void*>(p), r->type == hipMemoryTypeDevice ? nullptr : const_cast<void*>(p)};
+    char* const c = static_cast<char*>(const_cast<void*>(p));
+    *at = hipPointerAttribute_t{r->type, r->device, c + fake::mapped, r->type == hipMemoryTypeDevice ? nullptr : c};
     return hipSuccess;
 }
 inline hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, std::size_t* n, hipDeviceptr_t p)
 {
     char* b = nullptr;
-    const fake::Range* r = fake::range_of(p, &b);
+    const fake::Range* r = fake::range_of(static_cast<char*>(p) - fake::mapped, &b);
     if (!r) return hipErrorInvalidValue;
-    *base = b;
+    *base = b + fake::mapped;
     *n = r->bytes;
     return hipSuccess;
 }

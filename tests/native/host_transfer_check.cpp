@@ -74,24 +74,54 @@ int large()
     }
     return 0;
 }
-// A kernel on the context's device (0) touches only memory of that device, over
-// its whole allocation, aligned; what else the runtime knows it copies itself.
+// A kernel on the context's device (0) touches only memory of that device and
+// host memory pinned for it, over its whole allocation, aligned; what else the
+// runtime knows it copies itself, but for pinned memory, which the host can.
 int reach()
 {
     std::vector<char> a(64 * KB);
     char* const p = a.data();
-    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Host);
-    auto as = [&](hipMemoryType type, int device) { fake::ranges = {{p, fake::Range{64 * KB, type, device}}}; };
-    as(hipMemoryTypeDevice, 0);
-    CHECK(HostTransfer::reach(0, p, 64 * KB, 4) == Reach::Kernel);
-    CHECK(HostTransfer::reach(0, p + 4 * KB, 60 * KB, 8) == Reach::Kernel);
-    CHECK(HostTransfer::reach(0, p + 4 * KB, 60 * KB + 1, 4) == Reach::Runtime);
-    CHECK(HostTransfer::reach(0, p + 2, 4 * KB, 4) == Reach::Runtime);
-    CHECK(HostTransfer::reach(0, p + 4, 4 * KB, 8) == Reach::Runtime);
-    as(hipMemoryTypeDevice, 1);
-    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Runtime);
-    as(hipMemoryTypeManaged, 0);
-    CHECK(HostTransfer::reach(0, p, 4 * KB, 4) == Reach::Runtime);
+    auto how = [&](std::size_t shift, std::size_t bytes, std::size_t size) {
+        return HostTransfer::place(0, p + shift, bytes, size).reach;
+    };
+    CHECK(how(0, 4 * KB, 4) == Reach::Host && !HostTransfer::of_runtime(p));
+    for (hipMemoryType type : {hipMemoryTypeDevice, hipMemoryTypeHost, hipMemoryTypeManaged})
+        for (int device : {0, 1})
+        {
+            fake::ranges = {{p, fake::Range{64 * KB, type, device}}};
+            const Reach other = type == hipMemoryTypeHost ? Reach::Host : Reach::Runtime;
+            const Reach own = device == 0 && type != hipMemoryTypeManaged ? Reach::Kernel : other;
+            CHECK(HostTransfer::of_runtime(p));
+            CHECK(how(0, 64 * KB, 4) == own);
+            CHECK(how(4 * KB, 60 * KB, 8) == own);
+            CHECK(how(4 * KB, 60 * KB + 1, 4) == other);
+            CHECK(how(2, 4 * KB, 4) == other);
+            CHECK(how(4, 4 * KB, 8) == other);
+        }
+    // pinned memory has an address of its own on the device
+    fake::ranges = {{p, fake::Range{64 * KB, hipMemoryTypeHost, 0}}};
+    fake::mapped = 1 << 20;
+    const bool at = HostTransfer::place(0, p + 8, 4 * KB, 8).at == p + 8 + fake::mapped;
+    const bool on_host = HostTransfer::place(0, p + 4, 4 * KB, 8).at == p + 4;
+    fake::mapped = 0;
+    CHECK(at && on_host);
+    return 0;
+}
+
+// Whole arrays in pinned memory take plain copies at any size: no ring, no threads.
+int pinned()
+{
+    for (bool up : {true, false})
+    {
+        HostTransfer t;
+        Arrays a(8, 7 * MB + 13);
+        fake::ranges.clear();
+        for (auto& h : a.host) fake::ranges[h.data()] = fake::Range{h.size(), hipMemoryTypeHost, 0};
+        fake::reset();
+        CHECK(t.copy(0, nullptr, up, a.copies) == hipSuccess);
+        CHECK(a.equal());
+        CHECK(fake::copies == 8 && fake::pinned == 0 && fake::events == 0 && fake::threads_set == 0);
+    }
     return 0;
 }
 
@@ -138,7 +168,7 @@ int no_threads()
             char* const d = dev.data() + c * 16 * MB;
             return hipMemcpyAsync(up ? d : p, up ? p : d, chunks[c].bytes, hipMemcpyDefault, nullptr);
         }) == hipSuccess);
-        CHECK(array == dev && fake::copies == 4 && fake::threads_set == 0);
+        CHECK(array == dev && fake::copies == 4 && fake::threads_set == 0 && fake::pinned == 0);
     }
     return 0;
 }
@@ -150,6 +180,7 @@ int main(int argc, char** argv)
     if (what == "small") return small();
     if (what == "large") return large();
     if (what == "no_threads") return no_threads();
+    if (what == "pinned") return pinned();
     if (what == "reach") return reach();
     if (what == "foreign") return foreign();
     std::printf("unknown check %s\n", what.c_str());

@@ -767,15 +767,21 @@ def test_upload_then_download_returns_the_fields(hip_ctx, shape, precision):
 
 
 class RuntimeArray:
-    """`n` bytes from the HIP runtime that the library is bound to, `shift` into their allocation."""
+    """`n` bytes from the HIP runtime that the library is bound to, `shift` into their allocation: on the
+    device, or pinned on the host."""
 
-    def __init__(self, n, shift=0):
+    def __init__(self, n, shift=0, pinned=False):
         self.hip = ctypes.CDLL("libamdhip64.so.7")
         self.hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
         self.hip.hipFree.argtypes = [ctypes.c_void_p]
         self.hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+        self.hip.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+        self.hip.hipHostFree.argtypes = [ctypes.c_void_p]
         self.base = ctypes.c_void_p()
-        assert self.hip.hipMalloc(ctypes.byref(self.base), n + shift) == 0
+        self.release = self.hip.hipHostFree if pinned else self.hip.hipFree
+        rc = (self.hip.hipHostMalloc(ctypes.byref(self.base), n + shift, 0) if pinned else
+              self.hip.hipMalloc(ctypes.byref(self.base), n + shift))
+        assert rc == 0
         self.ptr = self.base.value + shift
 
     def put(self, a):
@@ -787,22 +793,23 @@ class RuntimeArray:
         return a
 
     def free(self):
-        assert self.hip.hipFree(self.base) == 0
+        assert self.release(self.base) == 0
 
 
 @pytest.mark.parametrize("precision", [L.PRECISION_MIXED, L.PRECISION_FP64])
+@pytest.mark.parametrize("pinned", [False, True])
 @pytest.mark.parametrize("shift", [0, 2])
-def test_state_in_device_arrays(hip_ctx, shift, precision):
-    """A member's state from and to device arrays, which the kernel reaches
-    itself, and ones at an address that is no multiple of the element size: as
-    with host arrays, bitwise."""
+def test_state_in_memory_of_the_runtime(hip_ctx, shift, pinned, precision):
+    """A member's state from and to device arrays and pinned ones, which the
+    kernel reaches itself, and ones at an address that is no multiple of the
+    element size: as with ordinary host arrays, bitwise."""
     shape = (70, 190, 61)
     g = L.make_grid(*shape, 1000.0, 1000.0, 20000.0 / shape[2])
     m = hip_ctx.member(g, L.step_config(3.0, 6), L.base_state(g), precision)
     dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
     r = np.random.default_rng(6)
     st = {f: r.random(shape, np.float32).astype(dtype) + dtype(0.25) for f in L.FIELDS}
-    arrays = {f: RuntimeArray(st[f].nbytes, shift) for f in L.FIELDS}
+    arrays = {f: RuntimeArray(st[f].nbytes, shift, pinned) for f in L.FIELDS}
     hs = L.HostState(**{f: a.ptr for f, a in arrays.items()})
     try:
         m.upload(dict(st, rain_mm=None))
