@@ -14,8 +14,8 @@
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -119,9 +119,9 @@ public:
                     }
                 });
         }
-        catch (const std::system_error&)
+        catch (const std::exception&)
         {
-            // the threads that did start, and this one, do the work
+            // no thread, or no memory for its state: those that did start, and this one, do the work
         }
         {
             std::unique_lock<std::mutex> lock(st.m);

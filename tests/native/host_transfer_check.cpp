@@ -3,7 +3,27 @@
 #include "host_transfer.hpp"
 
 #include <cstdio>
+#include <new>
 #include <string>
+
+// Allocations fail from the `fail_in`-th of the thread that sets it on.
+namespace
+{
+thread_local int fail_in = 0;
+}
+
+void* operator new(std::size_t n)
+{
+    if (fail_in > 0 && --fail_in == 0)
+    {
+        fail_in = 1;
+        throw std::bad_alloc();
+    }
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
 
 using namespace nimbus;
 
@@ -154,6 +174,40 @@ int foreign()
     }
     return 0;
 }
+// Memory that runs out while the team starts: the threads that did start, and
+// the caller, move the arrays.
+int no_memory()
+{
+    for (bool up : {true, false})
+        for (int n = 1; n < 12; ++n)
+        {
+            HostTransfer t;
+            std::vector<char> array(32 * MB, 1), dev(32 * MB, 2);
+            std::vector<HostChunk> chunks;
+            for (int c = 0; c < 16; ++c) chunks.push_back(HostChunk{array.data() + c * 2 * MB, 2 * MB, Reach::Host});
+            auto launch = [&](int c, char* p) {
+                char* const d = dev.data() + c * 2 * MB;
+                return hipMemcpyAsync(up ? d : p, up ? p : d, chunks[c].bytes, hipMemcpyDefault, nullptr);
+            };
+            CHECK(t.run(0, nullptr, up, chunks, launch) == hipSuccess);  // makes the ring
+            for (auto& b : up ? dev : array) b = 3;
+            fake::reset();
+            bool moved = true;
+            fail_in = n;
+            try
+            {
+                moved = t.run(0, nullptr, up, chunks, launch) == hipSuccess;
+            }
+            catch (const std::bad_alloc&)
+            {
+                moved = false;  // before any thread ran
+            }
+            fail_in = 0;
+            CHECK(moved ? array == dev : fake::threads_set == 0 && fake::copies == 0);
+        }
+    return 0;
+}
+
 // Arrays that the kernel reaches itself need no copying thread.
 int no_threads()
 {
@@ -180,6 +234,7 @@ int main(int argc, char** argv)
     if (what == "small") return small();
     if (what == "large") return large();
     if (what == "no_threads") return no_threads();
+    if (what == "no_memory") return no_memory();
     if (what == "pinned") return pinned();
     if (what == "reach") return reach();
     if (what == "foreign") return foreign();
