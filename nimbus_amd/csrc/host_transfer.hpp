@@ -17,6 +17,7 @@
 #include <exception>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace nimbus
@@ -102,7 +103,7 @@ public:
         // a thread for each 4 MB: one for each MB took 2,040 us where this takes 1,910 (a contract
         // call of 13 arrays of 96 x 96 x 60 floats) and 435 where this takes 408 (9 of 64 x 64 x 48
         // doubles), in starting them and in the release of device memory beside them
-        const int want = int(std::min<std::size_t>({std::size_t(kThreads), copies, bytes >> 22}));
+        const int want = !up && shared(chunks) ? 1 : int(std::min<std::size_t>({std::size_t(kThreads), copies, bytes >> 22}));
         std::vector<std::thread> team;
         team.reserve(kThreads);  // no allocation once a thread runs
         try
@@ -246,6 +247,19 @@ private:
         // chunk `next` has its data in the slot (down), or the slot's last user is enqueued (up)
         bool can_copy(bool up) const { return up ? next < issued + kSlots : next < issued; }
     };
+
+    // Whether two of the caller's arrays share memory: downloads to them go in order.
+    static bool shared(const std::vector<HostChunk>& chunks)
+    {
+        std::vector<std::pair<char*, char*>> arrays;
+        for (const HostChunk& c : chunks)
+            if (!arrays.empty() && arrays.back().second == c.host) arrays.back().second += c.bytes;
+            else arrays.emplace_back(c.host, c.host + c.bytes);
+        std::sort(arrays.begin(), arrays.end());
+        for (std::size_t q = 1; q < arrays.size(); ++q)
+            if (arrays[q].first < arrays[q - 1].second) return true;
+        return false;
+    }
 
     char* slot(int c) const { return static_cast<char*>(slots_) + std::size_t(c % kSlots) * kSlot; }
 

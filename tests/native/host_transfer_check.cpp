@@ -174,6 +174,27 @@ int foreign()
     }
     return 0;
 }
+// Arrays that share memory hold what the last of them is given, as plain copies
+// in order leave it.
+int shared()
+{
+    for (std::size_t shift : {std::size_t(0), MB})
+        for (int repeat = 0; repeat < 20; ++repeat)
+        {
+            HostTransfer t;
+            Arrays a(16, 2 * MB);
+            std::vector<char> sink(2 * MB + 15 * shift, 1), expect(sink);
+            for (int q = 0; q < 16; ++q)
+            {
+                a.copies[q].host = sink.data() + q * shift;
+                std::memcpy(expect.data() + q * shift, a.dev[q].data(), 2 * MB);
+            }
+            CHECK(t.copy(0, nullptr, false, a.copies) == hipSuccess);
+            CHECK(sink == expect);
+        }
+    return 0;
+}
+
 // Memory that runs out while the team starts: the threads that did start, and
 // the caller, move the arrays.
 int no_memory()
@@ -235,6 +256,7 @@ int main(int argc, char** argv)
     if (what == "large") return large();
     if (what == "no_threads") return no_threads();
     if (what == "no_memory") return no_memory();
+    if (what == "shared") return shared();
     if (what == "pinned") return pinned();
     if (what == "reach") return reach();
     if (what == "foreign") return foreign();

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["small", "large", "reach", "foreign", "no_threads", "pinned", "no_memory"])
+@pytest.mark.parametrize("check", ["small", "large", "reach", "foreign", "no_threads", "pinned", "no_memory", "shared"])
 def test_host_transfer(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
