@@ -294,7 +294,9 @@ private:
             events_.push_back(ev);
         }
         if (slots_ || !slots) return hipSuccess;
-        const hipError_t e = hipHostMalloc(&slots_, kSlot * kSlots, 0);
+        // coherent, whatever HIP_HOST_COHERENT says: a slot is read once its event has passed,
+        // which makes no other memory visible to the host
+        const hipError_t e = hipHostMalloc(&slots_, kSlot * kSlots, hipHostMallocCoherent);
         if (e != hipSuccess) slots_ = nullptr;
         return e;
     }

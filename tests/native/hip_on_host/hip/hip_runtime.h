@@ -13,7 +13,7 @@
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 enum hipMemcpyKind { hipMemcpyHostToHost, hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipMemcpyDeviceToDevice, hipMemcpyDefault };
 enum hipMemoryType { hipMemoryTypeUnregistered, hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged, hipMemoryTypeUnified };
-enum { hipEventDisableTiming = 2 };
+enum { hipEventDisableTiming = 2, hipHostMallocCoherent = 0x40000000 };
 typedef struct fake_stream* hipStream_t;
 typedef struct fake_event* hipEvent_t;
 typedef void* hipDeviceptr_t;
@@ -37,6 +37,7 @@ struct Range
 inline std::map<char*, Range> ranges;  // what the runtime knows of; set up before a transfer starts
 inline std::atomic<int> copies, blocking_copies, events, pinned, threads_set, queries;
 inline bool no_pinned = false;
+inline unsigned pinned_flags = 0;
 inline std::ptrdiff_t mapped = 0;  // distance of an array's address on the device
 
 inline void reset() { copies = blocking_copies = events = pinned = threads_set = queries = 0; }
@@ -54,8 +55,9 @@ inline const Range* range_of(const void* p, char** base = nullptr)
 
 inline hipError_t hipSetDevice(int) { ++fake::threads_set; return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
-inline hipError_t hipHostMalloc(void** p, std::size_t n, unsigned)
+inline hipError_t hipHostMalloc(void** p, std::size_t n, unsigned flags)
 {
+    fake::pinned_flags = flags;
     if (fake::no_pinned) return hipErrorOutOfMemory;
     ++fake::pinned;
     *p = std::malloc(n);

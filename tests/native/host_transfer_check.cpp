@@ -91,6 +91,7 @@ int large()
         CHECK(t.copy(0, nullptr, up, a.copies) == hipSuccess);
         CHECK(a.equal());
         CHECK(fake::pinned == 1 && fake::events == 8 * 4);
+        CHECK(fake::pinned_flags & hipHostMallocCoherent);
     }
     return 0;
 }
