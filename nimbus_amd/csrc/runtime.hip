@@ -67,7 +67,7 @@ std::size_t align256(std::size_t x) { return (x + 255) / 256 * 256; }
 
 struct Layout
 {
-    std::size_t field, rl, tri, rad_w, rad_s, rain, base, diag, lat, clock, total;
+    std::size_t field, rl, rad_w, rad_s, rain, base, diag, lat, clock, total;
 };
 
 // Lateral sponge band width in cells (0 when the sponge or its band is off).
@@ -77,14 +77,11 @@ int lateral_cells(const nimbus_step_config& c, const nimbus_grid& g)
     return std::max(0, std::min(c.sponge_lateral_cells, std::max(g.nx, g.ny)));
 }
 
-Layout layout_for(const DevGrid& g, int elem, bool hevi, int lateral = 0)
+Layout layout_for(const DevGrid& g, int elem, int lateral = 0)
 {
     Layout L{};
     L.field = align256(g.cells() * std::size_t(elem));
     L.rl = align256(g.cells() * sizeof(float));
-    // two FP64 arrays that a member whose form may be SEQUENTIAL holds: part of
-    // its published size, which admission counts on; no kernel uses them
-    L.tri = hevi && !hevi_partitioned_always(elem, g.nz) ? align256(g.cells() * sizeof(double)) : 0;
     L.rad_w = align256(std::size_t(g.ny) * g.nz * sizeof(float));
     L.rad_s = align256(std::size_t(g.nx) * g.nz * sizeof(float));
     L.rain = align256(std::size_t(g.nx) * g.ny * sizeof(double));
@@ -92,7 +89,7 @@ Layout layout_for(const DevGrid& g, int elem, bool hevi, int lateral = 0)
     L.diag = align256(std::size_t(kDiagBlocksPerMember + 1) * kDiagValues * sizeof(double));
     L.lat = align256(std::size_t(std::max(lateral, 1)) * sizeof(double));
     L.clock = align256(4 * sizeof(double));
-    L.total = L.field * F_COUNT + 3 * L.rl + 2 * L.tri + 2 * L.rad_w + 2 * L.rad_s + L.rain + L.base + L.diag +
+    L.total = L.field * F_COUNT + 3 * L.rl + 2 * L.rad_w + 2 * L.rad_s + L.rain + L.base + L.diag +
               L.lat + L.clock;
     return L;
 }
@@ -390,7 +387,7 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
             lat[d] = factor(c.sponge_lateral_alpha * sn * sn);
         }
     }
-    const Layout L = layout_for(m.args.g, m.elem, hevi, W);
+    const Layout L = layout_for(m.args.g, m.elem, W);
     m.bytes = L.total;
     hipError_t e = hipMalloc(&m.block, L.total);
     if (e != hipSuccess)
@@ -418,7 +415,6 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
     f.rl_qv = reinterpret_cast<float*>(p); p += L.rl;
     f.rl_qc = reinterpret_cast<float*>(p); p += L.rl;
     f.rl_qr = reinterpret_cast<float*>(p); p += L.rl;
-    p += 2 * L.tri;
     f.rad_w = reinterpret_cast<float*>(p); p += L.rad_w;
     f.rad_e = reinterpret_cast<float*>(p); p += L.rad_w;
     f.rad_s = reinterpret_cast<float*>(p); p += L.rad_s;
@@ -954,9 +950,7 @@ uint64_t nimbus_hip_member_bytes(const nimbus_member_desc* desc)
 {
     if (!desc || !valid_grid(desc->grid)) return 0;
     const int elem = desc->precision == NIMBUS_PRECISION_MIXED ? 4 : 8;
-    return layout_for(dev_grid(desc->grid, elem), elem, desc->config.acoustic_mode == NIMBUS_ACOUSTIC_HEVI,
-                      lateral_cells(desc->config, desc->grid))
-        .total;
+    return layout_for(dev_grid(desc->grid, elem), elem, lateral_cells(desc->config, desc->grid)).total;
 }
 
 int nimbus_hip_member_create(nimbus_hip_ctx* ctx, const nimbus_member_desc* desc, uint32_t* id)
@@ -1181,8 +1175,7 @@ struct SnapSizes
 
 SnapSizes snap_sizes(const Member& m)
 {
-    const bool hevi = m.desc.config.acoustic_mode == NIMBUS_ACOUSTIC_HEVI;
-    const Layout L = layout_for(m.args.g, m.elem, hevi, lateral_cells(m.desc.config, m.desc.grid));
+    const Layout L = layout_for(m.args.g, m.elem, lateral_cells(m.desc.config, m.desc.grid));
     SnapSizes z{};
     z.field = L.field;
     z.rain = std::size_t(m.g().nx) * m.g().ny * sizeof(double);
