@@ -535,7 +535,8 @@ def main():
                     help="cap on the cells resident at once in the serving run besides the 200 GB HBM budget "
                          "(0: no cap)")
     ap.add_argument("--column-solve", choices=["auto", "sequential", "partitioned"], default="sequential",
-                    help="HE-VI column-solve form of the ensemble and serving members (FP32 storage)")
+                    help="HE-VI column-solve form that the ensemble and serving members (FP32 storage) report; "
+                         "either is solved by the same kernel")
     ap.add_argument("--no-tuning", action="store_true",
                     help="ensemble and serving members keep the default launch geometry (no autotuning)")
     ap.add_argument("--accuracy", default="c2,c1",
@@ -548,7 +549,7 @@ def main():
     ap.add_argument("--profile-diffusion", action="store_true",
                     help="with --profile: the explicit diffusion of u, v, w, theta, qv on (K_h 50, K_v 10 m^2/s)")
     ap.add_argument("--profile-column-solve", choices=["auto", "sequential", "partitioned"], default="auto",
-                    help="HE-VI column-solve form of the --profile member (auto: the member's default)")
+                    help="HE-VI column-solve form that the --profile member reports (auto: the member's default)")
     ap.add_argument("--no-next-rows", action="store_true",
                     help="skip the diffusion, state I/O and sounding I/O timings")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",

@@ -351,14 +351,13 @@ int nimbus_hip_synchronize(nimbus_hip_ctx* ctx);
  * row-major plane, the wide-stencil passes (slow tendencies, WENO5 fluxes and update) in 64 x 4
  * tiles with k_chunks. */
 int nimbus_hip_member_set_tiling(nimbus_hip_ctx* ctx, uint32_t id, int tile_w, int k_chunks, int xcd_remap);
-/* HE-VI column-solve form of a member. It is fixed per member (never chosen
- * by the batch), so a member's results are the same alone and in any batch.
- * AUTO: partitioned for FP64 members of at most 129 levels and for FP32
+/* HE-VI column-solve form of a member, a name that is kept with it and in its
+ * snapshots. AUTO: partitioned for FP64 members of at most 129 levels and for FP32
  * members of fewer than 32768 columns and at most 129 levels, sequential
  * otherwise. PARTITIONED is refused above 129 levels, SEQUENTIAL for FP64
  * members of at most 129 levels. Both forms are solved by the same kernel with
  * the same operations (whole columns in LDS, eliminated from both ends), so
- * the choice changes neither results nor time. No reference counterpart: the
+ * the choice changes neither results nor time, nor any cached batch. No reference counterpart: the
  * reference has no vertically implicit solve. */
 enum
 {

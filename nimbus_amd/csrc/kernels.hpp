@@ -62,7 +62,6 @@ struct StepParams
     double mf_weight;   // retained mass-flux weight per substep (dts / dt in the large step)
     int substeps;
     int acoustic_mode;
-    int hevi_seg;       // the member's column-solve form reads PARTITIONED (fixed per member)
     double hevi_alpha;  // (1 + beta) / 2
     double coriolis_f;
     int bc_west, bc_east, bc_south, bc_north, bc_bottom, bc_top;
@@ -140,11 +139,11 @@ enum WorkKind
     W_KINDS = 6
 };
 
-// Column-solve form of a member (nimbus_hip_member_set_column_solve), fixed at
-// creation: PARTITIONED for FP64 members and for FP32 members of fewer than
+// Column-solve form of a member (nimbus_hip_member_set_column_solve), at its
+// creation PARTITIONED for FP64 members and for FP32 members of fewer than
 // kSweepColumns columns, both up to kSegMaxNz levels. A name that is accepted,
-// refused and reported; k_hevi_solve solves the columns of either form with
-// the same operations.
+// refused, reported and kept in snapshots; k_hevi_solve solves the columns of
+// either form with the same operations.
 constexpr int kSegMaxNz = 129;
 constexpr int kSweepColumns = 32768;
 constexpr bool hevi_partitioned_always(int elem, int nz) { return elem == 8 && nz <= kSegMaxNz; }

@@ -161,6 +161,7 @@ struct Member
     std::size_t bytes = 0;
     std::int64_t steps = 0;
     int tile_w = 64, k_chunks = 1, xcd_remap = 1;
+    int hevi_seg = 0;  // the member's column-solve form reads PARTITIONED
     const DevGrid& g() const { return args.g; }
     const DevFields& f() const { return args.f; }
 };
@@ -287,7 +288,7 @@ void set_geometry(Member& m, int tile_w, int k_chunks, int remap)
     fill_geometry(m.args, m.tile_w, m.k_chunks, m.xcd_remap);
 }
 
-// Fixes the HE-VI column-solve form of a member (NIMBUS_COLUMN_SOLVE_*).
+// Names the HE-VI column-solve form of a member (NIMBUS_COLUMN_SOLVE_*), which no launch depends on.
 int set_column_solve(Member& m, int form)
 {
     if (m.desc.config.acoustic_mode != NIMBUS_ACOUSTIC_HEVI)
@@ -298,18 +299,17 @@ int set_column_solve(Member& m, int form)
     {
     case NIMBUS_COLUMN_SOLVE_AUTO: seg = hevi_default_seg(m.elem, m.args.g.nx, m.args.g.ny, nz); break;
     case NIMBUS_COLUMN_SOLVE_PARTITIONED:
-        if (nz > kSegMaxNz) return fail(NIMBUS_EINVAL, "set_column_solve: the partitioned solve takes at most 129 levels");
+        if (nz > kSegMaxNz) return fail(NIMBUS_EINVAL, "set_column_solve: PARTITIONED is a form of at most 129 levels");
         seg = 1;
         break;
     case NIMBUS_COLUMN_SOLVE_SEQUENTIAL:
         if (hevi_partitioned_always(m.elem, nz))
-            return fail(NIMBUS_EINVAL, "set_column_solve: FP64 members of at most 129 levels hold no scratch for the "
-                                       "sequential sweep");
+            return fail(NIMBUS_EINVAL, "set_column_solve: SEQUENTIAL is no form of FP64 members of at most 129 levels");
         seg = 0;
         break;
     default: return fail(NIMBUS_EINVAL, "set_column_solve: unknown form");
     }
-    m.args.p.hevi_seg = seg;
+    m.hevi_seg = seg;
     return NIMBUS_OK;
 }
 
@@ -320,7 +320,6 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
     m.args.g = dev_grid(desc.grid, m.elem);
     m.args.geo.vec = 16 / m.elem;
     const int nz = desc.grid.nz;
-    const bool hevi = desc.config.acoustic_mode == NIMBUS_ACOUSTIC_HEVI;
     m.host_base.assign(std::size_t(kBaseCount) * nz, 0.0);
     const double* src[6] = {desc.base.rho0, desc.base.p0, desc.base.theta0, desc.base.qv0, desc.base.u0,
                             desc.base.v0};
@@ -443,7 +442,7 @@ int allocate_member(const nimbus_member_desc& desc, Member& m)
     sp.dts = c.dt / substeps;
     sp.mf_weight = sp.dts / c.dt;
     sp.acoustic_mode = c.acoustic_mode;
-    sp.hevi_seg = hevi ? hevi_default_seg(m.elem, desc.grid.nx, desc.grid.ny, nz) : 0;
+    m.hevi_seg = c.acoustic_mode == NIMBUS_ACOUSTIC_HEVI ? hevi_default_seg(m.elem, desc.grid.nx, desc.grid.ny, nz) : 0;
     sp.hevi_alpha = 0.5 * (1.0 + c.hevi_beta);
     sp.coriolis_f = c.coriolis_f;
     sp.bc_west = c.bc_west; sp.bc_east = c.bc_east; sp.bc_south = c.bc_south; sp.bc_north = c.bc_north;
@@ -1222,7 +1221,7 @@ int nimbus_hip_member_snapshot(nimbus_hip_ctx* ctx, uint32_t id, void* buf, uint
     h.tile_w = m->tile_w;
     h.k_chunks = m->k_chunks;
     h.xcd_remap = m->xcd_remap;
-    h.hevi_seg = m->args.p.hevi_seg;
+    h.hevi_seg = m->hevi_seg;
     h.steps = m->steps;
     h.field_bytes = z.field;
     h.rain_bytes = z.rain;
@@ -1380,10 +1379,7 @@ int nimbus_hip_member_set_column_solve(nimbus_hip_ctx* ctx, uint32_t id, int for
     if (!ctx) return fail(NIMBUS_EINVAL, "set_column_solve: null context");
     Member* m = find(ctx, id);
     if (!m) return fail(NIMBUS_ENOENT, "set_column_solve: unknown member");
-    const int before = m->args.p.hevi_seg;
-    const int rc = set_column_solve(*m, form);
-    if (rc == NIMBUS_OK && m->args.p.hevi_seg != before) drop_batches(ctx);
-    return rc;
+    return set_column_solve(*m, form);
 }
 
 int nimbus_hip_member_column_solve(nimbus_hip_ctx* ctx, uint32_t id, int* form)
@@ -1392,7 +1388,7 @@ int nimbus_hip_member_column_solve(nimbus_hip_ctx* ctx, uint32_t id, int* form)
     Member* m = find(ctx, id);
     if (!m) return fail(NIMBUS_ENOENT, "column_solve: unknown member");
     *form = m->desc.config.acoustic_mode != NIMBUS_ACOUSTIC_HEVI ? NIMBUS_COLUMN_SOLVE_AUTO
-            : m->args.p.hevi_seg                                  ? NIMBUS_COLUMN_SOLVE_PARTITIONED
+            : m->hevi_seg                                         ? NIMBUS_COLUMN_SOLVE_PARTITIONED
                                                                   : NIMBUS_COLUMN_SOLVE_SEQUENTIAL;
     return NIMBUS_OK;
 }

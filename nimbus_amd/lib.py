@@ -791,7 +791,7 @@ class Member:
                                                         int(xcd_remap)), "set_tiling")
 
     def set_column_solve(self, form):
-        """HE-VI column-solve form (COLUMN_SOLVE_*), fixed for the member until changed."""
+        """HE-VI column-solve form (COLUMN_SOLVE_*) that the member reports; it changes neither results nor time."""
         check(self.ctx.lib.nimbus_hip_member_set_column_solve(self.ctx.handle, self.id, int(form)),
               "set_column_solve")
 

@@ -31,9 +31,9 @@ Evicted members go back to the head of the queue under either order.
 
 With a TuningCache, every admitted member gets the autotuned launch geometry
 of its shape (tuned the first time the shape is seen); the geometry never
-changes results. `column_solve` fixes the HE-VI column-solve form of every
-member the server creates (None keeps each member's own default); it is part
-of the member's arithmetic, so run_alone must be given the same value.
+changes results. `column_solve` names the HE-VI column-solve form of every
+member the server creates (None keeps each member's own default); either form
+is solved with the same operations, so it changes neither results nor time.
 
 With `preempt` on, a request that does not fit may evict resident members
 whose remaining work (cells x steps) is at least `preempt_ratio` times its
@@ -382,8 +382,8 @@ class Server:
 
 
 def configure_member(m, mode, column_solve=None, tuning=None):
-    """The server's per-member settings: the HE-VI column-solve form (part of
-    the member's arithmetic) and the cached launch geometry (not)."""
+    """The server's per-member settings: the name of the HE-VI column-solve
+    form and the cached launch geometry. Neither changes results."""
     if column_solve is not None and mode == L.ACOUSTIC_HEVI:
         m.set_column_solve(column_solve)
     if tuning is not None:
@@ -396,8 +396,7 @@ def run_alone(ctx, req, precision=L.PRECISION_MIXED, acoustic_mode=L.ACOUSTIC_HE
     wl = req.workload
     dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
     m = ctx.member(wl.grid, wl.config(acoustic_mode=acoustic_mode), wl.base(), precision)
-    # the column-solve form applies to the FP32-storage members it was chosen
-    # for; FP64 reruns keep their default (partitioned up to 129 levels)
+    # FP64 members of at most 129 levels refuse the name SEQUENTIAL: FP64 reruns keep their default
     configure_member(m, acoustic_mode, column_solve if precision == L.PRECISION_MIXED else None, tuning)
     ctx.set_graphs(graphs)
     try:

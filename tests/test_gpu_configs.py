@@ -6,8 +6,7 @@ full sizes, in the precision and method each names:
   (N = 10);
 - 160 x 160 x 80 (500 m) and 400 x 400 x 100 (250 m): two FP64 large steps in
   both acoustic modes, and the mixed path against the FP64 oracle at its FP32
-  rounding bound (at 400 x 400 the FP32 member takes the sequential column
-  sweep);
+  rounding bound;
 - the 32-member uneven ensemble in one batch, each member bitwise equal to
   itself alone, the two smallest against the oracle;
 - the serving stream's request shapes (seeded Poisson arrivals, up to
@@ -70,7 +69,7 @@ def test_single_member_configs_fp64_and_mixed_match_oracle(hip_ctx, name):
             outm, _, _ = _run(hip_ctx, wl, cfg, L.PRECISION_MIXED, n_steps)
             check_mixed(outm, ref, f"{name} mixed hevi")
     if name == "c2":
-        # the FP32 member of this size takes the sequential column sweep by default
+        # the form that an FP32 member of this size reports by default
         m = hip_ctx.member(wl.grid, wl.config(acoustic_mode=L.ACOUSTIC_HEVI), wl.base(), L.PRECISION_MIXED)
         try:
             assert m.column_solve() == L.COLUMN_SOLVE_SEQUENTIAL

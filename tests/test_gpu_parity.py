@@ -332,10 +332,8 @@ def test_non_finite_state_is_sanitised_as_the_oracle_does(hip_ctx, mode, precisi
 
 @pytest.mark.parametrize("nz", [4, 14, 17, 33, 100, 129, 130, 140])
 def test_hevi_column_depths_fp64_match_fp64_oracle(hip_ctx, nz):
-    """The vertically implicit solve of FP64 members at column depths that
-    cover both of its forms: partitioned into runs of faces (nz <= 129:
-    one-face runs, uneven last runs, 16 runs of 8 faces) and the sequential
-    sweep (nz > 129); a 20 km deep domain with wind noise."""
+    """The vertically implicit solve of FP64 members from the fewest levels to
+    more than 129, even and odd; a 20 km deep domain with wind noise."""
     g, base, st = small_case(nx=12, ny=10, nz=nz, dz=20000.0 / nz, cloudy=True, wind_noise=1.0, dtype=np.float64)
     cfg = L.step_config(3.0, 6, acoustic_mode=L.ACOUSTIC_HEVI, lateral=L.BC_RIGID_SLIP)
     n_steps = 2
@@ -405,10 +403,10 @@ def check_mixed(out, ref, label, amplification=1e3):
 
 @pytest.mark.parametrize("form", [L.COLUMN_SOLVE_SEQUENTIAL, L.COLUMN_SOLVE_PARTITIONED])
 def test_mixed_column_solve_forms_match_fp64_oracle(hip_ctx, form):
-    """Both HE-VI column-solve forms of an FP32-storage member, forced on the
-    member, against the FP64 oracle at the FP32 rounding bound; the form is a
-    property of the member, so the same member beside a 264 x 256 member (a
-    batch of more than 32768 columns) gives bitwise the same result."""
+    """An FP32-storage member that reports either HE-VI column-solve form
+    against the FP64 oracle at the FP32 rounding bound, and bitwise the same
+    beside a 264 x 256 member that reports the other by default. Naming the
+    form drops no batch."""
     g, base, st64 = small_case(nx=20, ny=18, nz=14, cloudy=True, wind_noise=1.0, dtype=np.float64)
     st = {k: (v.astype(np.float32) if k in L.FIELDS else v) for k, v in st64.items()}
     cfg = L.step_config(3.0, 6, acoustic_mode=L.ACOUSTIC_HEVI, lateral=L.BC_RIGID_SLIP)
@@ -430,6 +428,10 @@ def test_mixed_column_solve_forms_match_fp64_oracle(hip_ctx, form):
         hip_ctx.step([alone], n_steps)
         hip_ctx.step([beside, big], n_steps)
         a, b = alone.download(), beside.download()
+        builds = hip_ctx.batch_stats()["batch_builds"]
+        alone.set_column_solve(L.COLUMN_SOLVE_SEQUENTIAL + L.COLUMN_SOLVE_PARTITIONED - form)
+        hip_ctx.step([alone], 1)
+        assert hip_ctx.batch_stats()["batch_builds"] == builds
     finally:
         for m in (big, alone, beside):
             m.destroy()
@@ -439,8 +441,8 @@ def test_mixed_column_solve_forms_match_fp64_oracle(hip_ctx, form):
 
 
 def test_mixed_deep_columns_sequential_match_fp64_oracle(hip_ctx):
-    """FP32 members deeper than 129 levels have only the sequential sweep:
-    140 levels of a 20 km domain against the FP64 oracle."""
+    """FP32 members deeper than 129 levels report SEQUENTIAL only: 140 levels
+    of a 20 km domain against the FP64 oracle."""
     nz = 140
     g, base, st64 = small_case(nx=12, ny=10, nz=nz, dz=20000.0 / nz, cloudy=True, wind_noise=1.0,
                                dtype=np.float64)
