@@ -11,7 +11,7 @@ reported: the other precision/method combinations, the operators beside the
 step (the step with explicit diffusion on, member snapshot/restore and NPY
 export, CM1 sounding I/O), the 32-member uneven ensemble run as one batch, and
 a short continuous-batching serving run with p50/p99 completion latency.
-Prints one JSON line.
+Prints one JSON line; the tables and series behind it go to stderr ("details").
 
   python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload c2]
                   [--serving-seconds S] [--no-ensemble] [--accuracy c2,c1|''] [--no-cpu-baseline]
@@ -302,6 +302,31 @@ def roofline_for(tab, cells, elem, workload, mode, n_sub, steps):
             "algorithmic_bytes_per_execution": ph["algorithmic_bytes_per_execution"],
             "bytes_per_cell": ph["bytes_per_cell"],
             "share_of_step": round(ph["ms_per_execution"] * ph["executions_per_step"] / total_ms, 3)}
+
+
+# Tables and series that go to stderr, so that the result line stays a few KB
+# whatever was run; of an hour's accuracy run the line keeps these figures.
+DETAILS = ("kernels_ms_per_step", "phases_roofline", "kernels_io_roofline", "roofline_mixed_explicit", "next_rows",
+           "cpu_baseline_more")
+ACCURACY_SUMMARY = ("workload", "simulated_seconds", "targets_met", "max_w_error", "rms_theta_p_error",
+                    "rain_relative_error")
+
+
+def split_details(result):
+    """The result line and what stays out of it, by name."""
+    line, details = {}, {}
+    for key, value in result.items():
+        if key in DETAILS:
+            details[key] = value
+        elif key.startswith("accuracy_1h"):
+            line[key] = {k: value[k] for k in ACCURACY_SUMMARY if k in value}
+            details[key] = value
+        elif key == "serving_c4":
+            line[key] = {k: v for k, v in value.items() if k != "fp64_rerun"}
+            details["serving_c4_fp64_rerun"] = value.get("fp64_rerun")
+        else:
+            line[key] = value
+    return line, details
 
 
 def column_solve_code(L, name):
@@ -715,8 +740,11 @@ def main():
         if "ensemble_c3" in result:
             result["gpu_over_cpu_more"]["ensemble"] = round(
                 result["ensemble_c3"]["cell_updates_per_s"] / result["cpu_baseline_more"]["ensemble_c3"]["value"], 1)
+    line, details = split_details(result)
+    for key, value in details.items():
+        progress(f"details {key}: {json.dumps(value)}")
     progress("done")
-    print(json.dumps(result))
+    print(json.dumps(line))
 
 
 if __name__ == "__main__":
