@@ -72,6 +72,36 @@ def test_acoustic_hydrostatic_rest_is_exact(hip_ctx):
     assert np.max(np.abs(u)) < 2e-3 and np.max(np.abs(v)) < 2e-3
 
 
+@pytest.mark.parametrize("lo, hi", [(0.88, 1.12), (1.1, 1.15), (0.85, 0.9), (1.0 / 64.0, 64.0), (1e-4, 1e-2), (1e3, 1e5)])
+def test_eos_far_from_the_base_state(hip_ctx, lo, hi):
+    """p = p00 (rho R theta / p00)^gamma of the FP32 perturbation form with
+    rho theta / (rho0 theta0) = 1 + x from lo to hi: the series (|x| < 1/8), the
+    line at 1/8 and beyond it, in air at rest, whose density stays. With u the
+    rounding of FP32, x is rounded (gamma u of p), then the power less one, p'
+    and p once each (u of p or p0): below 5 u (p + p0) together."""
+    g, base, st = small_case(nx=20, ny=18, nz=14)
+    shape = (g.nx, g.ny, g.nz)
+    r = np.random.default_rng(8)
+    ratio = np.exp(r.uniform(np.log(lo), np.log(hi), shape))
+    ratio.flat[0], ratio.flat[1] = lo, hi
+    rho = np.broadcast_to(base["rho0"], shape).astype(np.float32, order="C")
+    theta = (ratio * base["rho0"] * base["theta0"] / rho).astype(np.float32)
+    wind = [np.zeros(shape, np.float32) for _ in range(3)]
+    out_rho, p = rho.copy(), np.broadcast_to(base["p0"], shape).astype(np.float32, order="C")
+    d = L.AcousticFusedDispatch(
+        *[L.fptr(x) for x in wind], L.fptr(out_rho), L.fptr(p), L.fptr(theta), L.dptr(base["rho0"]),
+        L.dptr(base["p0"]), g.nz, g.nx, g.ny, g.nz, g.dx, g.dy, g.dz, 0.1, 1004.0 / 717.0, 1e-3, 10.0, 1e-6, 1e30,
+        1e5, 180.0, 120.0)
+    L.check(hip_ctx.lib.nimbus_hip_dispatch_acoustic_substep_fused(hip_ctx.handle, ctypes.byref(d)), "acoustic")
+    # the density as the member holds it: rho0 plus an FP32 perturbation
+    held = base["rho0"] + (rho - base["rho0"]).astype(np.float32)
+    ref = 1.0e5 * (held * 287.0 * theta.astype(np.float64) / 1.0e5) ** (1004.0 / 717.0)
+    bound = 5.0 * 2.0 ** -24 * (ref + base["p0"])
+    worst = float(np.max(np.abs(p - ref) / bound))
+    print(f"eos {lo:g} .. {hi:g}: {worst:.3f} of the bound")
+    assert np.all(np.isfinite(p)) and worst <= 1.0
+
+
 def test_kessler_matches_oracle(hip_ctx):
     g, base, st = small_case(cloudy=True)
     dt = 3.0
