@@ -3035,6 +3035,17 @@ void fill_geometry(MemberArgs& a, int tile_w, int k_chunks, int xcd_remap)
     G.edge_blocks = 3 * ((edge_cells(a.g.nx, a.g.ny) * a.g.nz + kBlock - 1) / kBlock);
 }
 
+// One thread per lane of a level (at least two waves); the staged profiles, two
+// doubles per cell, the meeting rows and the pivot verdicts in LDS.
+SolveShape solve_shape(int nz, int vec)
+{
+    const int lanes = solve_lanes(nz), cw = lanes * vec;
+    const unsigned threads = std::max(128u, unsigned(lanes * nz + 63) / 64u * 64u);
+    const std::size_t lds = std::size_t(nz) * (kLdsProfiles + 2 * cw) * sizeof(double) + 5 * cw * sizeof(double) +
+                            2 * cw * sizeof(int);
+    return SolveShape{threads, lds, int(std::min<std::size_t>(20 / (threads / 64), std::size_t(160) * 1024 / lds))};
+}
+
 int work_items(const MemberArgs& a, WorkKind kind)
 {
     const MemberGeom& G = a.geo;
@@ -3101,22 +3112,16 @@ void launch_map(Launcher& L, const char* name, K kernel, const BatchView& b, int
     L.end(name, ev);
 }
 
-// The column solve of the members with LL lanes per level, whose deepest has
-// nz levels: one thread per LL-th of a level (at least two waves), the staged
-// profiles, two doubles per cell and the meeting rows in LDS.
+// The column solve of one group.
 template <class S, int LL>
-void launch_hevi_solve(Launcher& L, const BatchView& b, int s, bool first, int nz)
+void launch_hevi_solve(Launcher& L, const BatchView& b, const SolveGroup& g, int s, bool first)
 {
-    constexpr int CW = LL * 16 / int(sizeof(S));
-    const BlockMap& m = b.maps[S_HEVI][W_SOLVE];
-    if (m.blocks <= 0) return;
-    const unsigned threads = std::max(128u, unsigned(LL * nz + 63) / 64u * 64u);
-    const std::size_t lds = std::size_t(nz) * (kLdsProfiles + 2 * CW) * sizeof(double) + 5 * CW * sizeof(double) +
-                            2 * CW * sizeof(int);
+    const SolveShape shape = solve_shape(g.nz, 16 / int(sizeof(S)));
     const auto kernel = first ? k_hevi_solve<S, true, LL> : k_hevi_solve<S, false, LL>;
     hipEvent_t ev;
     L.begin("acoustic_hevi_solve", ev);
-    hipLaunchKernelGGL(kernel, dim3(unsigned(m.blocks)), dim3(threads), lds, L.stream, b.args, m.entries, s);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(g.map.blocks)), dim3(shape.threads), shape.lds, L.stream, b.args,
+                       g.map.entries, s);
     L.end("acoustic_hevi_solve", ev);
 }
 
@@ -3147,9 +3152,10 @@ void launch_acoustic_substep(Launcher& L, const BatchView& b, int s, bool accumu
     launch_map(L, "acoustic_forward", k_acoustic_forward<S>, b, S_EXPLICIT, W_CELL, s, int(accumulate),
                int(init_at_first));
     const bool first = init_at_first && s == 0;
-    if (b.hevi_nz[0] > 0) launch_hevi_solve<S, 4>(L, b, s, first, b.hevi_nz[0]);
-    if (b.hevi_nz[1] > 0) launch_hevi_solve<S, 2>(L, b, s, first, b.hevi_nz[1]);
-    if (b.hevi_nz[2] > 0) launch_hevi_solve<S, 1>(L, b, s, first, b.hevi_nz[2]);
+    for (const SolveGroup& g : b.solves)
+        if (g.lanes == 4) launch_hevi_solve<S, 4>(L, b, g, s, first);
+        else if (g.lanes == 2) launch_hevi_solve<S, 2>(L, b, g, s, first);
+        else launch_hevi_solve<S, 1>(L, b, g, s, first);
     launch_map(L, "acoustic_momentum", k_momentum<S>, b, S_ALL, W_MOMENTUM, s, int(close));
     if (close && b.any_bc_split) launch_map(L, "boundary_closure", k_close<S>, b, S_ALL, W_SHELL, s);
 }

@@ -132,7 +132,7 @@ enum WorkKind
 {
     W_CELL = 0,    // one tile of columns at one level, or one run of a level (one cell per thread)
     W_DIAG = 1,    // one of kDiagBlocksPerMember reduction blocks
-    W_SOLVE = 2,   // solve_lanes x 16 bytes consecutive columns of one row, whole columns (HE-VI solve)
+    W_SOLVE = 2,   // solve_lanes x 16 bytes consecutive columns of one row, whole columns (BatchView::solves)
     W_TILECELL = 3,  // one tile of columns at one level whatever the geometry (wide stencils)
     W_MOMENTUM = 4,  // a wind component of 256 edge cells (edge_blocks of them), then as W_CELL
     W_SHELL = 5,     // a wind component of 256 edge cells (edge_blocks of them), then 256 other columns
@@ -157,6 +157,17 @@ constexpr int hevi_default_seg(int elem, int nx, int ny, int nz)
 // at most 1,024 threads.
 constexpr int solve_lanes(int nz) { return nz <= 256 ? 4 : nz <= 512 ? 2 : 1; }
 
+// Launch of the HE-VI solve for columns of up to nz levels (vec elements per 16
+// bytes), and how many of its workgroups a CU holds: 20 waves (the kernel's
+// launch bound) and 160 KB of LDS.
+struct SolveShape
+{
+    unsigned threads;
+    std::size_t lds;
+    int resident;
+};
+SolveShape solve_shape(int nz, int vec);
+
 // Member subsets a launch can be restricted to.
 enum MemberSubset
 {
@@ -170,6 +181,14 @@ struct BlockMap
 {
     const int2* entries = nullptr;  // device: {member index, local work index}
     int blocks = 0;
+};
+
+// HE-VI members of a batch that one launch solves: columns of up to nz levels,
+// all with the same lanes per level.
+struct SolveGroup
+{
+    int nz = 0, lanes = 0;
+    BlockMap map;
 };
 
 struct BatchView
@@ -189,7 +208,7 @@ struct BatchView
     int any_kessler_adaptive = 0; // a member whose microphysics subcycles follow its sedimentation limit
     int any_bc_split = 0;        // a member whose substeps are closed by k_close
     int max_nz = 0;
-    int hevi_nz[3] = {0, 0, 0};  // deepest of the HE-VI members with 4, 2 and 1 lanes per level
+    std::vector<SolveGroup> solves;
     int elem = 4;
     BlockMap maps[S_SUBSETS][W_KINDS];
 };

@@ -525,6 +525,44 @@ int xcd_logical(int b, int n)
     return x < r ? x * (q + 1) + local : r * (q + 1) + (x - r) * q + local;
 }
 
+// The HE-VI members of a batch by the launch that solves them, deepest first in
+// each. A workgroup has the threads and the LDS of its launch's deepest member,
+// so shallow columns beside deep ones leave a CU with few workgroups: of 8
+// members of 96 x 96 x 40 FP64 beside one of 32 x 32 x 129, two where six fit.
+// Members get a launch of their own where that saves a round of workgroups over
+// the 256 CUs, the most that the launch's own last round can cost (ms per step,
+// one launch -> two: that batch 3.36 -> 2.05, in mixed precision 1.60 -> 1.03,
+// beside one of 48 x 48 x 250 2.20 -> 1.21); smaller ones run beside the deeper.
+std::vector<std::vector<int>> solve_groups(const std::vector<Member*>& ms)
+{
+    constexpr double kCus = 256.0;
+    std::vector<int> order;
+    for (int q = 0; q < int(ms.size()); ++q)
+        if (ms[q]->args.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI) order.push_back(q);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return ms[a]->g().nz > ms[b]->g().nz; });
+    std::vector<std::vector<int>> groups;
+    for (std::size_t q = 0; q < order.size();)
+    {
+        // the members of one depth
+        std::size_t end = q;
+        double work = 0.0;
+        const MemberArgs& a = ms[order[q]]->args;
+        for (; end < order.size() && ms[order[end]]->g().nz == a.g.nz; ++end)
+            work += work_items(ms[order[end]]->args, W_SOLVE);
+        bool own = groups.empty();
+        if (!own)
+        {
+            const MemberArgs& deep = ms[groups.back().front()]->args;
+            const double beside = solve_shape(deep.g.nz, deep.geo.vec).resident, alone = solve_shape(a.g.nz, a.geo.vec).resident;
+            own = deep.geo.solve_lanes != a.geo.solve_lanes || work / beside - work / alone >= kCus;
+        }
+        if (own) groups.emplace_back();
+        groups.back().insert(groups.back().end(), order.begin() + q, order.begin() + end);
+        q = end;
+    }
+    return groups;
+}
+
 // Builds the device member table and block maps of a batch.
 int build_batch(Batch& b, const std::vector<Member*>& ms)
 {
@@ -554,11 +592,6 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
         b.view.any_diffusion |= m->args.p.dif_apply != 0;
         b.view.any_kessler_adaptive |= m->args.p.kessler_adaptive;
         b.view.any_bc_split |= bc_split(m->args.p);
-        if (m->args.p.acoustic_mode == NIMBUS_ACOUSTIC_HEVI)
-        {
-            int& nz = b.view.hevi_nz[m->args.geo.solve_lanes == 4 ? 0 : m->args.geo.solve_lanes == 2 ? 1 : 2];
-            nz = std::max(nz, m->args.g.nz);
-        }
         remap = remap && m->xcd_remap;
     }
     std::vector<int2> all;
@@ -568,7 +601,7 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
         for (int k = 0; k < W_KINDS; ++k)
         {
             std::vector<int2> logical;
-            for (std::size_t q = 0; q < ms.size(); ++q)
+            for (std::size_t q = 0; q < ms.size() && k != W_SOLVE; ++q)
             {
                 const int mode = ms[q]->args.p.acoustic_mode;
                 if (s == S_EXPLICIT && mode != NIMBUS_ACOUSTIC_EXPLICIT) continue;
@@ -589,6 +622,19 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
             counts[s][k] = n;
             for (int blk = 0; blk < n; ++blk) all.push_back(logical[remap ? xcd_logical(blk, n) : blk]);
         }
+    std::vector<std::size_t> solve_offsets;
+    b.view.solves.clear();
+    for (const std::vector<int>& group : solve_groups(ms))
+    {
+        std::vector<int2> logical;
+        for (int q : group)
+            for (int l = 0, n = work_items(ms[q]->args, W_SOLVE); l < n; ++l) logical.push_back(int2{q, l});
+        const int n = int(logical.size());
+        solve_offsets.push_back(all.size());
+        const MemberArgs& deepest = ms[group.front()]->args;
+        b.view.solves.push_back(SolveGroup{deepest.g.nz, deepest.geo.solve_lanes, BlockMap{nullptr, n}});
+        for (int blk = 0; blk < n; ++blk) all.push_back(logical[remap ? xcd_logical(blk, n) : blk]);
+    }
     NIMBUS_HIP_TRY(hipMalloc(&b.d_args, sizeof(MemberArgs) * args.size()));
     NIMBUS_HIP_TRY(hipMemcpy(b.d_args, args.data(), sizeof(MemberArgs) * args.size(), hipMemcpyHostToDevice));
     NIMBUS_HIP_TRY(hipMalloc(&b.d_maps, sizeof(int2) * std::max<std::size_t>(all.size(), 1)));
@@ -600,6 +646,7 @@ int build_batch(Batch& b, const std::vector<Member*>& ms)
     for (int s = 0; s < S_SUBSETS; ++s)
         for (int k = 0; k < W_KINDS; ++k)
             b.view.maps[s][k] = BlockMap{b.d_maps + offsets[s][k], counts[s][k]};
+    for (std::size_t q = 0; q < solve_offsets.size(); ++q) b.view.solves[q].map.entries = b.d_maps + solve_offsets[q];
     return NIMBUS_OK;
 }
 

@@ -724,6 +724,37 @@ def test_autotune_restores_state(hip_ctx):
         m.destroy()
 
 
+@pytest.mark.parametrize("precision", [L.PRECISION_MIXED, L.PRECISION_FP64])
+@pytest.mark.parametrize("shallow, launches", [((20, 18, 14), 1), ((144, 128, 14), 2)])
+def test_shallow_members_beside_a_deep_one(hip_ctx, shallow, launches, precision):
+    """A large shallow member beside one of 129 levels is solved by a launch of
+    its own, a small one by the deep member's; each as alone, bitwise."""
+    dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
+    cfg = L.step_config(3.0, 6, acoustic_mode=L.ACOUSTIC_HEVI)
+    members, alone = [], []
+    try:
+        for nx, ny, nz in ((16, 12, 129), shallow):
+            g, base, st = small_case(nx=nx, ny=ny, nz=nz, dz=min(500.0, 20000.0 / nz), cloudy=True, dtype=dtype)
+            alone.append(_run_member(hip_ctx, g, base, cfg, st, precision, 2)[0])
+            members.append(hip_ctx.member(g, cfg, base, precision))
+            members[-1].upload(st)
+        hip_ctx.step(members, 1)
+        hip_ctx.set_kernel_timing(True)
+        hip_ctx.reset_kernel_timing()
+        hip_ctx.step(members, 1)
+        solves = hip_ctx.kernel_timing()["acoustic_hevi_solve"][0]
+        hip_ctx.set_kernel_timing(False)
+        assert solves == launches * max(m.substeps for m in members)
+        beside = [m.download() for m in members]
+    finally:
+        hip_ctx.set_kernel_timing(False)
+        for m in members:
+            m.destroy()
+    for a, b in zip(alone, beside):
+        for f in L.FIELDS:
+            assert np.array_equal(a[f], b[f]), f
+
+
 def test_fp64_and_mixed_members_in_one_call(hip_ctx):
     g, base, st64 = small_case(nx=20, ny=18, nz=14, cloudy=True, dtype=np.float64)
     st32 = {k: (v.astype(np.float32) if k in L.FIELDS else v) for k, v in st64.items()}
