@@ -3031,7 +3031,7 @@ void fill_geometry(MemberArgs& a, int tile_w, int k_chunks, int xcd_remap)
     G.tiles_y = (a.g.ny + G.tile_h - 1) / G.tile_h;
     G.k_chunks = std::max(1, std::min(k_chunks, a.g.nz));
     G.xcd_remap = xcd_remap ? 1 : 0;
-    G.solve_lanes = solve_lanes(a.g.nz);
+    G.solve_lanes = solve_lanes(a.g.nz, G.vec);
     G.edge_blocks = 3 * ((edge_cells(a.g.nx, a.g.ny) * a.g.nz + kBlock - 1) / kBlock);
 }
 
@@ -3039,11 +3039,11 @@ void fill_geometry(MemberArgs& a, int tile_w, int k_chunks, int xcd_remap)
 // doubles per cell, the meeting rows and the pivot verdicts in LDS.
 SolveShape solve_shape(int nz, int vec)
 {
-    const int lanes = solve_lanes(nz), cw = lanes * vec;
-    const unsigned threads = std::max(128u, unsigned(lanes * nz + 63) / 64u * 64u);
+    const int lanes = solve_lanes(nz, vec), cw = lanes * vec;
+    const unsigned threads = std::max(128u, unsigned(lanes * nz + 63) / 64u * 64u), waves = threads / 64;
     const std::size_t lds = std::size_t(nz) * (kLdsProfiles + 2 * cw) * sizeof(double) + 5 * cw * sizeof(double) +
                             2 * cw * sizeof(int);
-    return SolveShape{threads, lds, int(std::min<std::size_t>(20 / (threads / 64), std::size_t(160) * 1024 / lds))};
+    return SolveShape{threads, lds, int(std::min<std::size_t>(waves > 8 ? 1 : 20 / waves, std::size_t(160) * 1024 / lds))};
 }
 
 int work_items(const MemberArgs& a, WorkKind kind)

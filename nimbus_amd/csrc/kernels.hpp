@@ -102,7 +102,7 @@ struct MemberGeom
     // per-cell work in runs of kBlock consecutive elements of one level's
     // padded [j][i] plane (`runs` per level) instead of column tiles at one level
     int linear, runs;
-    // HE-VI solve: 16-byte lanes per level of a workgroup (solve_lanes(nz)) and
+    // HE-VI solve: 16-byte lanes per level of a workgroup (solve_lanes) and
     // elements per 16 bytes (fixed by the storage type at creation)
     int solve_lanes, vec;
     // workgroups of the edge cells (close_edges), which the boundary closure spreads
@@ -152,14 +152,20 @@ constexpr int hevi_default_seg(int elem, int nx, int ny, int nz)
     return nz <= kSegMaxNz && (elem == 8 || long(nx) * long(ny) < long(kSweepColumns)) ? 1 : 0;
 }
 
-// HE-VI solve: lanes of 16 bytes per level, so that a workgroup of one thread
-// per lane holds a whole column of up to 1,024 levels (runtime grid check) in
-// at most 1,024 threads.
-constexpr int solve_lanes(int nz) { return nz <= 256 ? 4 : nz <= 512 ? 2 : 1; }
+// HE-VI solve: lanes of 16 bytes (vec elements) per level, so that a workgroup of
+// one thread per lane holds a whole column of up to 1,024 levels (runtime grid
+// check) in at most 1,024 threads. Workgroups of more than 8 waves go one to a
+// CU: FP64 members of 129 to 160 levels take two lanes, of which several fit (ms
+// per step with four lanes -> two: 128 x 128 x 129 1.61 -> 1.56, 160 x 160 x 140
+// 2.95 -> 2.77, 48 x 48 x 140 0.42 -> 0.37). FP32 members there lose as often as they gain (48 x 48 x 140
+// 6 % slower, 96 x 96 x 140 7 % faster), FP64 ones of 161 to 192 levels lose 3 %.
+constexpr int solve_lanes(int nz, int vec)
+{
+    return nz <= 256 && !(vec == 2 && nz > 128 && nz <= 160) ? 4 : nz <= 512 ? 2 : 1;
+}
 
-// Launch of the HE-VI solve for columns of up to nz levels (vec elements per 16
-// bytes), and how many of its workgroups a CU holds: 20 waves (the kernel's
-// launch bound) and 160 KB of LDS.
+// Launch of the HE-VI solve for columns of up to nz levels, and how many of its
+// workgroups a CU holds: 20 waves (the kernel's launch bound) and 160 KB of LDS.
 struct SolveShape
 {
     unsigned threads;

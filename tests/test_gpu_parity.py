@@ -492,7 +492,7 @@ def test_mixed_deep_columns_sequential_match_fp64_oracle(hip_ctx):
     check_mixed(out, ref, "deep mixed")
 
 
-@pytest.mark.parametrize("nx, ny, nz", [(5, 5, 4), (18, 5, 5), (15, 6, 40), (33, 7, 129), (5, 6, 130), (17, 5, 256),
+@pytest.mark.parametrize("nx, ny, nz", [(5, 5, 4), (18, 5, 5), (15, 6, 40), (33, 7, 129), (5, 6, 130), (6, 5, 161), (17, 5, 256),
                                         (9, 5, 257), (6, 5, 513), (5, 5, 1024)])
 def test_column_solve_depths_match_fp64_oracle(hip_ctx, nx, ny, nz):
     """The in-LDS column solve at the edges of its workgroup shapes (4, 2 and 1
@@ -727,13 +727,13 @@ def test_autotune_restores_state(hip_ctx):
 @pytest.mark.parametrize("precision", [L.PRECISION_MIXED, L.PRECISION_FP64])
 @pytest.mark.parametrize("shallow, launches", [((20, 18, 14), 1), ((144, 128, 14), 2)])
 def test_shallow_members_beside_a_deep_one(hip_ctx, shallow, launches, precision):
-    """A large shallow member beside one of 129 levels is solved by a launch of
+    """A large shallow member beside one of 120 levels is solved by a launch of
     its own, a small one by the deep member's; each as alone, bitwise."""
     dtype = np.float32 if precision == L.PRECISION_MIXED else np.float64
     cfg = L.step_config(3.0, 6, acoustic_mode=L.ACOUSTIC_HEVI)
     members, alone = [], []
     try:
-        for nx, ny, nz in ((16, 12, 129), shallow):
+        for nx, ny, nz in ((16, 12, 120), shallow):
             g, base, st = small_case(nx=nx, ny=ny, nz=nz, dz=min(500.0, 20000.0 / nz), cloudy=True, dtype=dtype)
             alone.append(_run_member(hip_ctx, g, base, cfg, st, precision, 2)[0])
             members.append(hip_ctx.member(g, cfg, base, precision))
