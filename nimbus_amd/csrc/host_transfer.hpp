@@ -5,7 +5,8 @@
 // overlaps it. Here the device side of chunk c (a kernel that reads or writes
 // its slot over the host link, 49-53 GB/s) runs while a few threads move other
 // chunks between slots and the caller's arrays (29 GB/s per thread in warm
-// pages, 13 in fresh ones, 55 together).
+// pages, 13 in fresh ones, 55 together). Small calls, and memory of the runtime
+// (pinned, or a device's), take other ways: see copy() and place().
 #pragma once
 
 #include <hip/hip_runtime.h>

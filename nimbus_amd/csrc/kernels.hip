@@ -746,20 +746,21 @@ __global__ __launch_bounds__(kBlock) void k_acoustic_forward(const MemberArgs* _
 // the same code with a zero g and H and keep their w; rows of y ghosts skip
 // the solve.
 //
-// Bound by latency: a workgroup's time is its loads (10-16 k cycles), the
-// cells (9 k), the two chains (13 k) and the end (7 k), and the register file
-// holds two (100 levels) to four (64 levels) workgroups per CU, so the time
-// follows the columns in flight. 16-byte lanes because 8- and 4-byte ones
-// took 576 and 914 us per substep where these take 426 (400 x 400 x 100), and
-// four lanes per level because a row segment is then one 64-byte line.
-// Against a kernel for the horizontal part and one thread per column, or one
-// per 8 faces, for the vertical (us per substep): 400 x 400 x 100 mixed
-// 441 -> 417, 640 x 640 x 60 674 -> 463, 100 x 120 x 140 138 -> 78,
-// 160 x 160 x 80 82 -> 64, 48 x 48 x 40 21 -> 13, 256 x 256 x 80 FP64 262 -> 251.
-// At most 96 VGPRs (the launch bound): five waves per SIMD, so that four
-// workgroups of 80 levels share a CU instead of three: 160 x 160 x 80 62.6 ->
-// 53.1 us against 104 VGPRs, 400 x 400 x 100 426 -> 405, 100 x 120 x 140 78 ->
-// 74. The next step, 80 VGPRs, spills.
+// Bound by latency: a workgroup's time is its loads, the cells, the two chains
+// and the end (10-16, 9, 13 and 7 k cycles of 400 x 400 x 100, in the build with
+// 104 VGPRs), and a CU has room for 20 waves (96 VGPRs, the launch bound: five
+// waves per SIMD): two workgroups of 100 levels, one from 129 levels on. So the
+// time follows the columns in flight. us per substep of a kernel for the
+// horizontal part and one thread per column, or one per 8 faces, for the vertical
+// -> of this one: 400 x 400 x 100 mixed 444 -> 400, 640 x 640 x 60 680 -> 445,
+// 320 x 320 x 100 268 -> 271, 256 x 256 x 80 141 -> 116, 160 x 160 x 80 82 -> 53,
+// 100 x 120 x 140 138 -> 75, 48 x 48 x 40 21 -> 13; FP64 256 x 256 x 80 258 -> 252,
+// 320 x 320 x 100 490 -> 517, 400 x 400 x 100 767 -> 779 (the closure in the momentum
+// update makes up for the last two).
+// Four 16-byte lanes per level, because a row segment is then one 64-byte line;
+// of the 104-register build 8- and 4-byte lanes took 576 and 914 us where 16-byte
+// ones took 426 (400 x 400 x 100). From 104 to 96 VGPRs 160 x 160 x 80 went from
+// 62.6 to 53.1, 100 x 120 x 140 from 78 to 74. The next step, 80 VGPRs, spills.
 template <class S>
 using Vec = __attribute__((ext_vector_type(16 / sizeof(S)))) S;
 

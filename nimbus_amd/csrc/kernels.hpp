@@ -157,8 +157,9 @@ constexpr int hevi_default_seg(int elem, int nx, int ny, int nz)
 // check) in at most 1,024 threads. Workgroups of more than 8 waves go one to a
 // CU: FP64 members of 129 to 160 levels take two lanes, of which several fit (ms
 // per step with four lanes -> two: 128 x 128 x 129 1.61 -> 1.56, 160 x 160 x 140
-// 2.95 -> 2.77, 48 x 48 x 140 0.42 -> 0.37). FP32 members there lose as often as they gain (48 x 48 x 140
-// 6 % slower, 96 x 96 x 140 7 % faster), FP64 ones of 161 to 192 levels lose 3 %.
+// 2.95 -> 2.77, 48 x 48 x 140 0.42 -> 0.37). FP32 members there lose as often as
+// they gain (48 x 48 x 140 6 % slower, 96 x 96 x 140 7 % faster), FP64 ones of 161
+// to 192 levels lose 3 %.
 constexpr int solve_lanes(int nz, int vec)
 {
     return nz <= 256 && !(vec == 2 && nz > 128 && nz <= 160) ? 4 : nz <= 512 ? 2 : 1;

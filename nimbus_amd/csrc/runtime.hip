@@ -1673,7 +1673,6 @@ int nimbus_hip_dispatch_slow_tendencies(nimbus_hip_ctx* ctx, const nimbus_slow_t
     Member& m = sm.m;
     m.args.p.coriolis_f = d->coriolis_f;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    const std::size_t n = std::size_t(d->nr) * d->nth * d->nz;
     nimbus_host_state hs{const_cast<float*>(d->u_data), const_cast<float*>(d->v_data), const_cast<float*>(d->w_data),
                          const_cast<float*>(d->rho_data), nullptr, nullptr, const_cast<float*>(d->qv_data),
                          const_cast<float*>(d->qc_data), const_cast<float*>(d->qr_data), nullptr};
@@ -1706,7 +1705,6 @@ int nimbus_hip_dispatch_slow_rk2(nimbus_hip_ctx* ctx, const nimbus_slow_rk2_disp
     m.args.p.coriolis_f = d->coriolis_f;
     m.args.p.dt = d->dt_large;
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    const std::size_t n = std::size_t(d->nx) * d->ny * d->nz;
     nimbus_host_state hs{d->u, d->v, d->w, const_cast<float*>(d->rho), nullptr, nullptr,
                          const_cast<float*>(d->qv), const_cast<float*>(d->qc), const_cast<float*>(d->qr), nullptr};
     rc = upload_scratch(ctx, m, hs);
@@ -1797,7 +1795,6 @@ int nimbus_hip_dispatch_kessler(nimbus_hip_ctx* ctx, const nimbus_kessler_dispat
     NIMBUS_HIP_TRY(hipMemset(f.base, 0, sizeof(double) * kBaseCount * d->nz));
     m.args.p.kessler = KesslerConst{d->qc0, d->c_auto, d->c_accr, d->evap_eff, d->vt_max};
     if ((rc = sm.finish_setup()) != NIMBUS_OK) return rc;
-    const std::size_t n = std::size_t(d->nx) * d->ny * d->nz;
     nimbus_host_state hs{nullptr, nullptr, nullptr, const_cast<float*>(d->rho), const_cast<float*>(d->p),
                          const_cast<float*>(d->theta), const_cast<float*>(d->qv), const_cast<float*>(d->qc),
                          const_cast<float*>(d->qr), nullptr};
