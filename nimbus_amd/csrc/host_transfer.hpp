@@ -54,6 +54,15 @@ public:
     static constexpr std::size_t kSlot = std::size_t(2) << 20;
     static constexpr int kSlots = 10;
     static constexpr int kThreads = 6;
+    // Bytes for each thread that copies, fields turned by the kernel and whole
+    // arrays. Starting a thread, and the release of device memory beside it, cost
+    // what it saves on less: fields with 1 MB against 4 MB for each, us: 9 of
+    // 64 x 64 x 48 doubles 435 to 408, the acoustic contract of 84 x 90 x 60 cells
+    // 2,216 to 1,815 (2 MB 1,965). Arrays with 1, 2 and 4 MB: the transport
+    // contract of 96 x 100 x 70 cells 2,680, 2,460 and 2,540, of 118 x 122 x 60
+    // 3,110, 3,130 and 3,640.
+    static constexpr std::size_t kFieldShare = std::size_t(4) << 20;
+    static constexpr std::size_t kArrayShare = std::size_t(2) << 20;
     // Whole arrays take the ring from these sizes of one direction on (down:
     // and of an array on average). Below them the ring's threads and the copy,
     // event and wait of every chunk cost more than they overlap. Plain copies
@@ -65,7 +74,7 @@ public:
     // 160 x 160 x 80 (33 MB) 3,840 to 3,530, with 5 of them 6,590 to 6,040.
     static constexpr std::size_t kRingDown = std::size_t(4) << 20;
     static constexpr std::size_t kRingArray = std::size_t(512) << 10;
-    static constexpr std::size_t kRingUp = std::size_t(32) << 20;
+    static constexpr std::size_t kRingUp = std::size_t(28) << 20;
     // Whether `count` arrays of `bytes` together take the ring.
     static constexpr bool takes_ring(bool up, std::size_t bytes, std::size_t count)
     {
@@ -86,7 +95,8 @@ public:
     // array. Returns when the caller's arrays are read or written. Transfers of
     // one ring run one after the other.
     template <class Launch>
-    hipError_t run(int device, hipStream_t stream, bool up, const std::vector<HostChunk>& chunks, Launch launch)
+    hipError_t run(int device, hipStream_t stream, bool up, const std::vector<HostChunk>& chunks, Launch launch,
+                   std::size_t share = kFieldShare)
     {
         std::lock_guard<std::mutex> one(busy_);
         State st;
@@ -101,10 +111,8 @@ public:
             }
         hipError_t e = prepare(copies != 0);
         if (e != hipSuccess) return e;
-        // a thread for each 4 MB: one for each MB took 2,040 us where this takes 1,910 (a contract
-        // call of 13 arrays of 96 x 96 x 60 floats) and 435 where this takes 408 (9 of 64 x 64 x 48
-        // doubles), in starting them and in the release of device memory beside them
-        const int want = !up && shared(chunks) ? 1 : int(std::min<std::size_t>({std::size_t(kThreads), copies, bytes >> 22}));
+        const std::size_t most = !up && shared(chunks) ? 1 : std::min(std::size_t(kThreads), copies);
+        const int want = int(std::min(most, (bytes + share / 2) / share));
         std::vector<std::thread> team;
         team.reserve(kThreads);  // no allocation once a thread runs
         try
@@ -194,7 +202,7 @@ public:
             }
         return run(device, stream, up, chunks, [&](int c, char* p) {
             return hipMemcpyAsync(up ? dev[c] : p, up ? p : dev[c], chunks[c].bytes, hipMemcpyDefault, stream);
-        });
+        }, kArrayShare);
     }
 
     // How a kernel on `device` reaches a caller's array of elements of `size`
